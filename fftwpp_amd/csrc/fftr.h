@@ -38,6 +38,15 @@ template<int M, int V=16> struct RPlan {
   static constexpr int NST=NV+(LAST > 1 ? 1 : 0);
   static constexpr int PAD=M+M/16;                      // exchange words
   __host__ __device__ static constexpr int radix(int s) { return s < NV ? V : LAST; }
+  // Stage s writes output u of butterfly j at dest<s>(j) + u ns(s); the bits
+  // of j move without mixing, so dest(a + b) = dest(a) + dest(b) for a and b
+  // without a bit in common.
+  template<int s>
+  static __device__ __forceinline__ int dest(int j)
+  {
+    const int kp=j & (ns(s)-1);
+    return (j-kp)*radix(s)+kp;
+  }
   // loops rather than recursion, so that calls with a run-time s inline
   __host__ __device__ static constexpr int ns(int s)
   {
@@ -45,6 +54,7 @@ template<int M, int V=16> struct RPlan {
     for(int i=0; i < s; ++i) n *= radix(i);
     return n;
   }
+  __host__ __device__ static constexpr int logns(int s) { return s < NV ? LV*s : LV*NV; }
   __host__ __device__ static constexpr int off(int s)
   {
     int o=0;
@@ -59,20 +69,23 @@ __device__ __forceinline__ int padr(int e) { return e+(e >> 4); }
 // swizzle of the low bits by higher bits that makes every exchange of the
 // transform conflict-free on gfx950's LDS (64-bit words: writes served 16
 // lanes per pass over 32 banks, reads 32 lanes over 64 banks; 32-bit words:
-// 32 lanes over 32 banks) for M >= 128 (FP64, V = 8), M >= 256 (FP32, V = 8)
-// or M >= 512 (FP32, V = 16); e + e/16 below that.  Indices stay below
-// M + M/16.
+// 32 lanes over 32 banks).  Shorter sequences (V = 8: M < 128 in FP64, M <
+// 256 in FP32; V = 16: M < 512) take e + e/16, whose compile-time part is an
+// immediate offset of the access: it has conflicts, but needs 10 to 60 fewer
+// registers and no instructions (complex rows of M = 64 FP64 98 us against
+// 107 swizzled, M = 128 FP32 67 against 91; M = 128 FP64 133 against 126).
+// Indices stay below M + M/16.
+template<typename T, int M, int V>
+__host__ __device__ constexpr bool xswizzled()
+{
+  return M >= (V == 16 ? 512 : sizeof(T) == 8 ? 128 : 256);
+}
 template<typename T, int M, int V>
 __device__ __forceinline__ int xidx(int e)
 {
-  if constexpr(sizeof(T) == 8 && V == 8 && M >= 128)
-    return e ^ ((e >> 4) & 7) ^ (((e >> 6) & 1) << 3);
-  else if constexpr(sizeof(T) == 4 && V == 8 && M >= 256)
-    return e ^ ((e >> 5) & 7) ^ (((e >> 6) & 3) << 3);
-  else if constexpr(sizeof(T) == 4 && V == 16 && M >= 512)
-    return e ^ ((e >> 4) & 7) ^ (((e >> 7) & 3) << 3);
-  else
-    return padr(e);
+  if constexpr(V == 8 && xswizzled<T,M,V>()) return e ^ ((e >> 3) & 7) ^ (((e >> 6) & 3) << 3);
+  else if constexpr(xswizzled<T,M,V>()) return e ^ ((e >> 4) & 7) ^ (((e >> 7) & 3) << 3);
+  else return padr(e);
 }
 
 // Twiddle table (M - 1 complex words) from zN of a dimension with N = M q.
@@ -82,15 +95,16 @@ __device__ __forceinline__ void fill_twr(cplx<T> *tw, const cplx<T> *zN, int q,
 {
   typedef RPlan<M,V> P;
   for(int e=tid; e < M-1; e += nthreads) {
-    // locate the stage of entry e (constants per unrolled k)
-    int Ns=P::ns(1), R=P::radix(1), off=0;
+    // locate the stage of entry e (constants per unrolled k); Ns and Ns R are
+    // powers of two: shifts only
+    int ln=P::logns(1), lr=P::logns(1)+__builtin_ctz(P::radix(1)), off=0;
 #pragma unroll
     for(int k=2; k < P::NST; ++k)
-      if(e >= P::off(k)) { Ns=P::ns(k); R=P::radix(k); off=P::off(k); }
+      if(e >= P::off(k)) { ln=P::logns(k); lr=ln+__builtin_ctz(P::radix(k)); off=P::off(k); }
     const int rel=e-off;
-    const int tp=rel/Ns+1, kp=rel-(tp-1)*Ns;
+    const int tp=(rel >> ln)+1, kp=rel & ((1 << ln)-1);
     // e^{2 pi i tp kp/(Ns R)} = zN[q tp kp M/(Ns R)]
-    tw[e]=zN[(int64_t) q*tp*kp*(M/(Ns*R))];
+    tw[e]=zN[(int64_t) q*((tp*kp) << (P::LOG-lr))];
   }
 }
 
@@ -116,8 +130,14 @@ __device__ __forceinline__ void rsync()
 }
 
 // Word of element e in a one-round exchange area (the default index map).
+// The maps act on disjoint bit fields one by one, so the word of an element
+// whose thread part and compile-time part have no bit in common is
+// join(at(thread part), at(constant)): one instruction per access and one
+// register per stage, where a map evaluated per element took several of each.
 template<typename T, int M, int V> struct RowXI {
+  static constexpr bool SWIZZLE=xswizzled<T,M,V>();
   static __device__ __forceinline__ int at(int e) { return xidx<T,M,V>(e); }
+  static __device__ __forceinline__ int join(int a, int b) { return SWIZZLE ? a ^ b : a+b; }
 };
 
 // Stage s of the transform (see the top of this file); recurses into s+1.
@@ -154,14 +174,12 @@ __device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const cplx<T> *tw,
   }
   if constexpr(s+1 < P::NST && CX) {
     // exchange: output u of butterfly b goes to (j/Ns) Ns R + k' + u Ns
+    const int wo=XI::at(P::template dest<s>(t)) ^ xm, ro=XI::at(t) ^ xm;
 #pragma unroll
     for(int b=0; b < NB; ++b) {
-      const int j=t+TPS*b;
-      const int kp=j & (Ns-1);
-      const int base=(j-kp)*R+kp;
 #pragma unroll
       for(int u=0; u < R; ++u) {
-        const int e=XI::at(base+u*Ns) ^ xm;
+        const int e=XI::join(wo,XI::at(P::template dest<s>(TPS*b)+u*Ns));
         xb[e]=v[b+u*NB].x;
         xb[P::PAD+e]=v[b+u*NB].y;
       }
@@ -169,7 +187,7 @@ __device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const cplx<T> *tw,
     rsync<TPS,BLK>();
 #pragma unroll
     for(int k=0; k < V; ++k) {
-      const int e=XI::at(t+TPS*k) ^ xm;
+      const int e=XI::join(ro,XI::at(TPS*k));
       v[k]=mk(xb[e],xb[P::PAD+e]);
     }
     rsync<TPS,BLK>();
@@ -240,17 +258,15 @@ __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
     }
   }
   if constexpr(s+1 < P::NST) {
+    const int wo=XI::at(P::template dest<s>(t)), ro=XI::at(t);
 #pragma unroll
     for(int pass=0; pass < 2; ++pass) {
       cplx<T> *Z=pass == 0 ? X : Y;
 #pragma unroll
       for(int b=0; b < NB; ++b) {
-        const int j=t+TPS*b;
-        const int kp=j & (Ns-1);
-        const int base=(j-kp)*R+kp;
 #pragma unroll
         for(int u=0; u < R; ++u) {
-          const int e=XI::at(base+u*Ns);
+          const int e=XI::join(wo,XI::at(P::template dest<s>(TPS*b)+u*Ns));
           xb[e]=Z[b+u*NB].x;
           xb[P::PAD+e]=Z[b+u*NB].y;
         }
@@ -258,7 +274,7 @@ __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
       rsync<TPS>();
 #pragma unroll
       for(int k=0; k < V; ++k) {
-        const int e=XI::at(t+TPS*k);
+        const int e=XI::join(ro,XI::at(TPS*k));
         Z[k]=mk(xb[e],xb[P::PAD+e]);
       }
       rsync<TPS>();

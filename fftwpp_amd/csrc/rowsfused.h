@@ -12,7 +12,8 @@
 //   m = 256, complex (not centred), L <= 256, q <= 8: rowconv256p_kernel
 //     (q = 2: both residues of a row in one wave) or rowconv256_kernel;
 //   power-of-two m in [16, 4096] covering the row (L <= m, or H <= m for
-//     Hermitian rows), m q < 2^30: rowreg_kernel.
+//     Hermitian rows), m q < 2^30: rowcx_kernel (complex and centred rows),
+//     hrowpk_kernel or rowreg_kernel (Hermitian rows).
 #pragma once
 #include <algorithm>
 #include <mutex>
@@ -90,6 +91,14 @@ inline int rows256_launch(const DimArgs &a, const void *f, const void *g, size_t
   return fused_status(hipGetLastError());
 }
 
+// Rows of stride rs words of E bytes that one buffer resource covers (their
+// byte offsets and the last row's 4096 words stay below 2^31); at least 1.
+inline size_t rows_in_buffer(size_t rs, size_t E)
+{
+  const size_t span=((size_t) 1 << 31)-4096*E;
+  return rs == 0 ? ((size_t) 1 << 31) : std::max<size_t>(1,span/(rs*E));
+}
+
 // RP residue lanes per row when rows are too few to fill the chip (under 512)
 // and the row has at least two residue passes (residues, or residue pairs for
 // Hermitian rows).
@@ -103,19 +112,38 @@ inline int rowreg_launch_rp(const DimArgs &a, const void *f, const void *g, size
   const size_t nt=RP > 1 ? RP*TPS : (TPS > 64 ? TPS : 256);
   const size_t slots=nt/TPS;
   const size_t lds=M*sizeof(cplx<T>)+slots*2*RPlan<M,V>::PAD*sizeof(T);
-  const hipError_t e=fused_allow_lds(rowreg_kernel<T,M,HERM,RP,Op>,lds);
-  if(e != hipSuccess) return fused_status(e);
   const size_t rpb=RP > 1 ? 1 : slots;
-  size_t nb=(rows+rpb-1)/rpb;
-  // persistent grid: the twiddle table is filled once per resident block
-  nb=std::min(nb,fused_resident(rowreg_kernel<T,M,HERM,RP,Op>,(int) nt,lds));
-  hipLaunchKernelGGL((rowreg_kernel<T,M,HERM,RP,Op>),dim3((unsigned) nb),dim3((unsigned) nt),
-                     lds,st,a,(const cplx<T> *) f,(const cplx<T> *) g,(int64_t) rows,
-                     (int64_t) rs,(cplx<T> *) out,(int64_t) os,(T) scale,op);
-  return fused_status(hipGetLastError());
+  if constexpr(HERM) {
+    const hipError_t e=fused_allow_lds(rowreg_kernel<T,M,RP,Op>,lds);
+    if(e != hipSuccess) return fused_status(e);
+    size_t nb=(rows+rpb-1)/rpb;
+    // persistent grid: the twiddle table is filled once per resident block
+    nb=std::min(nb,fused_resident(rowreg_kernel<T,M,RP,Op>,(int) nt,lds));
+    hipLaunchKernelGGL((rowreg_kernel<T,M,RP,Op>),dim3((unsigned) nb),dim3((unsigned) nt),
+                       lds,st,a,(const cplx<T> *) f,(const cplx<T> *) g,(int64_t) rows,
+                       (int64_t) rs,(cplx<T> *) out,(int64_t) os,(T) scale,op);
+    return fused_status(hipGetLastError());
+  } else {
+    const hipError_t e=fused_allow_lds(rowcx_kernel<T,M,RP,Op>,lds);
+    if(e != hipSuccess) return fused_status(e);
+    const size_t resident=fused_resident(rowcx_kernel<T,M,RP,Op>,(int) nt,lds);
+    // a block's rows within one buffer of 2^31 bytes: all of them in one
+    // launch unless the row stride is enormous (then as many as fit)
+    const size_t fit=rows_in_buffer(rs,sizeof(cplx<T>));
+    const size_t step=rpb <= fit ? rows : fit;
+    for(size_t r0=0; r0 < rows; r0 += step) {
+      const size_t n=std::min(step,rows-r0);
+      const size_t nb=std::min((n+rpb-1)/rpb,resident);
+      hipLaunchKernelGGL((rowcx_kernel<T,M,RP,Op>),dim3((unsigned) nb),dim3((unsigned) nt),lds,st,
+                         a,(const cplx<T> *) f+r0*rs,(const cplx<T> *) g+r0*rs,(int64_t) r0,
+                         (int64_t) n,(int64_t) rs,(cplx<T> *) out+r0*os,(int64_t) os,(T) scale,op);
+      if(const int rc=fused_status(hipGetLastError())) return rc;
+    }
+    return 0;
+  }
 }
 
-// Hermitian rows of M = 512 ... 2048 on the packed kernel (f + i g in one
+// Hermitian rows of M = 16 ... 2048 on the packed kernel (f + i g in one
 // transform per residue), persistent grid.
 template<typename T, int M, class Op>
 inline int hrowpk_launch(const DimArgs &a, const void *f, const void *g, size_t rows,
@@ -141,10 +169,15 @@ inline int rowreg_launch(const DimArgs &a, const void *f, const void *g, size_t 
 {
   constexpr int TPS=M/RowV::V;
   const int64_t passes=HERM ? (a.q+1)/2 : a.q;
-  // Hermitian rows of 512 ... 2048 points with enough rows to fill the chip:
-  // the packed kernel (measured 12-28% faster than rowreg_kernel there)
-  if constexpr(HERM && M >= 512 && M <= 2048)
-    if(rows >= 512) return hrowpk_launch<T,M>(a,f,g,rows,rs,out,os,scale,op,st);
+  // Hermitian rows of up to 2048 points with enough rows to fill the chip:
+  // the packed kernel (rowreg_kernel takes 1.3 to 1.5 times as long there:
+  // 73728 rows of H = M = 128, q = 3, FP64 207 against 297 us, 36864 of 256
+  // 205 against 302 us, FP32 99 against 140 us), whose block reads its rows
+  // through one buffer and whose residue twiddles stay within 16 KB of LDS
+  if constexpr(HERM && M <= 2048)
+    if(rows >= 512 && (size_t) HRowPk<T,M>::SLOTS <= rows_in_buffer(rs,sizeof(cplx<T>)) &&
+       (size_t) a.q*(RowV::V+1)*sizeof(cplx<T>) <= 16*1024)
+      return hrowpk_launch<T,M>(a,f,g,rows,rs,out,os,scale,op,st);
   if(TPS <= 256 && rows < 512 && passes >= 2)
     return rowreg_launch_rp<T,M,HERM,2>(a,f,g,rows,rs,out,os,scale,op,st);
   return rowreg_launch_rp<T,M,HERM,1>(a,f,g,rows,rs,out,os,scale,op,st);

@@ -18,6 +18,7 @@
 // after the inverse with the mirror element Z(M - sigma), fetched through the
 // slot's LDS exchange area.
 #pragma once
+#include <type_traits>
 #include "batch.h"
 
 namespace fftwpp_amd {
@@ -67,13 +68,142 @@ __device__ __forceinline__ void rowreg_combine(cplx<T> *acc, T *xbase, T *xb,
   }
 }
 
-// Dynamic LDS: M complex twiddles + slots * 2 RPlan<M,V>::PAD scalar words
+// Complex or centred rows.  Thread t of a row's slot keeps element sigma =
+// t + TPS k at index j = (sigma - k0) mod M of the row (j >= L: zero padding).
+//
+// Loads go through a buffer over the block's rows (one 32-bit offset per
+// thread; zero padding is an offset past the end, which reads 0), all issued
+// together.  The host keeps the span of a block's rows below 2^31 bytes.
+//
+// RP = 1: each slot owns a row (one slot per block when TPS > 64).  RP > 1:
+// the block holds one row and its RP slots take every RP-th residue; their
+// sums are added through LDS before the row is written.  Dynamic LDS: M
+// complex twiddles + slots * 2 RPlan<M,V>::PAD scalar words.
+//
+// Bound by the chain of LDS exchanges at two waves per SIMD (FP64: 176-218
+// registers; a bound of three waves spills, and loading the next row ahead
+// costs more registers than it hides).  The branch-free loads, one register
+// per exchange instead of one per access and the product chosen once per row
+// took 65536 rows of 120 points (q = 2, FP64) from 152 to 126 us, 2048 rows of
+// 1000 points padded to 2048 from 56 to 49 us (FP64) and 31.5 to 25.6 us
+// (FP32), one such row from 10.1 to 9.0 us.
+// W: waves per SIMD asked of the compiler; the short FP32 rows of the
+// library's own products fit four without spills (66 against 73 us with two at
+// M = 128); a caller's functor keeps the registers of two.
+template<typename T, int M, int RP, class Op> struct RowCx {
+  static constexpr int W=sizeof(T) == 4 && RP*M <= 512 && std::is_same<Op,RunMult>::value ? 4 : 2;
+};
+template<typename T, int M, int RP, class Op>
+__global__ void __launch_bounds__(RP*M/RowV::V > 256 ? 512 : 256,(RowCx<T,M,RP,Op>::W))
+rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_t rows,
+             int64_t rs, cplx<T> *out, int64_t os, T scale, Op op)
+{
+  constexpr int V=RowV::V;
+  typedef RPlan<M,V> P;
+  constexpr int TPS=P::TPS;
+  constexpr unsigned E=sizeof(cplx<T>);
+  extern __shared__ char smem_raw[];
+  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
+  const cplx<T> *zN=(const cplx<T> *) d.zN;
+  const int slots=RP > 1 ? 1 : blockDim.x/TPS;      // rows per block
+  const int slot=threadIdx.x/TPS, t=threadIdx.x-slot*TPS;
+  const int rp=RP > 1 ? slot : 0;                     // residue lane
+  const int rslot=RP > 1 ? 0 : slot;
+  T *xbase=reinterpret_cast<T *>(tw+M);
+  T *xb=xbase+slot*2*P::PAD;
+  const int q=(int) d.q, L=(int) d.L, k0=(int) d.k0;
+  cplx<T> a[V], b[V];
+  // the words of the slot's row of the block's rows from rb on
+  auto load=[&](int64_t rb) {
+    const int64_t nr=rows-rb < slots ? rows-rb : slots;
+    const size_t words=(size_t) ((nr-1)*rs+L);
+    const __amdgpu_buffer_rsrc_t rf=buf_rsrc(f+rb*rs,words), rg=buf_rsrc(g+rb*rs,words);
+    const unsigned ro=(unsigned) rslot*(unsigned) rs*E;
+#pragma unroll
+    for(int k=0; k < V; ++k) {
+      const int j=(t+TPS*k-k0) & (M-1);    // k0 <= 0, M a power of two
+      const unsigned o=j < L ? ro+(unsigned) j*E : 0x80000000u;   // past the end: reads 0
+      a[k]=ld_buf<T>(rf,o,0);
+      b[k]=ld_buf<T>(rg,o,0);
+    }
+  };
+  const int64_t step=(int64_t) gridDim.x*slots;
+  int64_t rb=(int64_t) blockIdx.x*slots;
+  fill_twr<T,M,V>(tw,zN,q,threadIdx.x,blockDim.x);
+  __syncthreads();
+  for(; rb < rows; rb += step) {
+    const int64_t row=rb+rslot;
+    cplx<T> acc[V];
+#pragma unroll
+    for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
+    for(int r=rp; r < q; r += RP) {
+      // w_N^{(j+k0) r}: j + k0 is sigma or sigma - M
+      const cplx<T> bt=zN[t*r], zm=conjg(zN[M*r]);
+      cplx<T> X[V], Y[V];
+      load(rb);
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        const int sigma=t+TPS*k;
+        const int j=(sigma-k0) & (M-1);
+        cplx<T> u=a[k], v=b[k];
+        if(r) {
+          cplx<T> w=bt*zN[TPS*k*r];
+          if(j+k0 < 0) w=w*zm;
+          u=w*u;
+          v=w*v;
+        }
+        X[k]=u;
+        Y[k]=v;
+      }
+      fftr_pair<T,M,V,1>(X,Y,xb,tw,t);
+      if constexpr(std::is_same<Op,RunMult>::value) {
+        // one uniform branch, not a choice per element
+        if(op.mult == 1) {
+#pragma unroll
+          for(int k=0; k < V; ++k) X[k]=X[k]*Y[k];
+        } else if(op.mult == 3) {
+#pragma unroll
+          for(int k=0; k < V; ++k) X[k]=mulc(X[k],Y[k]);
+        }
+      } else {
+        const auto rop=bind_row(op,row0+row);
+#pragma unroll
+        for(int k=0; k < V; ++k) X[k]=rop(X[k],Y[k],q*(t+TPS*k)+r);
+      }
+      fftr<T,M,V,-1,true>(X,xb,tw,t);
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        if(r) {
+          const int sigma=t+TPS*k;
+          const int j=(sigma-k0) & (M-1);
+          cplx<T> w=bt*zN[TPS*k*r];
+          if(j+k0 < 0) w=w*zm;
+          acc[k]=acc[k]+mulc(X[k],w);
+        } else
+          acc[k]=acc[k]+X[k];
+      }
+    }
+    rowreg_combine<T,M,RP>(acc,xbase,xb,rp,t);
+    if(rp == 0 && row < rows) {
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        const int sigma=t+TPS*k;
+        const int j=(sigma-k0) & (M-1);
+        if(j < L) out[row*os+j]=scale*acc[k];
+      }
+    }
+    if(RP > 1) __syncthreads();          // exchange areas are reused by the next row
+  }
+}
+
+// Hermitian rows (the rows that hrowpk_kernel below leaves: M = 4096, few
+// rows).  Dynamic LDS: M complex twiddles + slots * 2 RPlan<M,V>::PAD scalar words
 // (each slot's exchange area holds a whole complex sequence, so every
 // exchange is one round).
 // RP = 1: each slot owns a row (one slot per block when TPS > 64).  RP > 1:
 // the block holds one row and its RP slots take every RP-th residue (pair);
 // their sums are added through LDS before the row is written.
-template<typename T, int M, bool HERM, int RP, class Op>
+template<typename T, int M, int RP, class Op>
 __global__ void __launch_bounds__(512)
 rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
               int64_t rs, cplx<T> *out, int64_t os, T scale, Op op)
@@ -91,7 +221,7 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
   const int rp=RP > 1 ? slot : 0;                     // residue lane
   T *xbase=reinterpret_cast<T *>(tw+M);
   T *xb=xbase+slot*2*P::PAD;
-  const int q=(int) d.q, L=(int) d.L, H=(int) d.H, k0=(int) d.k0;
+  const int q=(int) d.q, H=(int) d.H;
   for(int64_t rb=(int64_t) blockIdx.x*slots; rb < rows; rb += (int64_t) gridDim.x*slots) {
     const int64_t row=rb+(RP > 1 ? 0 : slot);
     if(row >= rows) break;               // uniform over the block when RP > 1
@@ -99,136 +229,81 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
-    if constexpr(!HERM) {
-      for(int r=rp; r < q; r += RP) {
-        // w_N^{(j+k0) r}: j + k0 is sigma or sigma - M
-        const cplx<T> bt=zN[t*r], zm=conjg(zN[M*r]);
-        cplx<T> X[V], Y[V];
+    for(int r1=2*rp; r1 < q; r1 += 2*RP) {
+      const int r2=r1+1 < q ? r1+1 : -1;
+      // w_N^{sigma r} = w_N^{t r} w_N^{TPS k r}; w_N^{(sigma - M) r} adds
+      // the factor conj w_N^{M r}
+      const cplx<T> zero=mk((T) 0,(T) 0);
+      const cplx<T> b1=zN[t*r1], m1=conjg(zN[M*r1]);
+      const cplx<T> b2=r2 >= 0 ? zN[t*r2] : zero, m2=r2 >= 0 ? conjg(zN[M*r2]) : zero;
+      cplx<T> X[V], Y[V];
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        const int sigma=t+TPS*k;
+        const cplx<T> w1=b1*zN[TPS*k*r1];
+        const cplx<T> w2=r2 >= 0 ? b2*zN[TPS*k*r2] : zero;
+        cplx<T> a=mk((T) 0,(T) 0), b=a;
+        // k = sigma (when < H) and k = sigma - M (when > -H)
+        if(sigma < H) {
+          const cplx<T> w=w1+muli(w2,1);
+          a=w*fr[sigma];
+          b=w*gr[sigma];
+        }
+        if(M-sigma < H) {
+          const cplx<T> w=w1*m1+muli(w2*m2,1);
+          a=a+w*conjg(fr[M-sigma]);
+          b=b+w*conjg(gr[M-sigma]);
+        }
+        X[k]=a;
+        Y[k]=b;
+      }
+      fftr<T,M,V,1,true>(X,xb,tw,t);
+      fftr<T,M,V,1,true>(Y,xb,tw,t);
+      {
+        const auto rop=bind_row(op,row);
 #pragma unroll
         for(int k=0; k < V; ++k) {
-          const int sigma=t+TPS*k;
-          const int j=(sigma-k0) & (M-1);      // k0 <= 0, M a power of two
-          cplx<T> a=mk((T) 0,(T) 0), b=a;
-          if(j < L) {
-            a=fr[j];
-            b=gr[j];
-            if(r) {
-              cplx<T> w=bt*zN[TPS*k*r];
-              if(j+k0 < 0) w=w*zm;
-              a=w*a;
-              b=w*b;
-            }
-          }
-          X[k]=a;
-          Y[k]=b;
-        }
-        fftr_pair<T,M,V,1>(X,Y,xb,tw,t);
-        {
-          const auto rop=bind_row(op,row);
-#pragma unroll
-          for(int k=0; k < V; ++k) X[k]=rop(X[k],Y[k],q*(t+TPS*k)+r);
-        }
-        fftr<T,M,V,-1,true>(X,xb,tw,t);
-#pragma unroll
-        for(int k=0; k < V; ++k) {
-          const int sigma=t+TPS*k;
-          const int j=(sigma-k0) & (M-1);
-          if(j < L) {
-            if(r) {
-              cplx<T> w=bt*zN[TPS*k*r];
-              if(j+k0 < 0) w=w*zm;
-              acc[k]=acc[k]+mulc(X[k],w);
-            } else
-              acc[k]=acc[k]+X[k];
-          }
+          const int l=q*(t+TPS*k);
+          X[k]=mk(rop(X[k].x,Y[k].x,l+r1),r2 >= 0 ? rop(X[k].y,Y[k].y,l+r2) : (T) 0);
         }
       }
-      rowreg_combine<T,M,RP>(acc,xbase,xb,rp,t);
-      if(rp == 0) {
+      fftr<T,M,V,-1,true>(X,xb,tw,t);
+      // mirror elements Z(M - sigma) through LDS
+      cplx<T> Zm[V];
 #pragma unroll
-        for(int k=0; k < V; ++k) {
-          const int sigma=t+TPS*k;
-          const int j=(sigma-k0) & (M-1);
-          if(j < L) out[row*os+j]=scale*acc[k];
+      for(int k=0; k < V; ++k) {
+        const int e=xidx<T,M,V>(t+TPS*k);
+        xb[e]=X[k].x;
+        xb[P::PAD+e]=X[k].y;
+      }
+      rsync<TPS>();
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        const int e=xidx<T,M,V>((M-(t+TPS*k)) & (M-1));
+        Zm[k]=mk(xb[e],xb[P::PAD+e]);
+      }
+      rsync<TPS>();
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        const int sigma=t+TPS*k;
+        if(sigma < H) {
+          const cplx<T> z=X[k], zc=conjg(Zm[k]);
+          const cplx<T> y1=(T) 0.5*(z+zc);
+          cplx<T> v=mulc(y1,b1*zN[TPS*k*r1]);
+          if(r2 >= 0) {
+            const cplx<T> y2=muli((T) 0.5*(z-zc),-1);
+            v=v+mulc(y2,b2*zN[TPS*k*r2]);
+          }
+          acc[k]=acc[k]+v;
         }
       }
-    } else {
-      for(int r1=2*rp; r1 < q; r1 += 2*RP) {
-        const int r2=r1+1 < q ? r1+1 : -1;
-        // w_N^{sigma r} = w_N^{t r} w_N^{TPS k r}; w_N^{(sigma - M) r} adds
-        // the factor conj w_N^{M r}
-        const cplx<T> zero=mk((T) 0,(T) 0);
-        const cplx<T> b1=zN[t*r1], m1=conjg(zN[M*r1]);
-        const cplx<T> b2=r2 >= 0 ? zN[t*r2] : zero, m2=r2 >= 0 ? conjg(zN[M*r2]) : zero;
-        cplx<T> X[V], Y[V];
+    }
+    rowreg_combine<T,M,RP>(acc,xbase,xb,rp,t);
+    if(rp == 0) {
 #pragma unroll
-        for(int k=0; k < V; ++k) {
-          const int sigma=t+TPS*k;
-          const cplx<T> w1=b1*zN[TPS*k*r1];
-          const cplx<T> w2=r2 >= 0 ? b2*zN[TPS*k*r2] : zero;
-          cplx<T> a=mk((T) 0,(T) 0), b=a;
-          // k = sigma (when < H) and k = sigma - M (when > -H)
-          if(sigma < H) {
-            const cplx<T> w=w1+muli(w2,1);
-            a=w*fr[sigma];
-            b=w*gr[sigma];
-          }
-          if(M-sigma < H) {
-            const cplx<T> w=w1*m1+muli(w2*m2,1);
-            a=a+w*conjg(fr[M-sigma]);
-            b=b+w*conjg(gr[M-sigma]);
-          }
-          X[k]=a;
-          Y[k]=b;
-        }
-        fftr<T,M,V,1,true>(X,xb,tw,t);
-        fftr<T,M,V,1,true>(Y,xb,tw,t);
-        {
-          const auto rop=bind_row(op,row);
-#pragma unroll
-          for(int k=0; k < V; ++k) {
-            const int l=q*(t+TPS*k);
-            X[k]=mk(rop(X[k].x,Y[k].x,l+r1),r2 >= 0 ? rop(X[k].y,Y[k].y,l+r2) : (T) 0);
-          }
-        }
-        fftr<T,M,V,-1,true>(X,xb,tw,t);
-        // mirror elements Z(M - sigma) through LDS
-        cplx<T> Zm[V];
-#pragma unroll
-        for(int k=0; k < V; ++k) {
-          const int e=xidx<T,M,V>(t+TPS*k);
-          xb[e]=X[k].x;
-          xb[P::PAD+e]=X[k].y;
-        }
-        rsync<TPS>();
-#pragma unroll
-        for(int k=0; k < V; ++k) {
-          const int e=xidx<T,M,V>((M-(t+TPS*k)) & (M-1));
-          Zm[k]=mk(xb[e],xb[P::PAD+e]);
-        }
-        rsync<TPS>();
-#pragma unroll
-        for(int k=0; k < V; ++k) {
-          const int sigma=t+TPS*k;
-          if(sigma < H) {
-            const cplx<T> z=X[k], zc=conjg(Zm[k]);
-            const cplx<T> y1=(T) 0.5*(z+zc);
-            cplx<T> v=mulc(y1,b1*zN[TPS*k*r1]);
-            if(r2 >= 0) {
-              const cplx<T> y2=muli((T) 0.5*(z-zc),-1);
-              v=v+mulc(y2,b2*zN[TPS*k*r2]);
-            }
-            acc[k]=acc[k]+v;
-          }
-        }
-      }
-      rowreg_combine<T,M,RP>(acc,xbase,xb,rp,t);
-      if(rp == 0) {
-#pragma unroll
-        for(int k=0; k < V; ++k) {
-          const int sigma=t+TPS*k;
-          if(sigma < H) out[row*os+sigma]=scale*acc[k];
-        }
+      for(int k=0; k < V; ++k) {
+        const int sigma=t+TPS*k;
+        if(sigma < H) out[row*os+sigma]=scale*acc[k];
       }
     }
     if(RP > 1) __syncthreads();          // exchange areas are reused by the next row
@@ -250,7 +325,7 @@ template<typename T, int M>
 __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buffer_rsrc_t rf,
                                           __amdgpu_buffer_rsrc_t rg, const cplx<T> *tr1,
                                           const cplx<T> *tr2, cplx<T> b1, cplx<T> b2, int t,
-                                          int r1, int r2, int H)
+                                          int r1, int r2, int H, unsigned ro)
 {
   constexpr int V=RowV::V, TPS=M/V;
   constexpr unsigned E=sizeof(cplx<T>);
@@ -260,7 +335,7 @@ __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buf
   for(int k=0; k < V; ++k) {
     const int sigma=t+TPS*k;
     const bool iu=sigma < H, iv=M-sigma < H;
-    const unsigned ou=(unsigned) (iu ? sigma : 0)*E, ov=(unsigned) (iv ? M-sigma : 0)*E;
+    const unsigned ou=ro+(unsigned) (iu ? sigma : 0)*E, ov=ro+(unsigned) (iv ? M-sigma : 0)*E;
     const cplx<T> fu=ld_buf<T>(rf,ou,0), gu=ld_buf<T>(rg,ou,0);
     const cplx<T> fv=ld_buf<T>(rf,ov,0), gv=ld_buf<T>(rg,ov,0);
     const cplx<T> u=iu ? mk(fu.x-gu.y,fu.y+gu.x) : zero;
@@ -273,8 +348,9 @@ __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buf
   }
 }
 
-// Hermitian rows with H <= M and TPS = M/8 >= 64 (M >= 512), SLOTS = 256/TPS
-// rows per block of 256 threads (M = 1024: two rows of two waves).  The
+// Hermitian rows with H <= M <= 2048, SLOTS = 256/TPS rows per block of 256
+// threads (M = 1024: two rows of two waves; M = 128: sixteen rows, four to a
+// wave).  The
 // forward transforms of f and g share one complex FFT per residue: the fold
 // U_r of f + i g (hpk_fold2) transforms to F_r + i G_r with F_r, G_r real
 // (the folds of Hermitian data are Hermitian), so P_r = F_r G_r is
@@ -283,7 +359,8 @@ __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buf
 // P_{r1} + i P_{r2}, and unpacked with the mirror element Z(M - sigma) as in
 // rowreg_kernel (backward2, convolve.cc:4749-4843): q forward and ceil(q/2)
 // inverse transforms per row instead of 3 ceil(q/2).  Rows are read through
-// buffer resources (a 32-bit offset per element) and the uniform residue
+// buffer resources (a 32-bit offset per element; over one row when a slot is
+// whole waves, else over the block's rows with the row's offset per lane) and the uniform residue
 // twiddles w_N^{TPS k r} come from an LDS table, which keeps addresses and
 // twiddles out of the registers that the residue loop carries.  Slots past
 // the last row run on row rows - 1 without storing (the block barriers of the
@@ -310,7 +387,6 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
 {
   typedef HRowPk<T,M> K;
   constexpr int V=K::V, TPS=K::TPS, SLOTS=K::SLOTS;
-  static_assert(TPS >= 64, "a slot spans whole waves");
   typedef RPlan<M,V> P;
   constexpr unsigned E=sizeof(cplx<T>);
   extern __shared__ char smem_raw[];
@@ -324,15 +400,21 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
     tq[e]=zN[TPS*k*r];                        // TPS k r <= M r < N
   }
   __syncthreads();
-  // a slot spans whole waves: its index is uniform over the wave
-  const int slot=__builtin_amdgcn_readfirstlane((int) threadIdx.x)/TPS;
+  // a slot of whole waves: its index is uniform over the wave
+  int slot=(int) threadIdx.x/TPS;
+  if constexpr(TPS >= 64) slot=__builtin_amdgcn_readfirstlane(slot);
   const int t=threadIdx.x-slot*TPS;
   T *xb=reinterpret_cast<T *>(tq+q*(V+1))+slot*2*P::PAD;
   for(int64_t rb=(int64_t) blockIdx.x*SLOTS; rb < rows; rb += (int64_t) gridDim.x*SLOTS) {
     const int64_t row=rb+slot;
     const bool live=row < rows;
+    // buffers over the row (slots of whole waves), or over the rows of the
+    // block with the row's offset per lane
     const int64_t rr=live ? row : rows-1;
-    const __amdgpu_buffer_rsrc_t rf=buf_rsrc(f+rr*rs,H), rg=buf_rsrc(g+rr*rs,H);
+    const int64_t b0=TPS >= 64 ? rr : rb;
+    const size_t nw=TPS >= 64 ? (size_t) H : (size_t) ((rows-1 < rb+SLOTS-1 ? rows-1-rb : SLOTS-1)*rs+H);
+    const unsigned ro=TPS >= 64 ? 0 : (unsigned) ((rr-rb)*rs)*E;
+    const __amdgpu_buffer_rsrc_t rf=buf_rsrc(f+b0*rs,nw), rg=buf_rsrc(g+b0*rs,nw);
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
@@ -344,7 +426,7 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
       cplx<T> X[V], X2[V];
       T p1[V];
       hpk_fold2<T,M>(X,X2,rf,rg,tq+r1*(V+1),tq+(r2 >= 0 ? r2 : r1)*(V+1),b1,
-                     r2 >= 0 ? zN[t*r2] : b1,t,r1,r2 >= 0 ? r2 : r1,H);
+                       r2 >= 0 ? zN[t*r2] : b1,t,r1,r2 >= 0 ? r2 : r1,H,ro);
       if(r2 >= 0) {
         // the two residues' transforms with their butterflies interleaved
         fftr_pair<T,M,V,1>(X,X2,xb,tw,t);
@@ -380,10 +462,17 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
       rsync<TPS>();
     }
     if(live) {
-      const __amdgpu_buffer_rsrc_t ro=buf_rsrc(out+row*os,H);
+      if constexpr(TPS >= 64) {
+        const __amdgpu_buffer_rsrc_t rw=buf_rsrc(out+row*os,H);
 #pragma unroll
-      for(int k=0; k < V; ++k)
-        if(t+TPS*k < H) st_buf<T>(ro,(unsigned) (t+TPS*k)*E,0,scale*acc[k]);
+        for(int k=0; k < V; ++k)
+          if(t+TPS*k < H) st_buf<T>(rw,(unsigned) (t+TPS*k)*E,0,scale*acc[k]);
+      } else {
+        cplx<T> *orow=out+row*os;
+#pragma unroll
+        for(int k=0; k < V; ++k)
+          if(t+TPS*k < H) orow[t+TPS*k]=scale*acc[k];
+      }
     }
   }
 }
@@ -522,8 +611,8 @@ hrows_reduce_kernel(const cplx<T> *part, int64_t rows, int H, int passes,
 // TPS threads of a column span waves and exchange with block barriers, one
 // round per stage, through the column's LDS area of CS = 2 PAD + X words
 // (real parts, then imaginary parts PAD words on).  Element e of column c
-// sits at word base(e) ^ (c BETA mod 32), base being the identity or the
-// row kernels' swizzle (both keep words below M): the (base, X, BETA) of each
+// sits at word base(e) ^ (c BETA mod 32), base being the identity or an XOR
+// swizzle (both keep words below M): the (base, X, BETA) of each
 // size were found
 // by an exhaustive search under the gfx950 LDS bank model (64-bit words:
 // writes 16 lanes per pass over 32 banks, reads 32 lanes over 64 banks;
@@ -537,7 +626,7 @@ template<typename T, int M> struct ColReg {
   static constexpr int TC=TPS >= 512 ? 1 : (512/TPS < 64 ? 512/TPS : 64);
   static constexpr int PAD=RPlan<M,V>::PAD;
   static constexpr bool F64=sizeof(T) == 8;
-  // base: 0 identity, 2 swizzle (xidx)
+  // base: 0 identity, 2 swizzle
   static constexpr int BASE=M >= 1024 ? 2 : 0;
   static constexpr int X=M == 16 ? 1 : 0;
   static constexpr int BETA=M == 16 || M == 4096 ? 0 : M == 256 ? (F64 ? 17 : 2) : M == 512 ? 9 :
@@ -546,9 +635,12 @@ template<typename T, int M> struct ColReg {
   static constexpr int NT=TPS*TC;
   static __device__ __forceinline__ int at(int e)
   {
-    if constexpr(BASE == 2) return xidx<T,M,V>(e);
+    if constexpr(BASE == 2 && F64) return e ^ ((e >> 4) & 7) ^ (((e >> 6) & 1) << 3);
+    else if constexpr(BASE == 2) return e ^ ((e >> 5) & 7) ^ (((e >> 6) & 3) << 3);
     else return e;
   }
+  // both maps are linear over the bits of e (M >= 1024 swizzles)
+  static __device__ __forceinline__ int join(int a, int b) { return a ^ b; }
   // the column's XOR of the word index (M = 16: the words stay below 16)
   static __device__ __forceinline__ int xm(int c) { return (c*BETA) & (M < 32 ? M-1 : 31); }
 };
