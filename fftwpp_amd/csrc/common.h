@@ -135,42 +135,6 @@ __device__ __forceinline__ int64_t xcd_tile(int64_t x, int64_t gx)
   return x < 8*per ? (x % 8)*per+x/8 : x;
 }
 
-// Up to three arrays transformed by one launch (the inputs of a convolution,
-// or the cotangent and both inputs of its adjoint).  Block z of the grid takes
-// array z mod n and every gridDim.z/n-th residue from z/n on.
-constexpr int MAXARRAYS=3;
-
-struct ColArrays {
-  int n;
-  const void *in[MAXARRAYS];
-  void *out[MAXARRAYS];
-};
-
-struct ColBlock {
-  const void *in;
-  void *out;
-  int part, parts;
-};
-
-__device__ __forceinline__ ColBlock col_block(const ColArrays &io)
-{
-  // in scalar registers (a division runs on the vector unit and would take
-  // the pointers with it)
-  const int z=blockIdx.z, n=io.n;
-  const int part=n == 1 ? z : __builtin_amdgcn_readfirstlane(z/n);
-  const int a=z-part*n;
-  ColBlock b;
-  // device memory: as pointers out of a struct they would be taken for
-  // generic ones (flat accesses, more registers)
-  b.in=(const void *) (const __attribute__((address_space(1))) void *)
-    (a == 0 ? io.in[0] : (a == 1 ? io.in[1] : io.in[2]));
-  b.out=(void *) (__attribute__((address_space(1))) void *)
-    (a == 0 ? io.out[0] : (a == 1 ? io.out[1] : io.out[2]));
-  b.part=part;
-  b.parts=n == 1 ? (int) gridDim.z : __builtin_amdgcn_readfirstlane((int) gridDim.z/n);
-  return b;
-}
-
 template<typename T>
 __device__ __forceinline__ cplx<T> ztab(const DimArgs &d, int64_t j)
 {

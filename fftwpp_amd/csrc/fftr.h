@@ -36,8 +36,7 @@ template<int M, int V=16> struct RPlan {
   static constexpr int NV=LOG/LV;                       // radix-V stages
   static constexpr int LAST=1 << (LOG-LV*NV);           // remaining factor
   static constexpr int NST=NV+(LAST > 1 ? 1 : 0);
-  // exchange words (the swizzled sequences of 512 or more use M of them)
-  static constexpr int PAD=M >= 512 ? M : M+M/16;
+  static constexpr int PAD=M+M/16;                      // exchange words
   __host__ __device__ static constexpr int radix(int s) { return s < NV ? V : LAST; }
   // Stage s writes output u of butterfly j at dest<s>(j) + u ns(s); the bits
   // of j move without mixing, so dest(a + b) = dest(a) + dest(b) for a and b
@@ -75,7 +74,7 @@ __device__ __forceinline__ int padr(int e) { return e+(e >> 4); }
 // immediate offset of the access: it has conflicts, but needs 10 to 60 fewer
 // registers and no instructions (complex rows of M = 64 FP64 98 us against
 // 107 swizzled, M = 128 FP32 67 against 91; M = 128 FP64 133 against 126).
-// Indices stay below RPlan::PAD.
+// Indices stay below M + M/16.
 template<typename T, int M, int V>
 __host__ __device__ constexpr bool xswizzled()
 {
@@ -284,24 +283,13 @@ __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
   }
 }
 
-// t as a value that the compiler does not know to be the loop-invariant one:
-// without it the LDS addresses and twiddle positions of every stage, which
-// depend on t alone, are hoisted out of the caller's loop over rows and
-// residues and stay in registers through all of it (30 to 40 of them in a row
-// kernel); computed anew per transform they cost one instruction per access.
-__device__ __forceinline__ int fresh(int t)
-{
-  asm volatile("" : "+v"(t));
-  return t;
-}
-
 // fftr<T,M,V,S,true> of X and of Y, their butterflies interleaved stage by
 // stage; same results, same exchange area and barriers.
 template<typename T, int M, int V, int S>
 __device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const cplx<T> *tw,
                                           int t)
 {
-  fftr_pair_stage<T,M,V,S,0>(X,Y,xb,tw,fresh(t));
+  fftr_pair_stage<T,M,V,S,0>(X,Y,xb,tw,t);
 }
 
 // In-place transform of the sequence held by threads t < TPS (v[V] each)
@@ -311,7 +299,7 @@ __device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const c
 template<typename T, int M, int V, int S, bool CX=false>
 __device__ __forceinline__ void fftr(cplx<T> *v, T *xb, const cplx<T> *tw, int t)
 {
-  fftr_stage<T,M,V,S,0,false,CX>(v,xb,tw,fresh(t));
+  fftr_stage<T,M,V,S,0,false,CX>(v,xb,tw,t);
 }
 
 // The same transform when the threads of a sequence are not consecutive
@@ -320,7 +308,7 @@ template<typename T, int M, int V, int S, bool CX=false>
 __device__ __forceinline__ void fftr_blk(cplx<T> *v, T *xb, const cplx<T> *tw,
                                          int t)
 {
-  fftr_stage<T,M,V,S,0,true,CX>(v,xb,tw,fresh(t));
+  fftr_stage<T,M,V,S,0,true,CX>(v,xb,tw,t);
 }
 
 // fftr_blk with one-round exchanges through the index map XI, XORed by xm.
@@ -328,7 +316,7 @@ template<typename T, int M, int V, int S, class XI>
 __device__ __forceinline__ void fftr_blkx(cplx<T> *v, T *xb, const cplx<T> *tw,
                                           int t, int xm)
 {
-  fftr_stage<T,M,V,S,0,true,true,XI>(v,xb,tw,fresh(t),xm);
+  fftr_stage<T,M,V,S,0,true,true,XI>(v,xb,tw,t,xm);
 }
 
 } // namespace fftwpp_amd

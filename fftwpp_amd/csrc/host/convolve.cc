@@ -14,18 +14,6 @@
 // which engine takes the rows (stage 1) of a dimension (2: register FFT).
 extern "C" int fftwpp_amd_internal_rows_fit(const fftwpp_amd_dim *d, int dtype);
 extern "C" int fftwpp_amd_internal_engine(const fftwpp_amd_dim *d, int stage);
-// the forward residue transforms of up to three arrays of one layout in one launch
-extern "C" int fftwpp_amd_internal_forward_arrays(const fftwpp_amd_dim *d, int dtype, int real,
-                                                  int n, const void *const *f, size_t S,
-                                                  size_t C, size_t nbatch, size_t bstride_in,
-                                                  void *const *F, size_t SF, size_t bstride_out,
-                                                  size_t r0, size_t nres, void *stream);
-extern "C" int fftwpp_amd_internal_backward_arrays(const fftwpp_amd_dim *d, int dtype, int n,
-                                                   const void *const *F, size_t SF,
-                                                   size_t bstride_in, void *const *f, size_t S,
-                                                   size_t C, size_t nbatch, size_t bstride_out,
-                                                   size_t r0, size_t nres, int accumulate,
-                                                   double scale, void *stream);
 // the item table {i rs, L, i L} of `rows` rows for the batched row kernel
 extern "C" int fftwpp_amd_internal_row_items(void *items, size_t rows, size_t rs,
                                              size_t L, void *stream);
@@ -1051,11 +1039,13 @@ static void fusedRows(fftBase *fft, DeviceWork &work, size_t slot, int dtype,
   }
   if(tps) {
     // complex rows longer than one block of a power-of-two m: the batched
-    // register kernel with the rows as items (row i at i rs) in the sequence
-    // mode: every residue of every row is a work unit that writes its m words
-    // to a buffer, and the second launch folds a row's q sequences into out.
-    // out may alias f or g: it is written after every unit has read its row.
-    const size_t L=fft->L, q=fft->q, m=fft->m;
+    // register kernel with the rows as items (row i at i rs).  The residues
+    // always go to partial sums that its second launch adds into out (at
+    // least two groups when q > 1), since out may alias f or g and a unit
+    // that wrote its outputs would re-read them in its next residue's fold:
+    // one residue per unit when rows are few, two groups otherwise.
+    const size_t L=fft->L, q=fft->q;
+    const size_t D=rows >= 512 ? (q+1)/2 : 1;
     void *items=work.get(slot+1,rows*3*sizeof(int64_t));
     const std::vector<size_t> key={rows,rs,L};
     if(work.keys[slot+1] != key) {
@@ -1063,9 +1053,11 @@ static void fusedRows(fftBase *fft, DeviceWork &work, size_t slot, int dtype,
       check(fftwpp_amd_internal_row_items(items,rows,rs,L,stream),"item table");
       work.keys[slot+1]=key;
     }
-    void *part=work.get(slot,rows*q*m*(dtype == FFTWPP_AMD_F32 ? 8 : 16));
+    const size_t G=(q+D-1)/D;
+    void *part=G > 1 ? work.get(slot,G*rows*L*(dtype == FFTWPP_AMD_F32 ? 8 : 16)) : NULL;
+    const size_t units=rows*G;
     check(fftwpp_amd_batch_rows(fft->dev,dtype,code,items,rows,f,g,out,1,
-                                tps < 64 ? 64 : tps,std::min<size_t>(rows*q,2048),0,0,
+                                tps < 64 ? 64 : tps,std::min<size_t>(units,2048),0,D,
                                 part,rows*L,s,stream),what);
     return;
   }
@@ -1318,11 +1310,11 @@ void Convolution2::execComplex(void *out, const void *f0, const void *f1, bool n
     const size_t nres=std::min(Dx,qx-r0);
     const size_t rows=real ? maxrows : nres*mx;
     const bool first=r0 == 0, last=r0+nres == qx;
-    // both inputs in one launch, unless their stages are timed one by one
-    const int na=timeline ? 1 : 2;
-    for(int a=0; a < 2; a += na) {
-      check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,real,na,in+a,Sx,lyc,1,0,F+a,lyc,0,
-                                               r0,nres,stream),"x forward");
+    for(int a=0; a < 2; ++a) {
+      if(real)
+        check(fftwpp_amd_forward_real_many(fftx->dev,dtype,in[a],Sx,lyc,1,0,F[a],lyc,0,stream),"x forward");
+      else
+        check(fftwpp_amd_forward_many(fftx->dev,dtype,in[a],Sx,lyc,1,0,F[a],lyc,0,r0,nres,stream),"x forward");
       if(timeline) timeline->mark(real ? (a == 0 ? "x real forward f" : "x real forward g") : (a == 0 ? "x forward f" : "x forward g"));
     }
     if(rowHook)
@@ -1341,28 +1333,6 @@ void Convolution2::execComplex(void *out, const void *f0, const void *f1, bool n
                                      last ? s : 1.0,stream),"x backward");
     if(timeline) timeline->mark(real ? "x real backward" : "x backward");
   }
-}
-
-bool Convolution2::execShared(void *const out[2], const void *w, const void *const g[2],
-                              bool normalize, int dtype, void *stream, int mult)
-{
-  const int code=mult >= 0 ? mult : multCode;
-  requireBinary(A,B,code);
-  if(fftx->realInput() || memoryLimit || timeline || rowHook || ffty->C != 1 ||
-     !rowsSupported(ffty,dtype))
-    return false;
-  const size_t q=fftx->q, rows=q*fftx->m, bytes=rows*ly*eltsize(dtype);
-  const void *in[3]={w,g[0],g[1]};
-  void *F[3]={work.get(0,bytes),work.get(1,bytes),work.get(11,bytes)};
-  check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,0,3,in,Sx,ly,1,0,F,ly,0,0,q,stream),
-        "x forward");
-  // every row is read whole before it is written: the product may replace the
-  // second factor
-  for(int k=1; k < 3; ++k)
-    fusedRows(ffty,work,2,dtype,code,F[0],F[k],rows,ly,F[k],ly,1.0,stream,"y rows");
-  check(fftwpp_amd_internal_backward_arrays(fftx->dev,dtype,2,F+1,ly,0,out,Sx,ly,1,0,0,q,0,
-                                            normalize ? scale : 1.0,stream),"x backward");
-  return true;
 }
 
 // Work bytes of an execution with Dx x residues per pass (0: all): the two
@@ -1568,23 +1538,18 @@ void Convolution3::execComplex(void *out, const void *f0, const void *f1, bool n
     const size_t nres=std::min(Dx,qx-r0);
     const size_t nplanes=real ? maxplanes : nres*mx;
     const bool first=r0 == 0, last=r0+nres == qx;
-    // x forward: columns (y,z); non-contiguous y strides become batches.  Both
-    // inputs in one launch (one long tail per stage instead of two: 255 x 255 x
-    // 128 Hermitian modes FP64 1023 -> 999 us), unless their stages are timed
-    // one by one or an x-transformed array exceeds the 256 MB Infinity Cache:
-    // then f's y stage runs at once on what its x stage left there (real 256^3
-    // FP64, 270 MB: 1204 us against 1257 us paired).
-    const int na=timeline || nplanes*plane*E > ((size_t) 256 << 20) ? 1 : 2;
-    for(int a=0; a < 2; a += na) {
-      if(contiguous())
-        check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,real,na,in+a,Sx,plane,1,0,X+a,plane,0,
-                                                 r0,nres,stream),"x forward");
+    // x forward: columns (y,z); non-contiguous y strides become batches
+    for(int a=0; a < 2; ++a) {
+      if(real && contiguous())
+        check(fftwpp_amd_forward_real_many(fftx->dev,dtype,in[a],Sx,plane,1,0,X[a],plane,0,stream),"x forward");
+      else if(real)
+        check(fftwpp_amd_forward_real_many(fftx->dev,dtype,in[a],Sx,Lz,Ly,Sy,X[a],plane,Lz,stream),"x forward");
+      else if(contiguous())
+        check(fftwpp_amd_forward_many(fftx->dev,dtype,in[a],Sx,plane,1,0,X[a],plane,0,r0,nres,stream),"x forward");
       else
-        check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,real,na,in+a,Sx,Lz,Ly,Sy,X+a,plane,Lz,
-                                                 r0,nres,stream),"x forward");
+        check(fftwpp_amd_forward_many(fftx->dev,dtype,in[a],Sx,Lz,Ly,Sy,X[a],plane,Lz,r0,nres,stream),"x forward");
       if(timeline) timeline->mark(real ? (a == 0 ? "x real forward f" : "x real forward g") : (a == 0 ? "x forward f" : "x forward g"));
-      check(fftwpp_amd_internal_forward_arrays(ffty->dev,dtype,0,na,X+a,Lz,Lz,nplanes,plane,Y+a,Lz,yplane,
-                                               0,qy,stream),"y forward");
+      check(fftwpp_amd_forward_many(ffty->dev,dtype,X[a],Lz,Lz,nplanes,plane,Y[a],Lz,yplane,0,qy,stream),"y forward");
       if(timeline) timeline->mark(a == 0 ? "y forward f" : "y forward g");
     }
     if(rowHook)

@@ -646,13 +646,12 @@ __global__ void symxy3_kernel(int64_t Hx, int64_t Hy, int64_t Hz, int64_t x0,
 // ------------------------------------------------------------------------
 template<typename T>
 __global__ void hplane_kernel(int op, int64_t Hx, int64_t Hy, int64_t x0,
-                              int64_t y0, ColArrays io, int64_t Sx, int64_t Sy)
+                              int64_t y0, cplx<T> *f, int64_t Sx, int64_t Sy)
 {
   int64_t t=(int64_t) blockIdx.x*blockDim.x+threadIdx.x;
   if(t >= (2*Hx-1)*Hy) return;
   const int64_t i=t/Hy-(Hx-1), j=t % Hy;
   if(j == 0 && i < 0) return;
-  cplx<T> *f=(cplx<T> *) (blockIdx.y == 0 ? io.out[0] : (blockIdx.y == 1 ? io.out[1] : io.out[2]));
   cplx<T> *u=f+(x0+i)*Sx+(y0+j)*Sy;
   if(i == 0 && j == 0) {
     const cplx<T> v=*u;
@@ -668,36 +667,6 @@ __global__ void hplane_kernel(int op, int64_t Hx, int64_t Hy, int64_t x0,
     *u=a+conjg(b);
     *l=b+conjg(a);
   } else *l=mk((T) 0,(T) 0);
-}
-
-// Copies of whole arrays of `words` words (element (x, y) of the plane at x Sx
-// + y Sy, Sx a multiple of Sy) with plane operation 0 (symmetrize) applied to
-// array z of the grid, or operation 1 where bit z of ops1 is set: one pass
-// where a copy and a launch on the plane took two.
-template<typename T>
-__global__ void __launch_bounds__(256)
-hplane_copy_kernel(ColArrays io, int ops1, int64_t Hx, int64_t Hy, int64_t x0, int64_t y0,
-                   int64_t Sx, int64_t Sy, int64_t words)
-{
-  const ColBlock bk=col_block(io);
-  const cplx<T> *in=(const cplx<T> *) bk.in;
-  cplx<T> *out=(cplx<T> *) bk.out;
-  const bool add=(ops1 >> blockIdx.z) & 1;
-  for(int64_t e=(int64_t) blockIdx.x*256+threadIdx.x; e < words; e += (int64_t) gridDim.x*256) {
-    cplx<T> v=in[e];
-    if(e % Sy == 0) {
-      const int64_t x=e/Sx, i=x-x0, j=(e-x*Sx)/Sy-y0;
-      if(i > -Hx && i < Hx && j > -Hy && j < Hy) {
-        const bool upper=j > 0 || (j == 0 && i > 0);
-        if(add || !upper) {
-          const cplx<T> m=conjg(in[(x0-i)*Sx+(y0-j)*Sy]);
-          if(add) v=v+m;
-          else v=i == 0 && j == 0 ? mk(v.x,(T) 0) : m;
-        }
-      }
-    }
-    out[e]=v;
-  }
 }
 
 // Reference-layout residue blocks (fftBase::forward/backward of the C++
@@ -880,40 +849,16 @@ static bool cols_reg(const fftwpp_amd_dim *d)
   return d->L <= 2*m && m*d->q < ((size_t) 1 << 30);
 }
 
-// One array; `in` and `out` of array a of a set.
-static ColArrays col_arrays(const void *in, void *out)
-{
-  ColArrays io={};
-  io.n=1;
-  io.in[0]=in;
-  io.out[0]=out;
-  return io;
-}
-
-// Grid depth of a forward column launch of `blocks` blocks per array over nr
-// residues: one per array, times the parts the residues are dealt to when the
-// arrays' blocks leave compute units idle (256 CUs, two blocks of 512 threads
-// each).  A part reads its columns again, from the caches at these sizes.
-// 1023 x 512 modes, FP32 (64 blocks per array, 3 residues): two arrays in 128
-// blocks of three residues each took as long as one array alone.
-static unsigned col_depth(const ColArrays &io, size_t blocks, size_t nr)
-{
-  size_t parts=512/std::max<size_t>(1,blocks*(size_t) io.n);
-  parts=std::max<size_t>(1,std::min(parts,nr));
-  return (unsigned) (parts*(size_t) io.n);
-}
-
 template<typename T, int M>
-static int colreg_launch(const DimArgs &a, bool fwd, const ColArrays &io,
-                         size_t s_in, size_t bsi, size_t s_out,
+static int colreg_launch(const DimArgs &a, bool fwd, const void *in,
+                         size_t s_in, size_t bsi, void *out, size_t s_out,
                          size_t bso, size_t C, size_t nbatch, size_t r0,
                          size_t nres, int accumulate, double scale,
                          size_t ics, size_t ocs, hipStream_t st)
 {
   typedef ColReg<T,M> CR;
   size_t lds=M*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
-  dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
-  grid.z=fwd ? col_depth(io,(size_t) grid.x*nbatch,nres) : (unsigned) io.n;
+  const dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
   const bool p2=a.L > M;
   // the N residue twiddles in LDS when they fit without lowering occupancy
   auto zfit=[&](auto kernel) {
@@ -925,14 +870,16 @@ static int colreg_launch(const DimArgs &a, bool fwd, const ColArrays &io,
     if(p2) {
       if((rc=allow_lds(colfwd_reg_kernel<T,M,2>,lds_max()))) return rc;
       if((zl=zfit(colfwd_reg_kernel<T,M,2>))) lds += (size_t) a.N*sizeof(cplx<T>);
-      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,io,
-                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
+                         (const cplx<T> *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
+                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                          (int64_t) ics,(int64_t) ocs,zl);
     } else {
       if((rc=allow_lds(colfwd_reg_kernel<T,M,1>,lds_max()))) return rc;
       if((zl=zfit(colfwd_reg_kernel<T,M,1>))) lds += (size_t) a.N*sizeof(cplx<T>);
-      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,io,
-                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
+                         (const cplx<T> *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
+                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                          (int64_t) ics,(int64_t) ocs,zl);
     }
     return launch_check("colfwd_reg_kernel");
@@ -940,26 +887,28 @@ static int colreg_launch(const DimArgs &a, bool fwd, const ColArrays &io,
   if(p2) {
     if((rc=allow_lds(colbwd_reg_kernel<T,M,2>,lds_max()))) return rc;
     if((zl=zfit(colbwd_reg_kernel<T,M,2>))) lds += (size_t) a.N*sizeof(cplx<T>);
-    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,io,
-                       (int64_t) s_in,(int64_t) bsi,(int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
+                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(cplx<T> *) out,
+                       (int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                        accumulate,(T) scale,(int64_t) ics,(int64_t) ocs,zl);
   } else {
     if((rc=allow_lds(colbwd_reg_kernel<T,M,1>,lds_max()))) return rc;
     if((zl=zfit(colbwd_reg_kernel<T,M,1>))) lds += (size_t) a.N*sizeof(cplx<T>);
-    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,io,
-                       (int64_t) s_in,(int64_t) bsi,(int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
+                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(cplx<T> *) out,
+                       (int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                        accumulate,(T) scale,(int64_t) ics,(int64_t) ocs,zl);
   }
   return launch_check("colbwd_reg_kernel");
 }
 
 template<typename T>
-static int colreg_t(const DimArgs &a, bool fwd, const ColArrays &io, size_t s_in,
-                    size_t bsi, size_t s_out, size_t bso, size_t C,
+static int colreg_t(const DimArgs &a, bool fwd, const void *in, size_t s_in,
+                    size_t bsi, void *out, size_t s_out, size_t bso, size_t C,
                     size_t nbatch, size_t r0, size_t nres, int accumulate,
                     double scale, size_t ics, size_t ocs, hipStream_t st)
 {
-#define FFTWPP_AMD_COLREG(MM) case MM: return colreg_launch<T,MM>(a,fwd,io,s_in,bsi,s_out,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
+#define FFTWPP_AMD_COLREG(MM) case MM: return colreg_launch<T,MM>(a,fwd,in,s_in,bsi,out,s_out,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
   switch(a.m) {
   FFTWPP_AMD_COLREG(16) FFTWPP_AMD_COLREG(32) FFTWPP_AMD_COLREG(64)
   FFTWPP_AMD_COLREG(128) FFTWPP_AMD_COLREG(256) FFTWPP_AMD_COLREG(512)
@@ -980,29 +929,28 @@ static bool cols_real(const fftwpp_amd_dim *d)
 }
 
 template<typename T, int M>
-static int colreal_launch(const DimArgs &a, bool fwd, const ColArrays &io,
-                          size_t s_in, size_t bsi, size_t s_out,
+static int colreal_launch(const DimArgs &a, bool fwd, const void *in,
+                          size_t s_in, size_t bsi, void *out, size_t s_out,
                           size_t bso, size_t C, size_t nbatch, double scale,
                           size_t ics, size_t ocs, hipStream_t st)
 {
   typedef ColReg<T,M> CR;
   const size_t lds=M*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
-  dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
-  if(fwd) grid.z=col_depth(io,(size_t) grid.x*nbatch,(size_t) RealKept::residues(a.q));
+  const dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
   const bool p2=a.L > M;
   int rc;
   if(fwd) {
     if(p2) {
       if((rc=allow_lds(colfwd_real_kernel<T,M,2>,lds))) return rc;
-      hipLaunchKernelGGL((colfwd_real_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,io,
-                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,
-                         (int64_t) s_out,(int64_t) bso,(int64_t) ics,
+      hipLaunchKernelGGL((colfwd_real_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
+                         (const T *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
+                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) ics,
                          (int64_t) ocs);
     } else {
       if((rc=allow_lds(colfwd_real_kernel<T,M,1>,lds))) return rc;
-      hipLaunchKernelGGL((colfwd_real_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,io,
-                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,
-                         (int64_t) s_out,(int64_t) bso,(int64_t) ics,
+      hipLaunchKernelGGL((colfwd_real_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
+                         (const T *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
+                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) ics,
                          (int64_t) ocs);
     }
     return launch_check("colfwd_real_kernel");
@@ -1010,13 +958,13 @@ static int colreal_launch(const DimArgs &a, bool fwd, const ColArrays &io,
   if(p2) {
     if((rc=allow_lds(colbwd_real_kernel<T,M,2>,lds))) return rc;
     hipLaunchKernelGGL((colbwd_real_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
-                       (const cplx<T> *) io.in[0],(int64_t) s_in,(int64_t) bsi,(T *) io.out[0],
+                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(T *) out,
                        (int64_t) s_out,(int64_t) C,(int64_t) bso,(T) scale,(int64_t) ics,
                        (int64_t) ocs);
   } else {
     if((rc=allow_lds(colbwd_real_kernel<T,M,1>,lds))) return rc;
     hipLaunchKernelGGL((colbwd_real_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
-                       (const cplx<T> *) io.in[0],(int64_t) s_in,(int64_t) bsi,(T *) io.out[0],
+                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(T *) out,
                        (int64_t) s_out,(int64_t) C,(int64_t) bso,(T) scale,(int64_t) ics,
                        (int64_t) ocs);
   }
@@ -1026,8 +974,8 @@ static int colreal_launch(const DimArgs &a, bool fwd, const ColArrays &io,
 // Single columns of many batch entries become the columns of one launch, as
 // in fwd_many_t.
 template<typename T>
-static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const ColArrays &io, size_t s_in,
-                     size_t bsi, size_t s_out, size_t bso, size_t C,
+static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const void *in, size_t s_in,
+                     size_t bsi, void *out, size_t s_out, size_t bso, size_t C,
                      size_t nbatch, double scale, hipStream_t st)
 {
   const DimArgs &a=sizeof(T) == 8 ? d->a64 : d->a32;
@@ -1036,7 +984,7 @@ static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const ColArrays &io, siz
     C=nbatch; ics=bsi; ocs=bso;
     nbatch=1; bsi=bso=0;
   }
-#define FFTWPP_AMD_COLREAL(MM) case MM: return colreal_launch<T,MM>(a,fwd,io,s_in,bsi,s_out,bso,C,nbatch,scale,ics,ocs,st);
+#define FFTWPP_AMD_COLREAL(MM) case MM: return colreal_launch<T,MM>(a,fwd,in,s_in,bsi,out,s_out,bso,C,nbatch,scale,ics,ocs,st);
   switch(a.m) {
   FFTWPP_AMD_COLREAL(16) FFTWPP_AMD_COLREAL(32) FFTWPP_AMD_COLREAL(64)
   FFTWPP_AMD_COLREAL(128) FFTWPP_AMD_COLREAL(256) FFTWPP_AMD_COLREAL(512)
@@ -1047,8 +995,8 @@ static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const ColArrays &io, siz
 }
 
 template<typename T>
-static int fwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t S,
-                      size_t C, size_t nbatch, size_t bsi,
+static int fwd_many_t(const fftwpp_amd_dim *d, const void *f, size_t S,
+                      size_t C, size_t nbatch, size_t bsi, void *F,
                       size_t SF, size_t bso, size_t r0, size_t nres,
                       hipStream_t st)
 {
@@ -1065,20 +1013,19 @@ static int fwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t S,
   if(ics == 1 && ocs == 1 && C >= (size_t) Col256<T>::TC && fast256(d,S,SF)) {
     constexpr int TC=Col256<T>::TC;
     dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
-    grid.z=col_depth(io,(size_t) grid.x*nbatch,nres);
     size_t lds=col256_lds<T>(nres);
     int rc=allow_lds(colfwd256_kernel<T>,lds);
     if(rc) return rc;
     hipLaunchKernelGGL((colfwd256_kernel<T>),grid,dim3(16*TC),lds,st,
-                       io,(int64_t) S,(int64_t) C,(int64_t) bsi,
-                       (int64_t) SF,(int64_t) bso,(int) d->L,
+                       (const cplx<T> *) f,(int64_t) S,(int64_t) C,(int64_t) bsi,
+                       (cplx<T> *) F,(int64_t) SF,(int64_t) bso,(int) d->L,
                        (int64_t) r0,(int64_t) nres,(const cplx<T> *) a.zN,(int64_t) d->q);
     return launch_check("colfwd256_kernel");
   }
   // register columns: tiles of several columns below m = 2048, so a single
   // short column goes to the LDS path
   if(cols_reg(d) && (C >= 8 || d->m >= 2048))
-    return colreg_t<T>(a,true,io,S,bsi,SF,bso,C,nbatch,r0,nres,0,1.0,ics,ocs,st);
+    return colreg_t<T>(a,true,f,S,bsi,F,SF,bso,C,nbatch,r0,nres,0,1.0,ics,ocs,st);
   size_t elt=sizeof(cplx<T>);
   size_t per=2*(d->m+1)*elt;
   if(per > lds_max()) return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"m too large for the LDS transform");
@@ -1088,19 +1035,16 @@ static int fwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t S,
   dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
   int rc=allow_lds(fwd_many_kernel<T>,lds);
   if(rc) return rc;
-  for(int x=0; x < io.n; ++x) {
-    hipLaunchKernelGGL(fwd_many_kernel<T>,grid,dim3(256),lds,st,a,
-                       (const cplx<T> *) io.in[x],(int64_t) S,(int64_t) C,
-                       (int64_t) bsi,(cplx<T> *) io.out[x],(int64_t) SF,(int64_t) bso,
-                       (int64_t) r0,(int64_t) nres,(int) TC,(int64_t) ics,(int64_t) ocs);
-    if((rc=launch_check("fwd_many_kernel"))) return rc;
-  }
-  return FFTWPP_AMD_OK;
+  hipLaunchKernelGGL(fwd_many_kernel<T>,grid,dim3(256),lds,st,a,
+                     (const cplx<T> *) f,(int64_t) S,(int64_t) C,
+                     (int64_t) bsi,(cplx<T> *) F,(int64_t) SF,(int64_t) bso,
+                     (int64_t) r0,(int64_t) nres,(int) TC,(int64_t) ics,(int64_t) ocs);
+  return launch_check("fwd_many_kernel");
 }
 
 template<typename T>
-static int bwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t SF,
-                      size_t bsi, size_t S, size_t C,
+static int bwd_many_t(const fftwpp_amd_dim *d, const void *F, size_t SF,
+                      size_t bsi, void *f, size_t S, size_t C,
                       size_t nbatch, size_t bso, size_t r0, size_t nres,
                       int accumulate, double scale, hipStream_t st)
 {
@@ -1113,19 +1057,19 @@ static int bwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t SF,
   }
   if(ics == 1 && ocs == 1 && C >= (size_t) Col256<T>::TC && fast256(d,S,SF)) {
     constexpr int TC=Col256<T>::TC;
-    dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch,(unsigned) io.n);
+    dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
     size_t lds=col256_lds<T>(nres);
     int rc=allow_lds(colbwd256_kernel<T>,lds);
     if(rc) return rc;
     hipLaunchKernelGGL((colbwd256_kernel<T>),grid,dim3(16*TC),lds,st,
-                       io,(int64_t) SF,(int64_t) bsi,
+                       (const cplx<T> *) F,(int64_t) SF,(int64_t) bsi,(cplx<T> *) f,
                        (int64_t) S,(int64_t) C,(int64_t) bso,(int) d->L,(int64_t) r0,
                        (int64_t) nres,accumulate,(T) scale,(const cplx<T> *) a.zN,
                        (int64_t) d->q);
     return launch_check("colbwd256_kernel");
   }
   if(cols_reg(d) && (C >= 8 || d->m >= 2048))
-    return colreg_t<T>(a,false,io,SF,bsi,S,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
+    return colreg_t<T>(a,false,F,SF,bsi,f,S,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
   size_t elt=sizeof(cplx<T>);
   size_t per=2*(d->m+1)*elt;
   if(per > lds_max()) return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"m too large for the LDS transform");
@@ -1135,15 +1079,12 @@ static int bwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t SF,
   dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
   int rc=allow_lds(bwd_many_kernel<T>,lds);
   if(rc) return rc;
-  for(int x=0; x < io.n; ++x) {
-    hipLaunchKernelGGL(bwd_many_kernel<T>,grid,dim3(256),lds,st,a,
-                       (const cplx<T> *) io.in[x],(int64_t) SF,(int64_t) bsi,
-                       (cplx<T> *) io.out[x],(int64_t) S,(int64_t) C,(int64_t) bso,
-                       (int64_t) r0,(int64_t) nres,accumulate,(T) scale,(int) TC,
-                       (int64_t) ics,(int64_t) ocs);
-    if((rc=launch_check("bwd_many_kernel"))) return rc;
-  }
-  return FFTWPP_AMD_OK;
+  hipLaunchKernelGGL(bwd_many_kernel<T>,grid,dim3(256),lds,st,a,
+                     (const cplx<T> *) F,(int64_t) SF,(int64_t) bsi,
+                     (cplx<T> *) f,(int64_t) S,(int64_t) C,(int64_t) bso,
+                     (int64_t) r0,(int64_t) nres,accumulate,(T) scale,(int) TC,
+                     (int64_t) ics,(int64_t) ocs);
+  return launch_check("bwd_many_kernel");
 }
 
 // LDS bytes of batch_conv_kernel for sub-FFT size m, TR items and (with
@@ -1167,17 +1108,6 @@ struct BatchLaunch {
   size_t TR, threads, nblocks, lacc, D, ptotal, ld, lds;
   double scale;
 };
-
-// Grid of a pass over `count` items of up to `words` words each by blocks of
-// 256 threads: one block per item, and when the items are too few to occupy
-// the chip (2048 resident blocks of 256) slices of 256 or more words of each.
-// (One block summed the whole of a 10000-point row: 54 us of its 78.)
-static dim3 item_grid(size_t count, size_t words)
-{
-  const size_t nb=std::min<size_t>(count,4096);
-  const size_t slices=std::min<size_t>((words+255)/256,std::max<size_t>(1,2048/nb));
-  return dim3((unsigned) nb,(unsigned) std::max<size_t>(1,slices));
-}
 
 template<typename T, int MULT>
 static int batch_rows_launch(const DimArgs &a, const BatchLaunch &b,
@@ -1203,7 +1133,8 @@ static int batch_rows_launch(const DimArgs &a, const BatchLaunch &b,
   if(rc) return rc;
   const size_t G=(a.q+b.D-1)/b.D;
   if(G > 1) {
-    hipLaunchKernelGGL(batch_reduce_kernel<T>,item_grid(b.count,(size_t) a.L),dim3(256),0,st,
+    const size_t nb=b.count < 4096 ? b.count : 4096;
+    hipLaunchKernelGGL(batch_reduce_kernel<T>,dim3((unsigned) nb),dim3(256),0,st,
                        b.items,(int64_t) b.count,(const cplx<T> *) b.part,
                        (int64_t) b.ptotal,(int) G,(cplx<T> *) b.out,(T) b.scale);
     rc=launch_check("batch_reduce_kernel");
@@ -1227,7 +1158,7 @@ static void batch_reg_shape(size_t m, size_t q, size_t elt, size_t threads,
   const size_t tps=batch_tps(m,elt);
   size_t n=tps > 64 ? tps : std::max(threads,tps)/tps*tps;
   if(n > 512) n=512/tps*tps;
-  const size_t pad=m >= 512 ? m : m+m/16;      // RPlan::PAD
+  const size_t pad=m+m/16;
   *nt=n;
   *lds=m*elt+(n/tps)*2*pad*(elt/2)+q*(m/tps)*elt;
 }
@@ -1275,7 +1206,8 @@ static int batch_reg_t(const DimArgs &a, const BatchLaunch &b, int mult,
   }
   if(rc) return rc;
   if(b.D == 0) {
-    const dim3 grid=item_grid(b.count,(size_t) a.m), blk(256);
+    const size_t nb=b.count < 4096 ? b.count : 4096;
+    const dim3 grid((unsigned) nb), blk(256);
     const BatchItem *it=b.items;
     const int64_t n=(int64_t) b.count;
     const cplx<T> *Z=(const cplx<T> *) b.part, *zN=(const cplx<T> *) a.zN;
@@ -1293,7 +1225,8 @@ static int batch_reg_t(const DimArgs &a, const BatchLaunch &b, int mult,
   }
   const size_t G=(a.q+b.D-1)/b.D;
   if(G > 1) {
-    hipLaunchKernelGGL(batch_reduce_kernel<T>,item_grid(b.count,(size_t) a.L),dim3(256),0,st,
+    const size_t nb=b.count < 4096 ? b.count : 4096;
+    hipLaunchKernelGGL(batch_reduce_kernel<T>,dim3((unsigned) nb),dim3(256),0,st,
                        b.items,(int64_t) b.count,(const cplx<T> *) b.part,
                        (int64_t) b.ptotal,(int) G,(cplx<T> *) b.out,(T) b.scale);
     rc=launch_check("batch_reduce_kernel");
@@ -1709,40 +1642,6 @@ size_t fftwpp_amd_max_m(int dtype)
 }
 
 
-// fftwpp_amd_forward_many (real = 0) or fftwpp_amd_forward_real_many (real =
-// 1: every kept plane, r0 and nres unused) of n <= 3 arrays of the same
-// layout in one launch; the inputs may be the same array, the outputs not.
-int fftwpp_amd_internal_forward_arrays(const fftwpp_amd_dim *d, int dtype, int real, int n,
-                                       const void *const *f, size_t S, size_t C,
-                                       size_t nbatch, size_t bstride_in, void *const *F,
-                                       size_t SF, size_t bstride_out, size_t r0, size_t nres,
-                                       void *stream)
-{
-  if(!d || !f || !F || n < 1 || n > MAXARRAYS) return fail(FFTWPP_AMD_ERR_ARG,"bad array set");
-  ColArrays io={};
-  io.n=n;
-  for(int a=0; a < n; ++a) {
-    if(!f[a] || !F[a]) return fail(FFTWPP_AMD_ERR_ARG,"null argument");
-    io.in[a]=f[a];
-    io.out[a]=F[a];
-  }
-  if(d->kind == FFTWPP_AMD_KIND_HERMITIAN)
-    return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"Hermitian dimensions are innermost only");
-  if(real && !cols_real(d))
-    return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"real residue transforms take power-of-two m in [16, 4096] and L <= 2m");
-  if((!real && r0+nres > d->q) || C == 0 || nbatch == 0)
-    return fail(FFTWPP_AMD_ERR_ARG,"bad residue range or shape");
-  if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
-  hipStream_t st=(hipStream_t) stream;
-  if(real)
-    return dtype == FFTWPP_AMD_F32 ?
-      colreal_t<float>(d,true,io,S,bstride_in,SF,bstride_out,C,nbatch,1.0,st) :
-      colreal_t<double>(d,true,io,S,bstride_in,SF,bstride_out,C,nbatch,1.0,st);
-  return dtype == FFTWPP_AMD_F32 ?
-    fwd_many_t<float>(d,io,S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st) :
-    fwd_many_t<double>(d,io,S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st);
-}
-
 int fftwpp_amd_forward_many(const fftwpp_amd_dim *d, int dtype,
                             const void *f, size_t S, size_t C,
                             size_t nbatch, size_t bstride_in, void *F,
@@ -1756,35 +1655,10 @@ int fftwpp_amd_forward_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    fwd_many_t<float>(d,col_arrays(f,F),S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st) :
-    fwd_many_t<double>(d,col_arrays(f,F),S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st);
+    fwd_many_t<float>(d,f,S,C,nbatch,bstride_in,F,SF,bstride_out,r0,nres,st) :
+    fwd_many_t<double>(d,f,S,C,nbatch,bstride_in,F,SF,bstride_out,r0,nres,st);
 }
 
-
-// fftwpp_amd_backward_many of n <= 3 arrays of the same layout in one launch.
-int fftwpp_amd_internal_backward_arrays(const fftwpp_amd_dim *d, int dtype, int n,
-                                        const void *const *F, size_t SF, size_t bstride_in,
-                                        void *const *f, size_t S, size_t C, size_t nbatch,
-                                        size_t bstride_out, size_t r0, size_t nres,
-                                        int accumulate, double scale, void *stream)
-{
-  if(!d || !f || !F || n < 1 || n > MAXARRAYS) return fail(FFTWPP_AMD_ERR_ARG,"bad array set");
-  ColArrays io={};
-  io.n=n;
-  for(int a=0; a < n; ++a) {
-    if(!f[a] || !F[a]) return fail(FFTWPP_AMD_ERR_ARG,"null argument");
-    io.in[a]=F[a];
-    io.out[a]=f[a];
-  }
-  if(d->kind == FFTWPP_AMD_KIND_HERMITIAN)
-    return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"Hermitian dimensions are innermost only");
-  if(r0+nres > d->q || nres == 0 || C == 0 || nbatch == 0) return fail(FFTWPP_AMD_ERR_ARG,"bad residue range or shape");
-  if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
-  hipStream_t st=(hipStream_t) stream;
-  return dtype == FFTWPP_AMD_F32 ?
-    bwd_many_t<float>(d,io,SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st) :
-    bwd_many_t<double>(d,io,SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st);
-}
 
 int fftwpp_amd_backward_many(const fftwpp_amd_dim *d, int dtype,
                              const void *F, size_t SF, size_t bstride_in,
@@ -1799,8 +1673,8 @@ int fftwpp_amd_backward_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    bwd_many_t<float>(d,col_arrays(F,f),SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st) :
-    bwd_many_t<double>(d,col_arrays(F,f),SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st);
+    bwd_many_t<float>(d,F,SF,bstride_in,f,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st) :
+    bwd_many_t<double>(d,F,SF,bstride_in,f,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st);
 }
 
 
@@ -1828,8 +1702,8 @@ int fftwpp_amd_forward_real_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    colreal_t<float>(d,true,col_arrays(f,F),S,bstride_in,SF,bstride_out,C,nbatch,1.0,st) :
-    colreal_t<double>(d,true,col_arrays(f,F),S,bstride_in,SF,bstride_out,C,nbatch,1.0,st);
+    colreal_t<float>(d,true,f,S,bstride_in,F,SF,bstride_out,C,nbatch,1.0,st) :
+    colreal_t<double>(d,true,f,S,bstride_in,F,SF,bstride_out,C,nbatch,1.0,st);
 }
 
 int fftwpp_amd_backward_real_many(const fftwpp_amd_dim *d, int dtype,
@@ -1844,8 +1718,8 @@ int fftwpp_amd_backward_real_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    colreal_t<float>(d,false,col_arrays(F,f),SF,bstride_in,S,bstride_out,C,nbatch,scale,st) :
-    colreal_t<double>(d,false,col_arrays(F,f),SF,bstride_in,S,bstride_out,C,nbatch,scale,st);
+    colreal_t<float>(d,false,F,SF,bstride_in,f,S,bstride_out,C,nbatch,scale,st) :
+    colreal_t<double>(d,false,F,SF,bstride_in,f,S,bstride_out,C,nbatch,scale,st);
 }
 
 int fftwpp_amd_conv_rows(const fftwpp_amd_dim *d, int dtype, int mult,
@@ -2228,67 +2102,25 @@ int fftwpp_amd_symmetrize_xy(size_t Hx, size_t Hy, size_t Hz, size_t x0,
   return rc;
 }
 
-// fftwpp_amd_hermitian_plane on n <= 3 arrays of one layout in one launch.
-int fftwpp_amd_internal_hplanes(int dtype, int op, int n, size_t Hx, size_t Hy, size_t x0,
-                                size_t y0, void *const *f, size_t Sx, size_t Sy, void *stream)
-{
-  if(!f || n < 1 || n > MAXARRAYS || Hx == 0 || Hy == 0) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
-  if(op < 0 || op > 2) return fail(FFTWPP_AMD_ERR_ARG,"unknown plane operation");
-  if(x0+1 < Hx || y0+1 < Hy) return fail(FFTWPP_AMD_ERR_ARG,"origin too small");
-  ColArrays io={};
-  io.n=n;
-  for(int a=0; a < n; ++a) {
-    if(!f[a]) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
-    io.out[a]=f[a];
-  }
-  hipStream_t st=(hipStream_t) stream;
-  const dim3 grid((unsigned) (((2*Hx-1)*Hy+255)/256),(unsigned) n);
-  if(dtype == FFTWPP_AMD_F32)
-    hipLaunchKernelGGL(hplane_kernel<float>,grid,dim3(256),0,st,op,(int64_t) Hx,
-                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,io,(int64_t) Sx,(int64_t) Sy);
-  else
-    hipLaunchKernelGGL(hplane_kernel<double>,grid,dim3(256),0,st,op,(int64_t) Hx,
-                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,io,(int64_t) Sx,(int64_t) Sy);
-  return launch_check("hplane_kernel");
-}
-
 int fftwpp_amd_hermitian_plane(int dtype, int op, size_t Hx, size_t Hy,
                                size_t x0, size_t y0, void *f, size_t Sx,
                                size_t Sy, void *stream)
 {
-  return fftwpp_amd_internal_hplanes(dtype,op,1,Hx,Hy,x0,y0,&f,Sx,Sy,stream);
-}
-
-// out[a] = in[a] (arrays of `words` words, none of them the same) with plane
-// operation 0 applied, or operation 1 where bit a of ops1 is set, for n <= 3
-// arrays in one launch.
-int fftwpp_amd_internal_hplane_copies(int dtype, int n, int ops1, size_t Hx, size_t Hy,
-                                      size_t x0, size_t y0, const void *const *in,
-                                      void *const *out, size_t Sx, size_t Sy, size_t words,
-                                      void *stream)
-{
-  if(!in || !out || n < 1 || n > MAXARRAYS || Hx == 0 || Hy == 0 || Sx == 0 || Sy == 0 || words == 0)
-    return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
+  if(!f || Hx == 0 || Hy == 0) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
+  if(op < 0 || op > 2) return fail(FFTWPP_AMD_ERR_ARG,"unknown plane operation");
   if(x0+1 < Hx || y0+1 < Hy) return fail(FFTWPP_AMD_ERR_ARG,"origin too small");
-  if(Sx % Sy || (x0+Hx-1)*Sx+(y0+Hy-1)*Sy >= words) return fail(FFTWPP_AMD_ERR_ARG,"bad plane strides");
-  ColArrays io={};
-  io.n=n;
-  for(int a=0; a < n; ++a) {
-    if(!in[a] || !out[a] || in[a] == out[a]) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
-    io.in[a]=in[a];
-    io.out[a]=out[a];
-  }
   hipStream_t st=(hipStream_t) stream;
-  const dim3 grid((unsigned) std::min<size_t>((words+255)/256,8192),1,(unsigned) n);
+  const size_t n=(2*Hx-1)*Hy;
+  const dim3 grid((unsigned) ((n+255)/256));
   if(dtype == FFTWPP_AMD_F32)
-    hipLaunchKernelGGL(hplane_copy_kernel<float>,grid,dim3(256),0,st,io,ops1,(int64_t) Hx,
-                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,(int64_t) Sx,(int64_t) Sy,
-                       (int64_t) words);
+    hipLaunchKernelGGL(hplane_kernel<float>,grid,dim3(256),0,st,op,(int64_t) Hx,
+                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,(cplx<float> *) f,
+                       (int64_t) Sx,(int64_t) Sy);
   else
-    hipLaunchKernelGGL(hplane_copy_kernel<double>,grid,dim3(256),0,st,io,ops1,(int64_t) Hx,
-                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,(int64_t) Sx,(int64_t) Sy,
-                       (int64_t) words);
-  return launch_check("hplane_copy_kernel");
+    hipLaunchKernelGGL(hplane_kernel<double>,grid,dim3(256),0,st,op,(int64_t) Hx,
+                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,(cplx<double> *) f,
+                       (int64_t) Sx,(int64_t) Sy);
+  return launch_check("hplane_kernel");
 }
 
 // ---- memory and stream plumbing for host code that includes no HIP header

@@ -33,11 +33,6 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-def _tracked(t):
-    """Whether operations on t are recorded for autograd."""
-    return t.requires_grad and torch.is_grad_enabled()
-
-
 class DeviceConvolution:
     """Plan of a dealiased convolution of device tensors.
 
@@ -126,8 +121,6 @@ class DeviceConvolution:
         return out
 
     def __call__(self, a, b):
-        if a.is_contiguous() and not _tracked(a):
-            return self.convolve_out(torch.empty_like(a), a, b)
         out = a.clone()
         return self.convolve_(out, b)
 
@@ -163,25 +156,11 @@ class DeviceConvolution:
         """Copy of t with the self-conjugate plane made Hermitian
         (HermitianSymmetrize{,X,XY}, convolve.h:1168-1256)."""
         self._check(t)
-        if not _tracked(t):
-            return self._symmetrized_copies(t)[0]
         out = t.clone()
         Hx, Hy, x0, y0, Sx, Sy = self._plane()
         check(lib().fftwpp_amd_hermitian_plane(_dtype_code(self.dtype), 0, Hx, Hy, x0, y0,
                                                out.data_ptr(), Sx, Sy, _stream()))
         return out
-
-    def _symmetrized_copies(self, *ts):
-        """symmetrized() of up to three tensors in one launch."""
-        plane = self._plane()
-        outs = [torch.empty_like(t) for t in ts]
-        n = len(ts)
-        check(lib().fftwpp_amd_internal_hplane_copies(
-            _dtype_code(self.dtype), n, 0, *plane[:4],
-            (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts]),
-            (ctypes.c_void_p * n)(*[t.data_ptr() for t in outs]), *plane[4:], ts[0].numel(),
-            _stream()))
-        return outs
 
     def adjoint(self, w, a, b, need_a=True, need_b=True):
         """Cotangents of (a, b) for output cotangent w (PyTorch convention
@@ -208,10 +187,7 @@ class _ConvolveFn(torch.autograd.Function):
         ctx.plan = plan
         ctx.save_for_backward(a, b)
         if plan.kind == "hermitian":
-            plan._check(a)
-            plan._check(b)
-            sa, sb = plan._symmetrized_copies(a, b)
-            return plan.convolve_(sa, sb)
+            return plan(plan.symmetrized(a), plan.symmetrized(b))
         return plan(a, b)
 
     @staticmethod
