@@ -414,8 +414,8 @@ batch_reg_kernel(DimArgs d, const BatchItem *items, int64_t count,
 }
 
 // out[off + sigma + M b] = scale * sum_{r < q} w_q^{-b r} Z[i q M + r M + sigma]
-// for the blocks b of each item (sequence mode of batch_reg_kernel); one
-// block per item (grid-stride), threads over sigma.  With QMAX > 0 (q <= QMAX)
+// for the blocks b of each item (sequence mode of batch_reg_kernel); blocks
+// over items (grid-stride in x) and over slices of sigma (y).  With QMAX > 0 (q <= QMAX)
 // a thread loads its q values Z_r(sigma) once, before the sums over the
 // blocks (indices clamped to r < q, the extra terms given a zero factor);
 // QMAX = 0 takes any q and re-reads them per block.
@@ -428,7 +428,7 @@ batch_unfold_kernel(const BatchItem *items, int64_t count, const cplx<T> *Z,
     const BatchItem it=items[i];
     const cplx<T> *zi=Z+i*(int64_t) q*M;
     const int L=(int) it.L;
-    for(int sg=threadIdx.x; sg < M; sg += blockDim.x) {
+    for(int sg=blockIdx.y*blockDim.x+threadIdx.x; sg < M; sg += gridDim.y*blockDim.x) {
       if constexpr(QMAX > 0) {
         cplx<T> z[QMAX];
 #pragma unroll
@@ -460,8 +460,8 @@ batch_unfold_kernel(const BatchItem *items, int64_t count, const cplx<T> *Z,
   }
 }
 
-// out[off + j] = scale * sum_{g < G} part[g ptotal + poff + j], one block
-// per item (grid-stride), groups added in order.
+// out[off + j] = scale * sum_{g < G} part[g ptotal + poff + j], blocks over
+// items (grid-stride in x) and slices of an item (y), groups added in order.
 template<typename T>
 __global__ void __launch_bounds__(256)
 batch_reduce_kernel(const BatchItem *items, int64_t count,
@@ -470,7 +470,7 @@ batch_reduce_kernel(const BatchItem *items, int64_t count,
 {
   for(int64_t i=blockIdx.x; i < count; i += gridDim.x) {
     const BatchItem it=items[i];
-    for(int64_t j=threadIdx.x; j < it.L; j += blockDim.x) {
+    for(int64_t j=(int64_t) blockIdx.y*blockDim.x+threadIdx.x; j < it.L; j += (int64_t) gridDim.y*blockDim.x) {
       cplx<T> sum=part[it.poff+j];
       for(int g=1; g < G; ++g) sum=sum+part[g*ptotal+it.poff+j];
       out[it.off+j]=scale*sum;

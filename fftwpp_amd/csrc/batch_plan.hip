@@ -239,16 +239,42 @@ bool tile_fits(const fftwpp_amd_batch &h, const Cls &c, size_t TR)
   return fftwpp_amd_batch_rows_lds(c.dim,h.dtype,TR,0) != 0;
 }
 
-// Without tuning: small tiles of short items, and enough residue groups
-// for about two work units per compute unit.
+// Sub-FFT size without tuning.  One residue (m = 2^ceil(log2 M)) needs no
+// second launch and folds nothing, up to the size where the transform's
+// exchange area and twiddles leave too few blocks on a CU: 4096 in FP32, 1024
+// in FP64; longer items take two or more residues of m = 1024 (M <= 2048) or
+// 2048 (FP64, L <= 8192), else of 4096.  4096 sequences of 64 ... 16384 words
+// in FP64, with the units of default_tile:
+// 1065 us with m = 2^ceil(log2 L) and two units per CU, 830 us so.
+size_t default_m(size_t L, size_t M, int dtype)
+{
+  const size_t e=std::max<size_t>(16,ceilpow2(M));
+  if(dtype == FFTWPP_AMD_F32) return std::min<size_t>(e,BATCH_MAXM);
+  if(e <= 1024) return e;
+  if(e <= 2048) return 1024;
+  return L <= 8192 ? 2048 : BATCH_MAXM;
+}
+
+// Without tuning.  Register kernel: items of several residues run in the
+// sequence mode (D = 0: every residue a unit, the outputs folded by a second
+// launch), except q = 2 with m = 2048 in FP64, whose unit does both residues;
+// when several units share an item the grid is the blocks that stay resident
+// (two waves per SIMD, LDS permitting), so an item's units run close together
+// and find its words in L2.  LDS kernel: small tiles of short items, and
+// enough residue groups for about two work units per compute unit.
 Tile default_tile(const fftwpp_amd_batch &h, const Cls &c)
 {
   if(size_t tps=fftwpp_amd_batch_rows_tps(c.dim,h.dtype)) {
-    size_t threads=std::max<size_t>(256,tps);
-    size_t slots=tps > 64 ? 1 : threads/tps;
-    size_t G=std::min<size_t>({8,c.q,std::max<size_t>(1,ceilquot(2*(size_t) h.cus*slots,
-                                                                  c.ids.size()))});
-    return make_tile(h,c,1,threads,ceilquot(c.q,G));
+    const size_t threads=std::max<size_t>(256,tps);
+    const size_t D=c.q == 1 ? 1 : c.q == 2 && c.m == 2048 && h.dtype == FFTWPP_AMD_F64 ? 2 : 0;
+    Tile t=make_tile(h,c,1,threads,D);
+    if(tps > 64 && groups(c,t) > 1) {
+      const size_t elt=h.dtype == FFTWPP_AMD_F32 ? 8 : 16;
+      const size_t lds=(2*c.m+c.m/16+c.q*(c.m/tps))*elt;     // twiddles, exchange area
+      const size_t per=std::max<size_t>(1,std::min<size_t>(160*1024/lds,512/tps));
+      t.nblocks=std::min(t.nblocks,per*(size_t) h.cus);
+    }
+    return t;
   }
   size_t TR=std::max<size_t>(1,std::min<size_t>(32,2048/c.m));
   while(TR > 1 && !tile_fits(h,c,TR)) TR /= 2;
@@ -867,7 +893,7 @@ int fftwpp_amd_batch_create(fftwpp_amd_batch **out, size_t n, const size_t *L,
   if(rc) { destroy(h); return rc; }
   const size_t maxm=BATCH_MAXM;
   h->mof.resize(n);
-  for(size_t i=0; i < n; ++i) h->mof[i]=std::min(ceilpow2(h->L[i]),maxm);
+  for(size_t i=0; i < n; ++i) h->mof[i]=default_m(h->L[i],h->M[i],dtype);
   const bool tuned=flags & FFTWPP_AMD_BATCH_TUNE;
   TuneArrays ta;
   bool timing=false;                      // ta holds the timing arrays
@@ -884,7 +910,7 @@ int fftwpp_amd_batch_create(fftwpp_amd_batch **out, size_t n, const size_t *L,
       else h->mof[i]=it->second;
     }
     if(!cached) {
-      for(size_t i=0; i < n; ++i) h->mof[i]=std::min(ceilpow2(h->L[i]),maxm);
+      for(size_t i=0; i < n; ++i) h->mof[i]=default_m(h->L[i],h->M[i],dtype);
       rc=ta.init(*h);
       timing=true;
       if(!rc) rc=tune_geometry(*h,ta);

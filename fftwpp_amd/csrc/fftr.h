@@ -36,7 +36,8 @@ template<int M, int V=16> struct RPlan {
   static constexpr int NV=LOG/LV;                       // radix-V stages
   static constexpr int LAST=1 << (LOG-LV*NV);           // remaining factor
   static constexpr int NST=NV+(LAST > 1 ? 1 : 0);
-  static constexpr int PAD=M+M/16;                      // exchange words
+  // exchange words (the swizzled sequences of 512 or more use M of them)
+  static constexpr int PAD=M >= 512 ? M : M+M/16;
   __host__ __device__ static constexpr int radix(int s) { return s < NV ? V : LAST; }
   // Stage s writes output u of butterfly j at dest<s>(j) + u ns(s); the bits
   // of j move without mixing, so dest(a + b) = dest(a) + dest(b) for a and b
@@ -74,7 +75,7 @@ __device__ __forceinline__ int padr(int e) { return e+(e >> 4); }
 // immediate offset of the access: it has conflicts, but needs 10 to 60 fewer
 // registers and no instructions (complex rows of M = 64 FP64 98 us against
 // 107 swizzled, M = 128 FP32 67 against 91; M = 128 FP64 133 against 126).
-// Indices stay below M + M/16.
+// Indices stay below RPlan::PAD.
 template<typename T, int M, int V>
 __host__ __device__ constexpr bool xswizzled()
 {

@@ -1039,13 +1039,13 @@ static void fusedRows(fftBase *fft, DeviceWork &work, size_t slot, int dtype,
   }
   if(tps) {
     // complex rows longer than one block of a power-of-two m: the batched
-    // register kernel with the rows as items (row i at i rs).  The residues
-    // always go to partial sums that its second launch adds into out (at
-    // least two groups when q > 1), since out may alias f or g and a unit
-    // that wrote its outputs would re-read them in its next residue's fold:
-    // one residue per unit when rows are few, two groups otherwise.
-    const size_t L=fft->L, q=fft->q;
-    const size_t D=rows >= 512 ? (q+1)/2 : 1;
+    // register kernel with the rows as items (row i at i rs) in the sequence
+    // mode: every residue of every row is a work unit that writes its m words
+    // to a buffer, and the second launch folds a row's q sequences into out.
+    // out may alias f or g: it is written after every unit has read its row.
+    // One row of 10000 in FP32: 78 us with partial sums of L words per group
+    // (one block added them up in 54 us), 21.5 us so.
+    const size_t L=fft->L, q=fft->q, m=fft->m;
     void *items=work.get(slot+1,rows*3*sizeof(int64_t));
     const std::vector<size_t> key={rows,rs,L};
     if(work.keys[slot+1] != key) {
@@ -1053,11 +1053,9 @@ static void fusedRows(fftBase *fft, DeviceWork &work, size_t slot, int dtype,
       check(fftwpp_amd_internal_row_items(items,rows,rs,L,stream),"item table");
       work.keys[slot+1]=key;
     }
-    const size_t G=(q+D-1)/D;
-    void *part=G > 1 ? work.get(slot,G*rows*L*(dtype == FFTWPP_AMD_F32 ? 8 : 16)) : NULL;
-    const size_t units=rows*G;
+    void *part=work.get(slot,rows*q*m*(dtype == FFTWPP_AMD_F32 ? 8 : 16));
     check(fftwpp_amd_batch_rows(fft->dev,dtype,code,items,rows,f,g,out,1,
-                                tps < 64 ? 64 : tps,std::min<size_t>(units,2048),0,D,
+                                tps < 64 ? 64 : tps,std::min<size_t>(rows*q,2048),0,0,
                                 part,rows*L,s,stream),what);
     return;
   }
