@@ -135,6 +135,42 @@ __device__ __forceinline__ int64_t xcd_tile(int64_t x, int64_t gx)
   return x < 8*per ? (x % 8)*per+x/8 : x;
 }
 
+// Up to three arrays transformed by one launch (the inputs of a convolution,
+// or the cotangent and both inputs of its adjoint).  Block z of the grid takes
+// array z mod n and every gridDim.z/n-th residue from z/n on.
+constexpr int MAXARRAYS=3;
+
+struct ColArrays {
+  int n;
+  const void *in[MAXARRAYS];
+  void *out[MAXARRAYS];
+};
+
+struct ColBlock {
+  const void *in;
+  void *out;
+  int part, parts;
+};
+
+__device__ __forceinline__ ColBlock col_block(const ColArrays &io)
+{
+  // in scalar registers (a division runs on the vector unit and would take
+  // the pointers with it)
+  const int z=blockIdx.z, n=io.n;
+  const int part=n == 1 ? z : __builtin_amdgcn_readfirstlane(z/n);
+  const int a=z-part*n;
+  ColBlock b;
+  // device memory: as pointers out of a struct they would be taken for
+  // generic ones (flat accesses, more registers)
+  b.in=(const void *) (const __attribute__((address_space(1))) void *)
+    (a == 0 ? io.in[0] : (a == 1 ? io.in[1] : io.in[2]));
+  b.out=(void *) (__attribute__((address_space(1))) void *)
+    (a == 0 ? io.out[0] : (a == 1 ? io.out[1] : io.out[2]));
+  b.part=part;
+  b.parts=n == 1 ? (int) gridDim.z : __builtin_amdgcn_readfirstlane((int) gridDim.z/n);
+  return b;
+}
+
 template<typename T>
 __device__ __forceinline__ cplx<T> ztab(const DimArgs &d, int64_t j)
 {
@@ -148,6 +184,28 @@ __device__ __forceinline__ cplx<T> zeta(const DimArgs &d, int64_t e)
   int64_t r=e % d.N;
   if(r < 0) r += d.N;
   return ztab<T>(d,r);
+}
+
+// t as a value that the compiler does not know to be the loop-invariant one:
+// without it the LDS addresses and twiddle positions of every stage, which
+// depend on t alone, are hoisted out of the caller's loop over rows and
+// residues and stay in registers through all of it (30 to 40 of them in a row
+// kernel); computed anew per transform they cost one instruction per access.
+__device__ __forceinline__ int fresh(int t)
+{
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// A complex word of a table in LDS whose words are aligned to their size: one
+// access with a 64 KB range of immediate offsets (two words of half the size
+// reach 2 KB, and the rest of a table costs an addition each).
+template<typename T>
+__device__ __forceinline__ cplx<T> table_word(const cplx<T> *p)
+{
+  typedef T pair __attribute__((ext_vector_type(2)));
+  const pair v=*reinterpret_cast<const pair *>(p);
+  return mk(v.x,v.y);
 }
 
 // Buffer access: a complex word at byte offset off (per lane) + soff

@@ -165,7 +165,7 @@ __device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const cplx<T> *tw,
       const cplx<T> *w=tw+OFF+kp;
 #pragma unroll
       for(int tp=1; tp < R; ++tp) {
-        const cplx<T> z=w[(tp-1)*Ns];
+        const cplx<T> z=table_word(w+(tp-1)*Ns);
         u[tp]=S > 0 ? u[tp]*z : mulc(u[tp],z);
       }
     }
@@ -245,7 +245,7 @@ __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
       const cplx<T> *w=tw+OFF+kp;
 #pragma unroll
       for(int tp=1; tp < R; ++tp) {
-        const cplx<T> z=w[(tp-1)*Ns];
+        const cplx<T> z=table_word(w+(tp-1)*Ns);
         u[tp]=S > 0 ? u[tp]*z : mulc(u[tp],z);
         v[tp]=S > 0 ? v[tp]*z : mulc(v[tp],z);
       }
@@ -290,7 +290,7 @@ template<typename T, int M, int V, int S>
 __device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const cplx<T> *tw,
                                           int t)
 {
-  fftr_pair_stage<T,M,V,S,0>(X,Y,xb,tw,t);
+  fftr_pair_stage<T,M,V,S,0>(X,Y,xb,tw,fresh(t));
 }
 
 // In-place transform of the sequence held by threads t < TPS (v[V] each)
@@ -300,7 +300,7 @@ __device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const c
 template<typename T, int M, int V, int S, bool CX=false>
 __device__ __forceinline__ void fftr(cplx<T> *v, T *xb, const cplx<T> *tw, int t)
 {
-  fftr_stage<T,M,V,S,0,false,CX>(v,xb,tw,t);
+  fftr_stage<T,M,V,S,0,false,CX>(v,xb,tw,fresh(t));
 }
 
 // The same transform when the threads of a sequence are not consecutive
@@ -309,15 +309,16 @@ template<typename T, int M, int V, int S, bool CX=false>
 __device__ __forceinline__ void fftr_blk(cplx<T> *v, T *xb, const cplx<T> *tw,
                                          int t)
 {
-  fftr_stage<T,M,V,S,0,true,CX>(v,xb,tw,t);
+  fftr_stage<T,M,V,S,0,true,CX>(v,xb,tw,fresh(t));
 }
 
 // fftr_blk with one-round exchanges through the index map XI, XORed by xm.
-template<typename T, int M, int V, int S, class XI>
+// FRESH: positions computed anew (see fresh()).
+template<typename T, int M, int V, int S, class XI, bool FRESH=true>
 __device__ __forceinline__ void fftr_blkx(cplx<T> *v, T *xb, const cplx<T> *tw,
                                           int t, int xm)
 {
-  fftr_stage<T,M,V,S,0,true,true,XI>(v,xb,tw,t,xm);
+  fftr_stage<T,M,V,S,0,true,true,XI>(v,xb,tw,FRESH ? fresh(t) : t,xm);
 }
 
 } // namespace fftwpp_amd

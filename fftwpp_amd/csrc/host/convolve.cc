@@ -14,6 +14,18 @@
 // which engine takes the rows (stage 1) of a dimension (2: register FFT).
 extern "C" int fftwpp_amd_internal_rows_fit(const fftwpp_amd_dim *d, int dtype);
 extern "C" int fftwpp_amd_internal_engine(const fftwpp_amd_dim *d, int stage);
+// the forward residue transforms of up to three arrays of one layout in one launch
+extern "C" int fftwpp_amd_internal_forward_arrays(const fftwpp_amd_dim *d, int dtype, int real,
+                                                  int n, const void *const *f, size_t S,
+                                                  size_t C, size_t nbatch, size_t bstride_in,
+                                                  void *const *F, size_t SF, size_t bstride_out,
+                                                  size_t r0, size_t nres, void *stream);
+extern "C" int fftwpp_amd_internal_backward_arrays(const fftwpp_amd_dim *d, int dtype, int n,
+                                                   const void *const *F, size_t SF,
+                                                   size_t bstride_in, void *const *f, size_t S,
+                                                   size_t C, size_t nbatch, size_t bstride_out,
+                                                   size_t r0, size_t nres, int accumulate,
+                                                   double scale, void *stream);
 // the item table {i rs, L, i L} of `rows` rows for the batched row kernel
 extern "C" int fftwpp_amd_internal_row_items(void *items, size_t rows, size_t rs,
                                              size_t L, void *stream);
@@ -1308,11 +1320,11 @@ void Convolution2::execComplex(void *out, const void *f0, const void *f1, bool n
     const size_t nres=std::min(Dx,qx-r0);
     const size_t rows=real ? maxrows : nres*mx;
     const bool first=r0 == 0, last=r0+nres == qx;
-    for(int a=0; a < 2; ++a) {
-      if(real)
-        check(fftwpp_amd_forward_real_many(fftx->dev,dtype,in[a],Sx,lyc,1,0,F[a],lyc,0,stream),"x forward");
-      else
-        check(fftwpp_amd_forward_many(fftx->dev,dtype,in[a],Sx,lyc,1,0,F[a],lyc,0,r0,nres,stream),"x forward");
+    // both inputs in one launch, unless their stages are timed one by one
+    const int na=timeline ? 1 : 2;
+    for(int a=0; a < 2; a += na) {
+      check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,real,na,in+a,Sx,lyc,1,0,F+a,lyc,0,
+                                               r0,nres,stream),"x forward");
       if(timeline) timeline->mark(real ? (a == 0 ? "x real forward f" : "x real forward g") : (a == 0 ? "x forward f" : "x forward g"));
     }
     if(rowHook)
@@ -1536,18 +1548,23 @@ void Convolution3::execComplex(void *out, const void *f0, const void *f1, bool n
     const size_t nres=std::min(Dx,qx-r0);
     const size_t nplanes=real ? maxplanes : nres*mx;
     const bool first=r0 == 0, last=r0+nres == qx;
-    // x forward: columns (y,z); non-contiguous y strides become batches
-    for(int a=0; a < 2; ++a) {
-      if(real && contiguous())
-        check(fftwpp_amd_forward_real_many(fftx->dev,dtype,in[a],Sx,plane,1,0,X[a],plane,0,stream),"x forward");
-      else if(real)
-        check(fftwpp_amd_forward_real_many(fftx->dev,dtype,in[a],Sx,Lz,Ly,Sy,X[a],plane,Lz,stream),"x forward");
-      else if(contiguous())
-        check(fftwpp_amd_forward_many(fftx->dev,dtype,in[a],Sx,plane,1,0,X[a],plane,0,r0,nres,stream),"x forward");
+    // x forward: columns (y,z); non-contiguous y strides become batches.  Both
+    // inputs in one launch (one long tail per stage instead of two: 255 x 255 x
+    // 128 Hermitian modes FP64 1023 -> 999 us), unless their stages are timed
+    // one by one or an x-transformed array exceeds the 256 MB Infinity Cache:
+    // then f's y stage runs at once on what its x stage left there (real 256^3
+    // FP64, 270 MB: 1204 us against 1257 us paired).
+    const int na=timeline || nplanes*plane*E > ((size_t) 256 << 20) ? 1 : 2;
+    for(int a=0; a < 2; a += na) {
+      if(contiguous())
+        check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,real,na,in+a,Sx,plane,1,0,X+a,plane,0,
+                                                 r0,nres,stream),"x forward");
       else
-        check(fftwpp_amd_forward_many(fftx->dev,dtype,in[a],Sx,Lz,Ly,Sy,X[a],plane,Lz,r0,nres,stream),"x forward");
+        check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,real,na,in+a,Sx,Lz,Ly,Sy,X+a,plane,Lz,
+                                                 r0,nres,stream),"x forward");
       if(timeline) timeline->mark(real ? (a == 0 ? "x real forward f" : "x real forward g") : (a == 0 ? "x forward f" : "x forward g"));
-      check(fftwpp_amd_forward_many(ffty->dev,dtype,X[a],Lz,Lz,nplanes,plane,Y[a],Lz,yplane,0,qy,stream),"y forward");
+      check(fftwpp_amd_internal_forward_arrays(ffty->dev,dtype,0,na,X+a,Lz,Lz,nplanes,plane,Y+a,Lz,yplane,
+                                               0,qy,stream),"y forward");
       if(timeline) timeline->mark(a == 0 ? "y forward f" : "y forward g");
     }
     if(rowHook)

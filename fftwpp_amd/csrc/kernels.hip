@@ -849,16 +849,40 @@ static bool cols_reg(const fftwpp_amd_dim *d)
   return d->L <= 2*m && m*d->q < ((size_t) 1 << 30);
 }
 
+// One array; `in` and `out` of array a of a set.
+static ColArrays col_arrays(const void *in, void *out)
+{
+  ColArrays io={};
+  io.n=1;
+  io.in[0]=in;
+  io.out[0]=out;
+  return io;
+}
+
+// Grid depth of a forward column launch of `blocks` blocks per array over nr
+// residues: one per array, times the parts the residues are dealt to when the
+// arrays' blocks leave compute units idle (256 CUs, two blocks of 512 threads
+// each).  A part reads its columns again, from the caches at these sizes.
+// 1023 x 512 modes, FP32 (64 blocks per array, 3 residues): two arrays in 128
+// blocks of three residues each took as long as one array alone.
+static unsigned col_depth(const ColArrays &io, size_t blocks, size_t nr)
+{
+  size_t parts=512/std::max<size_t>(1,blocks*(size_t) io.n);
+  parts=std::max<size_t>(1,std::min(parts,nr));
+  return (unsigned) (parts*(size_t) io.n);
+}
+
 template<typename T, int M>
-static int colreg_launch(const DimArgs &a, bool fwd, const void *in,
-                         size_t s_in, size_t bsi, void *out, size_t s_out,
+static int colreg_launch(const DimArgs &a, bool fwd, const ColArrays &io,
+                         size_t s_in, size_t bsi, size_t s_out,
                          size_t bso, size_t C, size_t nbatch, size_t r0,
                          size_t nres, int accumulate, double scale,
                          size_t ics, size_t ocs, hipStream_t st)
 {
   typedef ColReg<T,M> CR;
   size_t lds=M*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
-  const dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
+  dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
+  grid.z=fwd ? col_depth(io,(size_t) grid.x*nbatch,nres) : (unsigned) io.n;
   const bool p2=a.L > M;
   // the N residue twiddles in LDS when they fit without lowering occupancy
   auto zfit=[&](auto kernel) {
@@ -870,16 +894,14 @@ static int colreg_launch(const DimArgs &a, bool fwd, const void *in,
     if(p2) {
       if((rc=allow_lds(colfwd_reg_kernel<T,M,2>,lds_max()))) return rc;
       if((zl=zfit(colfwd_reg_kernel<T,M,2>))) lds += (size_t) a.N*sizeof(cplx<T>);
-      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
-                         (const cplx<T> *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
-                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,io,
+                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                          (int64_t) ics,(int64_t) ocs,zl);
     } else {
       if((rc=allow_lds(colfwd_reg_kernel<T,M,1>,lds_max()))) return rc;
       if((zl=zfit(colfwd_reg_kernel<T,M,1>))) lds += (size_t) a.N*sizeof(cplx<T>);
-      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
-                         (const cplx<T> *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
-                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+      hipLaunchKernelGGL((colfwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,io,
+                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,(int64_t) s_out,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                          (int64_t) ics,(int64_t) ocs,zl);
     }
     return launch_check("colfwd_reg_kernel");
@@ -887,28 +909,26 @@ static int colreg_launch(const DimArgs &a, bool fwd, const void *in,
   if(p2) {
     if((rc=allow_lds(colbwd_reg_kernel<T,M,2>,lds_max()))) return rc;
     if((zl=zfit(colbwd_reg_kernel<T,M,2>))) lds += (size_t) a.N*sizeof(cplx<T>);
-    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
-                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(cplx<T> *) out,
-                       (int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,io,
+                       (int64_t) s_in,(int64_t) bsi,(int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                        accumulate,(T) scale,(int64_t) ics,(int64_t) ocs,zl);
   } else {
     if((rc=allow_lds(colbwd_reg_kernel<T,M,1>,lds_max()))) return rc;
     if((zl=zfit(colbwd_reg_kernel<T,M,1>))) lds += (size_t) a.N*sizeof(cplx<T>);
-    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
-                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(cplx<T> *) out,
-                       (int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
+    hipLaunchKernelGGL((colbwd_reg_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,io,
+                       (int64_t) s_in,(int64_t) bsi,(int64_t) s_out,(int64_t) C,(int64_t) bso,(int64_t) r0,(int64_t) nres,
                        accumulate,(T) scale,(int64_t) ics,(int64_t) ocs,zl);
   }
   return launch_check("colbwd_reg_kernel");
 }
 
 template<typename T>
-static int colreg_t(const DimArgs &a, bool fwd, const void *in, size_t s_in,
-                    size_t bsi, void *out, size_t s_out, size_t bso, size_t C,
+static int colreg_t(const DimArgs &a, bool fwd, const ColArrays &io, size_t s_in,
+                    size_t bsi, size_t s_out, size_t bso, size_t C,
                     size_t nbatch, size_t r0, size_t nres, int accumulate,
                     double scale, size_t ics, size_t ocs, hipStream_t st)
 {
-#define FFTWPP_AMD_COLREG(MM) case MM: return colreg_launch<T,MM>(a,fwd,in,s_in,bsi,out,s_out,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
+#define FFTWPP_AMD_COLREG(MM) case MM: return colreg_launch<T,MM>(a,fwd,io,s_in,bsi,s_out,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
   switch(a.m) {
   FFTWPP_AMD_COLREG(16) FFTWPP_AMD_COLREG(32) FFTWPP_AMD_COLREG(64)
   FFTWPP_AMD_COLREG(128) FFTWPP_AMD_COLREG(256) FFTWPP_AMD_COLREG(512)
@@ -929,28 +949,29 @@ static bool cols_real(const fftwpp_amd_dim *d)
 }
 
 template<typename T, int M>
-static int colreal_launch(const DimArgs &a, bool fwd, const void *in,
-                          size_t s_in, size_t bsi, void *out, size_t s_out,
+static int colreal_launch(const DimArgs &a, bool fwd, const ColArrays &io,
+                          size_t s_in, size_t bsi, size_t s_out,
                           size_t bso, size_t C, size_t nbatch, double scale,
                           size_t ics, size_t ocs, hipStream_t st)
 {
   typedef ColReg<T,M> CR;
   const size_t lds=M*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
-  const dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
+  dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
+  if(fwd) grid.z=col_depth(io,(size_t) grid.x*nbatch,(size_t) RealKept::residues(a.q));
   const bool p2=a.L > M;
   int rc;
   if(fwd) {
     if(p2) {
       if((rc=allow_lds(colfwd_real_kernel<T,M,2>,lds))) return rc;
-      hipLaunchKernelGGL((colfwd_real_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
-                         (const T *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
-                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) ics,
+      hipLaunchKernelGGL((colfwd_real_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,io,
+                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,
+                         (int64_t) s_out,(int64_t) bso,(int64_t) ics,
                          (int64_t) ocs);
     } else {
       if((rc=allow_lds(colfwd_real_kernel<T,M,1>,lds))) return rc;
-      hipLaunchKernelGGL((colfwd_real_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
-                         (const T *) in,(int64_t) s_in,(int64_t) C,(int64_t) bsi,
-                         (cplx<T> *) out,(int64_t) s_out,(int64_t) bso,(int64_t) ics,
+      hipLaunchKernelGGL((colfwd_real_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,io,
+                         (int64_t) s_in,(int64_t) C,(int64_t) bsi,
+                         (int64_t) s_out,(int64_t) bso,(int64_t) ics,
                          (int64_t) ocs);
     }
     return launch_check("colfwd_real_kernel");
@@ -958,13 +979,13 @@ static int colreal_launch(const DimArgs &a, bool fwd, const void *in,
   if(p2) {
     if((rc=allow_lds(colbwd_real_kernel<T,M,2>,lds))) return rc;
     hipLaunchKernelGGL((colbwd_real_kernel<T,M,2>),grid,dim3(CR::NT),lds,st,a,
-                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(T *) out,
+                       (const cplx<T> *) io.in[0],(int64_t) s_in,(int64_t) bsi,(T *) io.out[0],
                        (int64_t) s_out,(int64_t) C,(int64_t) bso,(T) scale,(int64_t) ics,
                        (int64_t) ocs);
   } else {
     if((rc=allow_lds(colbwd_real_kernel<T,M,1>,lds))) return rc;
     hipLaunchKernelGGL((colbwd_real_kernel<T,M,1>),grid,dim3(CR::NT),lds,st,a,
-                       (const cplx<T> *) in,(int64_t) s_in,(int64_t) bsi,(T *) out,
+                       (const cplx<T> *) io.in[0],(int64_t) s_in,(int64_t) bsi,(T *) io.out[0],
                        (int64_t) s_out,(int64_t) C,(int64_t) bso,(T) scale,(int64_t) ics,
                        (int64_t) ocs);
   }
@@ -974,8 +995,8 @@ static int colreal_launch(const DimArgs &a, bool fwd, const void *in,
 // Single columns of many batch entries become the columns of one launch, as
 // in fwd_many_t.
 template<typename T>
-static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const void *in, size_t s_in,
-                     size_t bsi, void *out, size_t s_out, size_t bso, size_t C,
+static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const ColArrays &io, size_t s_in,
+                     size_t bsi, size_t s_out, size_t bso, size_t C,
                      size_t nbatch, double scale, hipStream_t st)
 {
   const DimArgs &a=sizeof(T) == 8 ? d->a64 : d->a32;
@@ -984,7 +1005,7 @@ static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const void *in, size_t s
     C=nbatch; ics=bsi; ocs=bso;
     nbatch=1; bsi=bso=0;
   }
-#define FFTWPP_AMD_COLREAL(MM) case MM: return colreal_launch<T,MM>(a,fwd,in,s_in,bsi,out,s_out,bso,C,nbatch,scale,ics,ocs,st);
+#define FFTWPP_AMD_COLREAL(MM) case MM: return colreal_launch<T,MM>(a,fwd,io,s_in,bsi,s_out,bso,C,nbatch,scale,ics,ocs,st);
   switch(a.m) {
   FFTWPP_AMD_COLREAL(16) FFTWPP_AMD_COLREAL(32) FFTWPP_AMD_COLREAL(64)
   FFTWPP_AMD_COLREAL(128) FFTWPP_AMD_COLREAL(256) FFTWPP_AMD_COLREAL(512)
@@ -995,8 +1016,8 @@ static int colreal_t(const fftwpp_amd_dim *d, bool fwd, const void *in, size_t s
 }
 
 template<typename T>
-static int fwd_many_t(const fftwpp_amd_dim *d, const void *f, size_t S,
-                      size_t C, size_t nbatch, size_t bsi, void *F,
+static int fwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t S,
+                      size_t C, size_t nbatch, size_t bsi,
                       size_t SF, size_t bso, size_t r0, size_t nres,
                       hipStream_t st)
 {
@@ -1013,19 +1034,20 @@ static int fwd_many_t(const fftwpp_amd_dim *d, const void *f, size_t S,
   if(ics == 1 && ocs == 1 && C >= (size_t) Col256<T>::TC && fast256(d,S,SF)) {
     constexpr int TC=Col256<T>::TC;
     dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
+    grid.z=col_depth(io,(size_t) grid.x*nbatch,nres);
     size_t lds=col256_lds<T>(nres);
     int rc=allow_lds(colfwd256_kernel<T>,lds);
     if(rc) return rc;
     hipLaunchKernelGGL((colfwd256_kernel<T>),grid,dim3(16*TC),lds,st,
-                       (const cplx<T> *) f,(int64_t) S,(int64_t) C,(int64_t) bsi,
-                       (cplx<T> *) F,(int64_t) SF,(int64_t) bso,(int) d->L,
+                       io,(int64_t) S,(int64_t) C,(int64_t) bsi,
+                       (int64_t) SF,(int64_t) bso,(int) d->L,
                        (int64_t) r0,(int64_t) nres,(const cplx<T> *) a.zN,(int64_t) d->q);
     return launch_check("colfwd256_kernel");
   }
   // register columns: tiles of several columns below m = 2048, so a single
   // short column goes to the LDS path
   if(cols_reg(d) && (C >= 8 || d->m >= 2048))
-    return colreg_t<T>(a,true,f,S,bsi,F,SF,bso,C,nbatch,r0,nres,0,1.0,ics,ocs,st);
+    return colreg_t<T>(a,true,io,S,bsi,SF,bso,C,nbatch,r0,nres,0,1.0,ics,ocs,st);
   size_t elt=sizeof(cplx<T>);
   size_t per=2*(d->m+1)*elt;
   if(per > lds_max()) return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"m too large for the LDS transform");
@@ -1035,16 +1057,19 @@ static int fwd_many_t(const fftwpp_amd_dim *d, const void *f, size_t S,
   dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
   int rc=allow_lds(fwd_many_kernel<T>,lds);
   if(rc) return rc;
-  hipLaunchKernelGGL(fwd_many_kernel<T>,grid,dim3(256),lds,st,a,
-                     (const cplx<T> *) f,(int64_t) S,(int64_t) C,
-                     (int64_t) bsi,(cplx<T> *) F,(int64_t) SF,(int64_t) bso,
-                     (int64_t) r0,(int64_t) nres,(int) TC,(int64_t) ics,(int64_t) ocs);
-  return launch_check("fwd_many_kernel");
+  for(int x=0; x < io.n; ++x) {
+    hipLaunchKernelGGL(fwd_many_kernel<T>,grid,dim3(256),lds,st,a,
+                       (const cplx<T> *) io.in[x],(int64_t) S,(int64_t) C,
+                       (int64_t) bsi,(cplx<T> *) io.out[x],(int64_t) SF,(int64_t) bso,
+                       (int64_t) r0,(int64_t) nres,(int) TC,(int64_t) ics,(int64_t) ocs);
+    if((rc=launch_check("fwd_many_kernel"))) return rc;
+  }
+  return FFTWPP_AMD_OK;
 }
 
 template<typename T>
-static int bwd_many_t(const fftwpp_amd_dim *d, const void *F, size_t SF,
-                      size_t bsi, void *f, size_t S, size_t C,
+static int bwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t SF,
+                      size_t bsi, size_t S, size_t C,
                       size_t nbatch, size_t bso, size_t r0, size_t nres,
                       int accumulate, double scale, hipStream_t st)
 {
@@ -1057,19 +1082,19 @@ static int bwd_many_t(const fftwpp_amd_dim *d, const void *F, size_t SF,
   }
   if(ics == 1 && ocs == 1 && C >= (size_t) Col256<T>::TC && fast256(d,S,SF)) {
     constexpr int TC=Col256<T>::TC;
-    dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
+    dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch,(unsigned) io.n);
     size_t lds=col256_lds<T>(nres);
     int rc=allow_lds(colbwd256_kernel<T>,lds);
     if(rc) return rc;
     hipLaunchKernelGGL((colbwd256_kernel<T>),grid,dim3(16*TC),lds,st,
-                       (const cplx<T> *) F,(int64_t) SF,(int64_t) bsi,(cplx<T> *) f,
+                       io,(int64_t) SF,(int64_t) bsi,
                        (int64_t) S,(int64_t) C,(int64_t) bso,(int) d->L,(int64_t) r0,
                        (int64_t) nres,accumulate,(T) scale,(const cplx<T> *) a.zN,
                        (int64_t) d->q);
     return launch_check("colbwd256_kernel");
   }
   if(cols_reg(d) && (C >= 8 || d->m >= 2048))
-    return colreg_t<T>(a,false,F,SF,bsi,f,S,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
+    return colreg_t<T>(a,false,io,SF,bsi,S,bso,C,nbatch,r0,nres,accumulate,scale,ics,ocs,st);
   size_t elt=sizeof(cplx<T>);
   size_t per=2*(d->m+1)*elt;
   if(per > lds_max()) return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"m too large for the LDS transform");
@@ -1079,12 +1104,15 @@ static int bwd_many_t(const fftwpp_amd_dim *d, const void *F, size_t SF,
   dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
   int rc=allow_lds(bwd_many_kernel<T>,lds);
   if(rc) return rc;
-  hipLaunchKernelGGL(bwd_many_kernel<T>,grid,dim3(256),lds,st,a,
-                     (const cplx<T> *) F,(int64_t) SF,(int64_t) bsi,
-                     (cplx<T> *) f,(int64_t) S,(int64_t) C,(int64_t) bso,
-                     (int64_t) r0,(int64_t) nres,accumulate,(T) scale,(int) TC,
-                     (int64_t) ics,(int64_t) ocs);
-  return launch_check("bwd_many_kernel");
+  for(int x=0; x < io.n; ++x) {
+    hipLaunchKernelGGL(bwd_many_kernel<T>,grid,dim3(256),lds,st,a,
+                       (const cplx<T> *) io.in[x],(int64_t) SF,(int64_t) bsi,
+                       (cplx<T> *) io.out[x],(int64_t) S,(int64_t) C,(int64_t) bso,
+                       (int64_t) r0,(int64_t) nres,accumulate,(T) scale,(int) TC,
+                       (int64_t) ics,(int64_t) ocs);
+    if((rc=launch_check("bwd_many_kernel"))) return rc;
+  }
+  return FFTWPP_AMD_OK;
 }
 
 // LDS bytes of batch_conv_kernel for sub-FFT size m, TR items and (with
@@ -1650,6 +1678,40 @@ size_t fftwpp_amd_max_m(int dtype)
 }
 
 
+// fftwpp_amd_forward_many (real = 0) or fftwpp_amd_forward_real_many (real =
+// 1: every kept plane, r0 and nres unused) of n <= 3 arrays of the same
+// layout in one launch; the inputs may be the same array, the outputs not.
+int fftwpp_amd_internal_forward_arrays(const fftwpp_amd_dim *d, int dtype, int real, int n,
+                                       const void *const *f, size_t S, size_t C,
+                                       size_t nbatch, size_t bstride_in, void *const *F,
+                                       size_t SF, size_t bstride_out, size_t r0, size_t nres,
+                                       void *stream)
+{
+  if(!d || !f || !F || n < 1 || n > MAXARRAYS) return fail(FFTWPP_AMD_ERR_ARG,"bad array set");
+  ColArrays io={};
+  io.n=n;
+  for(int a=0; a < n; ++a) {
+    if(!f[a] || !F[a]) return fail(FFTWPP_AMD_ERR_ARG,"null argument");
+    io.in[a]=f[a];
+    io.out[a]=F[a];
+  }
+  if(d->kind == FFTWPP_AMD_KIND_HERMITIAN)
+    return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"Hermitian dimensions are innermost only");
+  if(real && !cols_real(d))
+    return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"real residue transforms take power-of-two m in [16, 4096] and L <= 2m");
+  if((!real && r0+nres > d->q) || C == 0 || nbatch == 0)
+    return fail(FFTWPP_AMD_ERR_ARG,"bad residue range or shape");
+  if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
+  hipStream_t st=(hipStream_t) stream;
+  if(real)
+    return dtype == FFTWPP_AMD_F32 ?
+      colreal_t<float>(d,true,io,S,bstride_in,SF,bstride_out,C,nbatch,1.0,st) :
+      colreal_t<double>(d,true,io,S,bstride_in,SF,bstride_out,C,nbatch,1.0,st);
+  return dtype == FFTWPP_AMD_F32 ?
+    fwd_many_t<float>(d,io,S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st) :
+    fwd_many_t<double>(d,io,S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st);
+}
+
 int fftwpp_amd_forward_many(const fftwpp_amd_dim *d, int dtype,
                             const void *f, size_t S, size_t C,
                             size_t nbatch, size_t bstride_in, void *F,
@@ -1663,10 +1725,35 @@ int fftwpp_amd_forward_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    fwd_many_t<float>(d,f,S,C,nbatch,bstride_in,F,SF,bstride_out,r0,nres,st) :
-    fwd_many_t<double>(d,f,S,C,nbatch,bstride_in,F,SF,bstride_out,r0,nres,st);
+    fwd_many_t<float>(d,col_arrays(f,F),S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st) :
+    fwd_many_t<double>(d,col_arrays(f,F),S,C,nbatch,bstride_in,SF,bstride_out,r0,nres,st);
 }
 
+
+// fftwpp_amd_backward_many of n <= 3 arrays of the same layout in one launch.
+int fftwpp_amd_internal_backward_arrays(const fftwpp_amd_dim *d, int dtype, int n,
+                                        const void *const *F, size_t SF, size_t bstride_in,
+                                        void *const *f, size_t S, size_t C, size_t nbatch,
+                                        size_t bstride_out, size_t r0, size_t nres,
+                                        int accumulate, double scale, void *stream)
+{
+  if(!d || !f || !F || n < 1 || n > MAXARRAYS) return fail(FFTWPP_AMD_ERR_ARG,"bad array set");
+  ColArrays io={};
+  io.n=n;
+  for(int a=0; a < n; ++a) {
+    if(!f[a] || !F[a]) return fail(FFTWPP_AMD_ERR_ARG,"null argument");
+    io.in[a]=F[a];
+    io.out[a]=f[a];
+  }
+  if(d->kind == FFTWPP_AMD_KIND_HERMITIAN)
+    return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"Hermitian dimensions are innermost only");
+  if(r0+nres > d->q || nres == 0 || C == 0 || nbatch == 0) return fail(FFTWPP_AMD_ERR_ARG,"bad residue range or shape");
+  if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
+  hipStream_t st=(hipStream_t) stream;
+  return dtype == FFTWPP_AMD_F32 ?
+    bwd_many_t<float>(d,io,SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st) :
+    bwd_many_t<double>(d,io,SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st);
+}
 
 int fftwpp_amd_backward_many(const fftwpp_amd_dim *d, int dtype,
                              const void *F, size_t SF, size_t bstride_in,
@@ -1681,8 +1768,8 @@ int fftwpp_amd_backward_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    bwd_many_t<float>(d,F,SF,bstride_in,f,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st) :
-    bwd_many_t<double>(d,F,SF,bstride_in,f,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st);
+    bwd_many_t<float>(d,col_arrays(F,f),SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st) :
+    bwd_many_t<double>(d,col_arrays(F,f),SF,bstride_in,S,C,nbatch,bstride_out,r0,nres,accumulate,scale,st);
 }
 
 
@@ -1710,8 +1797,8 @@ int fftwpp_amd_forward_real_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    colreal_t<float>(d,true,f,S,bstride_in,F,SF,bstride_out,C,nbatch,1.0,st) :
-    colreal_t<double>(d,true,f,S,bstride_in,F,SF,bstride_out,C,nbatch,1.0,st);
+    colreal_t<float>(d,true,col_arrays(f,F),S,bstride_in,SF,bstride_out,C,nbatch,1.0,st) :
+    colreal_t<double>(d,true,col_arrays(f,F),S,bstride_in,SF,bstride_out,C,nbatch,1.0,st);
 }
 
 int fftwpp_amd_backward_real_many(const fftwpp_amd_dim *d, int dtype,
@@ -1726,8 +1813,8 @@ int fftwpp_amd_backward_real_many(const fftwpp_amd_dim *d, int dtype,
   if(S < C || SF < C) return fail(FFTWPP_AMD_ERR_ARG,"stride smaller than count");
   hipStream_t st=(hipStream_t) stream;
   return dtype == FFTWPP_AMD_F32 ?
-    colreal_t<float>(d,false,F,SF,bstride_in,f,S,bstride_out,C,nbatch,scale,st) :
-    colreal_t<double>(d,false,F,SF,bstride_in,f,S,bstride_out,C,nbatch,scale,st);
+    colreal_t<float>(d,false,col_arrays(F,f),SF,bstride_in,S,bstride_out,C,nbatch,scale,st) :
+    colreal_t<double>(d,false,col_arrays(F,f),SF,bstride_in,S,bstride_out,C,nbatch,scale,st);
 }
 
 int fftwpp_amd_conv_rows(const fftwpp_amd_dim *d, int dtype, int mult,

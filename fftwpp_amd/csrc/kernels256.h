@@ -54,12 +54,14 @@ inline size_t row256_lds(int NR, size_t q)
 }
 
 // Forward residue transforms of one column: for each residue r = r0 + rr,
-// F_r(s) = DFT_256[w_N^{r k} f(k)](s), written at Fb + rr*256*SF.
+// F_r(s) = DFT_256[w_N^{r k} f(k)](s), written at Fb + rr*256*SF; the block
+// takes every parts-th rr from part on.
 template<typename T>
 __device__ __forceinline__ void colfwd_body(const cplx<T> *fb, cplx<T> *Fb,
                                             int64_t S, int64_t SF, bool ok,
                                             int c, int j, int L, int64_t r0,
-                                            int64_t nres, const cplx<T> *rtab,
+                                            int64_t nres, int part, int parts,
+                                            const cplx<T> *rtab,
                                             const cplx<T> *tw16, T *row, int h)
 {
   const unsigned lin=(unsigned) (c+j*S);
@@ -71,7 +73,7 @@ __device__ __forceinline__ void colfwd_body(const cplx<T> *fb, cplx<T> *Fb,
     const cplx<T> *bk=fb+(int64_t) 16*k*S;
     x0[k]=(ok && j+16*k < L) ? bk[lin] : zero<T>();
   }
-  for(int64_t rr=0; rr < nres; ++rr) {
+  for(int64_t rr=part; rr < nres; rr += parts) {
     const int64_t r=r0+rr;
     const cplx<T> *rt=rtab+256*rr;
     cplx<T> v[16];
@@ -131,8 +133,8 @@ __device__ __forceinline__ void colbwd_body(const cplx<T> *Fb, cplx<T> *fb,
 
 template<typename T>
 __global__ void __launch_bounds__(16*Col256<T>::TC,sizeof(T) == 4 ? 3 : 2)
-colfwd256_kernel(const cplx<T> *f, int64_t S, int64_t C, int64_t bsi,
-                 cplx<T> *F, int64_t SF, int64_t bso, int L, int64_t r0,
+colfwd256_kernel(ColArrays io, int64_t S, int64_t C, int64_t bsi,
+                 int64_t SF, int64_t bso, int L, int64_t r0,
                  int64_t nres, const cplx<T> *zN, int64_t q)
 {
   constexpr int TC=Col256<T>::TC;
@@ -146,14 +148,15 @@ colfwd256_kernel(const cplx<T> *f, int64_t S, int64_t C, int64_t bsi,
   T *row=reinterpret_cast<T *>(tw16+256)+c*Col256<T>::CS;
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
-  const cplx<T> *fb=f+(int64_t) blockIdx.y*bsi+c0;
-  cplx<T> *Fb=F+(int64_t) blockIdx.y*bso+c0;
-  colfwd_body<T>(fb,Fb,S,SF,ok,c,j,L,r0,nres,rtab,tw16,row,Col256<T>::swz(c));
+  const ColBlock bk=col_block(io);
+  const cplx<T> *fb=(const cplx<T> *) bk.in+(int64_t) blockIdx.y*bsi+c0;
+  cplx<T> *Fb=(cplx<T> *) bk.out+(int64_t) blockIdx.y*bso+c0;
+  colfwd_body<T>(fb,Fb,S,SF,ok,c,j,L,r0,nres,bk.part,bk.parts,rtab,tw16,row,Col256<T>::swz(c));
 }
 
 template<typename T>
 __global__ void __launch_bounds__(16*Col256<T>::TC,sizeof(T) == 4 ? 3 : 2)
-colbwd256_kernel(const cplx<T> *F, int64_t SF, int64_t bsi, cplx<T> *f,
+colbwd256_kernel(ColArrays io, int64_t SF, int64_t bsi,
                  int64_t S, int64_t C, int64_t bso, int L, int64_t r0,
                  int64_t nres, int accumulate, T scale, const cplx<T> *zN,
                  int64_t q)
@@ -169,8 +172,9 @@ colbwd256_kernel(const cplx<T> *F, int64_t SF, int64_t bsi, cplx<T> *f,
   T *row=reinterpret_cast<T *>(tw16+256)+c*Col256<T>::CS;
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
-  const cplx<T> *Fb=F+(int64_t) blockIdx.y*bsi+c0;
-  cplx<T> *fb=f+(int64_t) blockIdx.y*bso+c0;
+  const ColBlock bk=col_block(io);
+  const cplx<T> *Fb=(const cplx<T> *) bk.in+(int64_t) blockIdx.y*bsi+c0;
+  cplx<T> *fb=(cplx<T> *) bk.out+(int64_t) blockIdx.y*bso+c0;
   colbwd_body<T>(Fb,fb,S,SF,ok,c,j,L,r0,nres,accumulate,scale,rtab,tw16,row,
                  Col256<T>::swz(c));
 }

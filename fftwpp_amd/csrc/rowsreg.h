@@ -80,18 +80,21 @@ __device__ __forceinline__ void rowreg_combine(cplx<T> *acc, T *xbase, T *xb,
 // sums are added through LDS before the row is written.  Dynamic LDS: M
 // complex twiddles + slots * 2 RPlan<M,V>::PAD scalar words.
 //
-// Bound by the chain of LDS exchanges at two waves per SIMD (FP64: 176-218
-// registers; a bound of three waves spills, and loading the next row ahead
-// costs more registers than it hides).  The branch-free loads, one register
-// per exchange instead of one per access and the product chosen once per row
-// took 65536 rows of 120 points (q = 2, FP64) from 152 to 126 us, 2048 rows of
-// 1000 points padded to 2048 from 56 to 49 us (FP64) and 31.5 to 25.6 us
-// (FP32), one such row from 10.1 to 9.0 us.
-// W: waves per SIMD asked of the compiler; the short FP32 rows of the
-// library's own products fit four without spills (66 against 73 us with two at
-// M = 128); a caller's functor keeps the registers of two.
+// Bound by the chain of LDS exchanges, with two or three waves per SIMD in
+// FP64 (166-175 registers: the two transforms and the residue sums alone are
+// 96) and four or five in FP32 (about 100).  Branch-free loads, one register
+// per exchange instead of one per access, positions computed anew per
+// transform (fresh) and the product chosen once per row took 65536 rows of 120
+// points (q = 2) from 152 to 113 us in FP64 and from 72 to 55 us in FP32, 8192
+// rows of 500 points from 79 to 60 and from 52 to 38 us, 2048 rows of 1000
+// points padded to 2048 from 56 to 46 and from 31.5 to 25 us, one such FP64
+// row from 10.1 to 9.0 us.
+// W: waves per SIMD asked of the compiler; three in FP64 where the library's
+// own products fit without spills and LDS leaves room for the blocks (113
+// against 124 us at M = 128); a caller's functor keeps the registers of two.
 template<typename T, int M, int RP, class Op> struct RowCx {
-  static constexpr int W=sizeof(T) == 4 && RP*M <= 512 && std::is_same<Op,RunMult>::value ? 4 : 2;
+  static constexpr bool MORE=sizeof(T) == 8 && RP == 1 && M >= 128 && M <= 512;
+  static constexpr int W=MORE && std::is_same<Op,RunMult>::value ? 3 : 2;
 };
 template<typename T, int M, int RP, class Op>
 __global__ void __launch_bounds__(RP*M/RowV::V > 256 ? 512 : 256,(RowCx<T,M,RP,Op>::W))
@@ -371,6 +374,9 @@ struct HRowPk {
   static constexpr int TPS=M/V;
   static constexpr int SLOTS=256/TPS > 0 ? 256/TPS : 1;
   static constexpr int NT=SLOTS*TPS;
+  // waves per SIMD where the short rows fit them without spills (150 and 90
+  // registers)
+  static constexpr int W=M > 256 ? 2 : sizeof(T) == 4 ? 4 : 3;
 };
 
 template<typename T, int M>
@@ -381,7 +387,7 @@ inline size_t hrowpk_lds(int q)
 }
 
 template<typename T, int M, class Op>
-__global__ void __launch_bounds__((HRowPk<T,M>::NT))
+__global__ void __launch_bounds__((HRowPk<T,M>::NT),(HRowPk<T,M>::W))
 hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
               cplx<T> *out, int64_t os, T scale, Op op)
 {
@@ -421,12 +427,15 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
     const auto rop=bind_row(op,row);
     for(int r1=0; r1 < q; r1 += 2) {
       const int r2=r1+1 < q ? r1+1 : -1;
-      const cplx<T> b1=zN[t*r1];
+      // (the loop's own positions too on short rows: 203 -> 183 us at M = 64,
+      // longer ones lose 2%)
+      const int ti=M <= 256 ? fresh(t) : t;
+      const cplx<T> b1=zN[ti*r1];
       // both residues folded from one read of the row
       cplx<T> X[V], X2[V];
       T p1[V];
       hpk_fold2<T,M>(X,X2,rf,rg,tq+r1*(V+1),tq+(r2 >= 0 ? r2 : r1)*(V+1),b1,
-                       r2 >= 0 ? zN[t*r2] : b1,t,r1,r2 >= 0 ? r2 : r1,H,ro);
+                       r2 >= 0 ? zN[ti*r2] : b1,ti,r1,r2 >= 0 ? r2 : r1,H,ro);
       if(r2 >= 0) {
         // the two residues' transforms with their butterflies interleaved
         fftr_pair<T,M,V,1>(X,X2,xb,tw,t);
@@ -442,36 +451,38 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
       }
       fftr<T,M,V,-1,true>(X,xb,tw,t);
       // mirror elements Z(M - sigma) through LDS
+      const int tm=M <= 256 ? fresh(t) : t;
 #pragma unroll
       for(int k=0; k < V; ++k) {
-        const int e=xidx<T,M,V>(t+TPS*k);
+        const int e=xidx<T,M,V>(tm+TPS*k);
         xb[e]=X[k].x;
         xb[P::PAD+e]=X[k].y;
       }
       rsync<TPS>();
       const cplx<T> *t1=tq+r1*(V+1), *t2=tq+(r2 >= 0 ? r2 : 0)*(V+1);
-      const cplx<T> b2=r2 >= 0 ? zN[t*r2] : mk((T) 0,(T) 0);
+      const cplx<T> c1=zN[tm*r1], c2=r2 >= 0 ? zN[tm*r2] : mk((T) 0,(T) 0);
 #pragma unroll
       for(int k=0; k < V; ++k) {
-        const int e=xidx<T,M,V>((M-(t+TPS*k)) & (M-1));
+        const int e=xidx<T,M,V>((M-(tm+TPS*k)) & (M-1));
         const cplx<T> z=X[k], zc=mk(xb[e],-xb[P::PAD+e]);
-        cplx<T> v=mulc((T) 0.5*(z+zc),b1*t1[k]);
-        if(r2 >= 0) v=v+mulc(muli((T) 0.5*(z-zc),-1),b2*t2[k]);
+        cplx<T> v=mulc((T) 0.5*(z+zc),c1*t1[k]);
+        if(r2 >= 0) v=v+mulc(muli((T) 0.5*(z-zc),-1),c2*t2[k]);
         acc[k]=acc[k]+v;
       }
       rsync<TPS>();
     }
     if(live) {
+      const int to=M <= 256 ? fresh(t) : t;
       if constexpr(TPS >= 64) {
         const __amdgpu_buffer_rsrc_t rw=buf_rsrc(out+row*os,H);
 #pragma unroll
         for(int k=0; k < V; ++k)
-          if(t+TPS*k < H) st_buf<T>(rw,(unsigned) (t+TPS*k)*E,0,scale*acc[k]);
+          if(to+TPS*k < H) st_buf<T>(rw,(unsigned) (to+TPS*k)*E,0,scale*acc[k]);
       } else {
         cplx<T> *orow=out+row*os;
 #pragma unroll
         for(int k=0; k < V; ++k)
-          if(t+TPS*k < H) orow[t+TPS*k]=scale*acc[k];
+          if(to+TPS*k < H) orow[to+TPS*k]=scale*acc[k];
       }
     }
   }
@@ -645,13 +656,29 @@ template<typename T, int M> struct ColReg {
   static __device__ __forceinline__ int xm(int c) { return (c*BETA) & (M < 32 ? M-1 : 31); }
 };
 
+// Waves per SIMD asked of the complex column kernels: four, so that two blocks
+// of 512 threads share a CU and one loads while the other transforms, where
+// the registers allow it without spills: all FP32 columns (at most 114), FP64
+// with p = 1 (110 forward; 122 to 128 backward with M = 64 and 512 above) and
+// M below 4096, whose LDS holds one block.
+template<typename T, int M, int P2, bool FWD> struct ColW {
+  static constexpr bool FIT=P2 == 1 && M < 4096 && (FWD || (M != 64 && M != 512));
+  static constexpr int W=sizeof(T) == 4 || FIT ? 4 : 2;
+};
+
 // The stage twiddle table of the column kernels (tw) and the residue twiddle
 // table they read: zlds = 1 copies the dimension's N twiddles into LDS after
 // the exchange areas (the residue twiddles are per-lane gathers, about 10%
 // faster from LDS; the host asks for it when the LDS fits without lowering
 // occupancy), else the table in global memory.  Ends with a block barrier.
+template<typename T, int M> struct ColTwiddles {
+  const cplx<T> *zl;      // LDS copy
+  const cplx<T> *zN;      // global table
+  int zlds;
+};
+
 template<typename T, int M>
-__device__ __forceinline__ const cplx<T> *col_twiddles(const DimArgs &d, cplx<T> *tw, int zlds)
+__device__ __forceinline__ ColTwiddles<T,M> col_twiddles(const DimArgs &d, cplx<T> *tw, int zlds)
 {
   typedef ColReg<T,M> CR;
   const cplx<T> *zN=(const cplx<T> *) d.zN;
@@ -660,23 +687,50 @@ __device__ __forceinline__ const cplx<T> *col_twiddles(const DimArgs &d, cplx<T>
   if(zlds)
     for(int e=threadIdx.x; e < (int) d.N; e += CR::NT) zl[e]=zN[e];
   __syncthreads();
-  return zlds ? zl : zN;
+  return ColTwiddles<T,M>{zl,zN,zlds};
 }
 
-// F[b][(r-r0) M + s][c] = sum_j f[b][j][c] w_N^{(j+k0)(q s + r)}, j < L;
+// w[i][k] = w_N^{(j0 + M i + k0) r} of the elements kk + k, k < KH, of a
+// column, all loaded before the first use (r = 0 reads 1; a load per branch
+// made each wait for the previous one).  One uniform branch on the table's place: a pointer to
+// either would make every load a generic one.
+template<typename T, int M, int P2, int KH>
+__device__ __forceinline__ void col_residue(cplx<T> (*w)[KH], const ColTwiddles<T,M> &z,
+                                            int t, int kk, int k0, int r, int N)
+{
+  constexpr int TPS=M/RowV::V;
+  typedef const __attribute__((address_space(3))) T *lds_words;
+  typedef const __attribute__((address_space(1))) T *global_words;
+  auto loads=[&](auto zt) {
+#pragma unroll
+    for(int k=0; k < KH; ++k) {
+      const int j0=(t+TPS*(kk+k)-k0) & (M-1);
+#pragma unroll
+      for(int i=0; i < P2; ++i) {
+        const int e=2*wrapN((j0+M*i+k0)*r,N);
+        w[i][k]=mk(zt[e],zt[e+1]);
+      }
+    }
+  };
+  if(z.zlds) loads((lds_words) reinterpret_cast<const T *>(z.zl));
+  else loads((global_words) reinterpret_cast<const T *>(z.zN));
+}
+
+// F[b][(r-r0) M + s][c] = sum_j f[b][j][c] w_N^{(j+k0)(q s + r)}, j < L, for
+// each array (f, F) of io;
 // column c starts at c*ics of f and c*ocs of F (unit strides for
 // interleaved columns, row strides for contiguous rows taken as columns).
 template<typename T, int M, int P2>
-__global__ void __launch_bounds__(512)
-colfwd_reg_kernel(DimArgs d, const cplx<T> *f, int64_t S, int64_t C,
-                  int64_t bsi, cplx<T> *F, int64_t SF, int64_t bso, int64_t r0,
+__global__ void __launch_bounds__(512,(ColW<T,M,P2,true>::W))
+colfwd_reg_kernel(DimArgs d, ColArrays io, int64_t S, int64_t C,
+                  int64_t bsi, int64_t SF, int64_t bso, int64_t r0,
                   int64_t nres, int64_t ics, int64_t ocs, int zlds)
 {
   typedef ColReg<T,M> CR;
   constexpr int V=CR::V, TPS=CR::TPS, TC=CR::TC;
   extern __shared__ char smem_raw[];
   cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
-  const cplx<T> *zN=col_twiddles<T,M>(d,tw,zlds);
+  const ColTwiddles<T,M> zt=col_twiddles<T,M>(d,tw,zlds);
   // interleaved columns: consecutive lanes on consecutive columns; rows
   // (column stride ics > 1): a row's threads on consecutive lanes
   const bool rowmap=ics != 1;
@@ -686,8 +740,9 @@ colfwd_reg_kernel(DimArgs d, const cplx<T> *f, int64_t S, int64_t C,
   const int xm=CR::xm(c);
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
-  const cplx<T> *fb=f+(int64_t) blockIdx.y*bsi+(c0+c)*ics;
-  cplx<T> *Fb=F+(int64_t) blockIdx.y*bso+(c0+c)*ocs;
+  const ColBlock bk=col_block(io);
+  const cplx<T> *fb=(const cplx<T> *) bk.in+(int64_t) blockIdx.y*bsi+(c0+c)*ics;
+  cplx<T> *Fb=(cplx<T> *) bk.out+(int64_t) blockIdx.y*bso+(c0+c)*ocs;
   const int N=(int) d.N, L=(int) d.L, k0=(int) d.k0;
   // the column, read once: element j = j0 + M i with j0 = (sigma - k0) mod M
   cplx<T> raw[P2][V];
@@ -700,17 +755,10 @@ colfwd_reg_kernel(DimArgs d, const cplx<T> *f, int64_t S, int64_t C,
       raw[i][k]=ok && j < L ? fb[(int64_t) j*S] : mk((T) 0,(T) 0);
     }
   }
-  for(int64_t rr=0; rr < nres; ++rr) {
+  for(int64_t rr=bk.part; rr < nres; rr += bk.parts) {
     const int r=(int) (r0+rr);
-    // the residue's twiddles loaded before the first use (r = 0 reads
-    // w_N^0 = 1): a load per branch made each wait for the previous one
     cplx<T> w[P2][V];
-#pragma unroll
-    for(int k=0; k < V; ++k) {
-      const int j0=(t+TPS*k-k0) & (M-1);
-#pragma unroll
-      for(int i=0; i < P2; ++i) w[i][k]=zN[wrapN((j0+M*i+k0)*r,N)];
-    }
+    col_residue<T,M,P2>(w,zt,fresh(t),0,k0,r,N);
     cplx<T> X[V];
 #pragma unroll
     for(int k=0; k < V; ++k) {
@@ -719,21 +767,22 @@ colfwd_reg_kernel(DimArgs d, const cplx<T> *f, int64_t S, int64_t C,
       for(int i=1; i < P2; ++i) a=a+raw[i][k]*w[i][k];
       X[k]=a;
     }
-    fftr_blkx<T,M,V,1,CR>(X,xb,tw,t,xm);
+    fftr_blkx<T,M,V,1,CR,(sizeof(T) == 8 || P2 == 2)>(X,xb,tw,t,xm);
     if(ok) {
       cplx<T> *Fr=Fb+rr*M*SF;
+      const int tf=fresh(t);
 #pragma unroll
-      for(int k=0; k < V; ++k) Fr[(int64_t) (t+TPS*k)*SF]=X[k];
+      for(int k=0; k < V; ++k) Fr[(int64_t) (tf+TPS*k)*SF]=X[k];
     }
   }
 }
 
 // f[b][j][c] = scale * ((accumulate ? f : 0) + sum_r w_N^{-(j+k0) r}
-// DFT^{-1}[F_r]((j+k0) mod M)), j < L.
+// DFT^{-1}[F_r]((j+k0) mod M)), j < L, for each array (F, f) of io.
 template<typename T, int M, int P2>
-__global__ void __launch_bounds__(512)
-colbwd_reg_kernel(DimArgs d, const cplx<T> *F, int64_t SF, int64_t bsi,
-                  cplx<T> *f, int64_t S, int64_t C, int64_t bso, int64_t r0,
+__global__ void __launch_bounds__(512,(ColW<T,M,P2,false>::W))
+colbwd_reg_kernel(DimArgs d, ColArrays io, int64_t SF, int64_t bsi,
+                  int64_t S, int64_t C, int64_t bso, int64_t r0,
                   int64_t nres, int accumulate, T scale, int64_t ics, int64_t ocs,
                   int zlds)
 {
@@ -741,7 +790,7 @@ colbwd_reg_kernel(DimArgs d, const cplx<T> *F, int64_t SF, int64_t bsi,
   constexpr int V=CR::V, TPS=CR::TPS, TC=CR::TC;
   extern __shared__ char smem_raw[];
   cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
-  const cplx<T> *zN=col_twiddles<T,M>(d,tw,zlds);
+  const ColTwiddles<T,M> zt=col_twiddles<T,M>(d,tw,zlds);
   // interleaved columns: consecutive lanes on consecutive columns; rows
   // (column stride ics > 1): a row's threads on consecutive lanes
   const bool rowmap=ics != 1;
@@ -751,8 +800,9 @@ colbwd_reg_kernel(DimArgs d, const cplx<T> *F, int64_t SF, int64_t bsi,
   const int xm=CR::xm(c);
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
-  const cplx<T> *Fb=F+(int64_t) blockIdx.y*bsi+(c0+c)*ics;
-  cplx<T> *fb=f+(int64_t) blockIdx.y*bso+(c0+c)*ocs;
+  const ColBlock bk=col_block(io);
+  const cplx<T> *Fb=(const cplx<T> *) bk.in+(int64_t) blockIdx.y*bsi+(c0+c)*ics;
+  cplx<T> *fb=(cplx<T> *) bk.out+(int64_t) blockIdx.y*bso+(c0+c)*ocs;
   const int N=(int) d.N, L=(int) d.L, k0=(int) d.k0;
   cplx<T> acc[P2][V];
 #pragma unroll
@@ -762,28 +812,28 @@ colbwd_reg_kernel(DimArgs d, const cplx<T> *F, int64_t SF, int64_t bsi,
   for(int64_t rr=0; rr < nres; ++rr) {
     const int r=(int) (r0+rr);
     const cplx<T> *Fr=Fb+rr*M*SF;
+    const int tf=fresh(t);
     cplx<T> X[V];
 #pragma unroll
-    for(int k=0; k < V; ++k) X[k]=ok ? Fr[(int64_t) (t+TPS*k)*SF] : mk((T) 0,(T) 0);
-    fftr_blkx<T,M,V,-1,CR>(X,xb,tw,t,xm);
-    // twiddles loaded before the first use (r = 0 reads 1), as forward
-    cplx<T> w[P2][V];
+    for(int k=0; k < V; ++k) X[k]=ok ? Fr[(int64_t) (tf+TPS*k)*SF] : mk((T) 0,(T) 0);
+    fftr_blkx<T,M,V,-1,CR,(sizeof(T) == 8 || P2 == 2)>(X,xb,tw,t,xm);
+    // half of the twiddles at a time (all at once costs registers and spills)
+    constexpr int KH=V/2;
 #pragma unroll
-    for(int k=0; k < V; ++k) {
-      const int j0=(t+TPS*k-k0) & (M-1);
+    for(int kk=0; kk < V; kk += KH) {
+      cplx<T> w[P2][KH];
+      col_residue<T,M,P2>(w,zt,tf,kk,k0,r,N);
 #pragma unroll
-      for(int i=0; i < P2; ++i) w[i][k]=zN[wrapN((j0+M*i+k0)*r,N)];
-    }
+      for(int k=0; k < KH; ++k)
 #pragma unroll
-    for(int k=0; k < V; ++k) {
-#pragma unroll
-      for(int i=0; i < P2; ++i) acc[i][k]=acc[i][k]+mulc(X[k],w[i][k]);
+        for(int i=0; i < P2; ++i) acc[i][kk+k]=acc[i][kk+k]+mulc(X[kk+k],w[i][k]);
     }
   }
   if(ok) {
+    const int tf=fresh(t);
 #pragma unroll
     for(int k=0; k < V; ++k) {
-      const int j0=(t+TPS*k-k0) & (M-1);
+      const int j0=(tf+TPS*k-k0) & (M-1);
 #pragma unroll
       for(int i=0; i < P2; ++i) {
         const int j=j0+M*i;
@@ -830,9 +880,9 @@ struct RealKept {
 // kept (r, s); f real with element stride S and column stride ics (real
 // words), F complex with plane stride SF and column stride ocs.
 template<typename T, int M, int P2>
-__global__ void __launch_bounds__(512)
-colfwd_real_kernel(DimArgs d, const T *f, int64_t S, int64_t C, int64_t bsi,
-                   cplx<T> *F, int64_t SF, int64_t bso, int64_t ics, int64_t ocs)
+__global__ void __launch_bounds__(512,P2 == 1 ? 4 : 2)
+colfwd_real_kernel(DimArgs d, ColArrays io, int64_t S, int64_t C, int64_t bsi,
+                   int64_t SF, int64_t bso, int64_t ics, int64_t ocs)
 {
   typedef ColReg<T,M> CR;
   constexpr int V=CR::V, TPS=CR::TPS, TC=CR::TC;
@@ -848,8 +898,9 @@ colfwd_real_kernel(DimArgs d, const T *f, int64_t S, int64_t C, int64_t bsi,
   const int xm=CR::xm(c);
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
-  const T *fb=f+(int64_t) blockIdx.y*bsi+(c0+c)*ics;
-  cplx<T> *Fb=F+(int64_t) blockIdx.y*bso+(c0+c)*ocs;
+  const ColBlock bk=col_block(io);
+  const T *fb=(const T *) bk.in+(int64_t) blockIdx.y*bsi+(c0+c)*ics;
+  cplx<T> *Fb=(cplx<T> *) bk.out+(int64_t) blockIdx.y*bso+(c0+c)*ocs;
   const int N=(int) d.N, L=(int) d.L, q=(int) d.q;
   T raw[P2][V];
 #pragma unroll
@@ -860,7 +911,7 @@ colfwd_real_kernel(DimArgs d, const T *f, int64_t S, int64_t C, int64_t bsi,
       raw[i][k]=ok && j < L ? fb[(int64_t) j*S] : (T) 0;
     }
   const int R=(int) RealKept::residues(q);
-  for(int r=0; r < R; ++r) {
+  for(int r=bk.part; r < R; r += bk.parts) {
     // twiddles loaded before the first use (r = 0 reads 1)
     cplx<T> w[P2][V];
 #pragma unroll
@@ -875,7 +926,9 @@ colfwd_real_kernel(DimArgs d, const T *f, int64_t S, int64_t C, int64_t bsi,
       for(int i=1; i < P2; ++i) a=a+raw[i][k]*w[i][k];
       X[k]=a;
     }
-    fftr_blkx<T,M,V,1,CR>(X,xb,tw,t,xm);
+    // fewer registers are live than in the complex columns: on short columns
+    // the positions stay in them (256^3 FP64 124 us with fresh ones)
+    fftr_blkx<T,M,V,1,CR,(M >= 512)>(X,xb,tw,t,xm);
     if(ok) {
       const int cnt=(int) RealKept::count(M,q,r);
       cplx<T> *Fr=Fb+RealKept::base(M,r)*SF;
@@ -933,7 +986,7 @@ colbwd_real_kernel(DimArgs d, const cplx<T> *F, int64_t SF, int64_t bsi,
       }
       X[k]=v;
     }
-    fftr_blkx<T,M,V,-1,CR>(X,xb,tw,t,xm);
+    fftr_blkx<T,M,V,-1,CR,(M >= 512)>(X,xb,tw,t,xm);
     const T cr=self ? (T) 1 : (T) 2;
     // twiddles loaded before their use (r = 0 reads 1), half of the values
     // at a time (all at once costs a wave per SIMD)
