@@ -48,6 +48,8 @@ SIGNATURES = {
     "fftwpp_amd_symmetrize_x": (I, [Z, Z, Z, P, Z, P]),
     "fftwpp_amd_symmetrize_xy": (I, [Z, Z, Z, Z, Z, P, Z, Z, P]),
     "fftwpp_amd_hermitian_plane": (I, [I, I, Z, Z, Z, Z, P, Z, Z, P]),
+    "fftwpp_amd_internal_hplane_copies": (I, [I, I, I, Z, Z, Z, Z, ctypes.POINTER(P),
+                                              ctypes.POINTER(P), Z, Z, Z, P]),
     "fftwpp_amd_malloc": (I, [ctypes.POINTER(P), Z]),
     "fftwpp_amd_free": (I, [P]),
     "fftwpp_amd_memcpy": (I, [P, P, Z, P]),

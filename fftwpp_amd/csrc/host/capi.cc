@@ -159,6 +159,15 @@ struct HybridConvolutionHermitian3 {
 static thread_local char capi_error[512];
 
 extern "C" void fftwpp_amd_internal_set_error(const char *msg);
+// the plane operation on several arrays, or on copies of them, in one launch
+extern "C" int fftwpp_amd_internal_hplanes(int dtype, int op, int n, size_t Hx, size_t Hy,
+                                           size_t x0, size_t y0, void *const *f, size_t Sx,
+                                           size_t Sy, void *stream);
+extern "C" int fftwpp_amd_internal_hplane_copies(int dtype, int n, int ops1, size_t Hx,
+                                                 size_t Hy, size_t x0, size_t y0,
+                                                 const void *const *in, void *const *out,
+                                                 size_t Sx, size_t Sy, size_t words,
+                                                 void *stream);
 
 static void report_error(const char *where, const std::exception &e)
 {
@@ -468,26 +477,20 @@ static int hermitian_adjoint(fftwpp_amd_conv *c, const void *w, const void *a,
       int rc=fftwpp_amd_malloc(&q,bytes);
       if(rc) return rc;
     }
-  void *wh=c->adj[0], *sa=c->adj[1], *sb=c->adj[2];
   const int dt=c->dtype;
-  auto plane=[&](int op, void *f) {
-    return fftwpp_amd_hermitian_plane(dt,op,p[0],p[1],p[2],p[3],f,p[4],p[5],stream);
-  };
-  int rc=fftwpp_amd_memcpy(wh,w,bytes,stream);
-  if(!rc) rc=plane(1,wh);
+  // w_H, and S b and S a for the gradients asked for
+  const void *in[3]={w,grad_a ? b : a,a};
+  const int n=grad_a && grad_b ? 3 : (grad_a || grad_b ? 2 : 1);
+  void *grad[2]={grad_a ? grad_a : grad_b,grad_b};
+  void *const *t=c->adj;
+  int rc=fftwpp_amd_internal_hplane_copies(dt,n,1,p[0],p[1],p[2],p[3],in,t,p[4],p[5],c->words,
+                                           stream);
+  if(rc || n == 1) return rc;
   try {
-    if(!rc && grad_a) {
-      rc=fftwpp_amd_memcpy(sb,b,bytes,stream);
-      if(!rc) rc=plane(0,sb);
-      if(!rc) c->exec(grad_a,wh,sb,stream,-1);
-      if(!rc) rc=plane(2,grad_a);
-    }
-    if(!rc && grad_b) {
-      rc=fftwpp_amd_memcpy(sa,a,bytes,stream);
-      if(!rc) rc=plane(0,sa);
-      if(!rc) c->exec(grad_b,wh,sa,stream,-1);
-      if(!rc) rc=plane(2,grad_b);
-    }
+    const void *g[2]={t[1],t[2]};
+    if(!(n == 3 && c->h2 && c->h2->convolve2->execShared(grad,t[0],g,true,dt,stream)))
+      for(int k=0; k+1 < n; ++k) c->exec(grad[k],t[0],t[k+1],stream,-1);
+    rc=fftwpp_amd_internal_hplanes(dt,2,n-1,p[0],p[1],p[2],p[3],grad,p[4],p[5],stream);
   } catch(const std::exception &e) {
     return conv_status("fftwpp_amd_conv_adjoint",e);
   }
@@ -725,18 +728,19 @@ int fftwpp_amd_conv_adjoint(fftwpp_amd_conv *c, const void *w, const void *a,
       return FFTWPP_AMD_ERR_ARG;
     }
   if(c->hermitian == 1) return hermitian_adjoint(c,w,a,b,grad_a,grad_b,stream,bytes);
+  if((grad_a && !b) || (grad_b && !a)) return FFTWPP_AMD_ERR_ARG;
   try {
-    if(grad_a) {
-      if(!b) return FFTWPP_AMD_ERR_ARG;
-      int rc=fftwpp_amd_memcpy(grad_a,w,bytes,stream);
+    // both products share the transform of w where the plan allows it
+    void *const grad[2]={grad_a,grad_b};
+    const void *const g[2]={b,a};
+    if(grad_a && grad_b && c->c2 &&
+       c->c2->convolve2->execShared(grad,w,g,true,c->dtype,stream,FFTWPP_AMD_MULT_CORRELATION))
+      return FFTWPP_AMD_OK;
+    for(int k=0; k < 2; ++k) {
+      if(!grad[k]) continue;
+      int rc=fftwpp_amd_memcpy(grad[k],w,bytes,stream);
       if(rc) return rc;
-      c->exec(grad_a,grad_a,b,stream,FFTWPP_AMD_MULT_CORRELATION);
-    }
-    if(grad_b) {
-      if(!a) return FFTWPP_AMD_ERR_ARG;
-      int rc=fftwpp_amd_memcpy(grad_b,w,bytes,stream);
-      if(rc) return rc;
-      c->exec(grad_b,grad_b,a,stream,FFTWPP_AMD_MULT_CORRELATION);
+      c->exec(grad[k],grad[k],g[k],stream,FFTWPP_AMD_MULT_CORRELATION);
     }
   } catch(const std::exception &e) {
     return conv_status("fftwpp_amd_conv_adjoint",e);

@@ -1345,6 +1345,28 @@ void Convolution2::execComplex(void *out, const void *f0, const void *f1, bool n
   }
 }
 
+bool Convolution2::execShared(void *const out[2], const void *w, const void *const g[2],
+                              bool normalize, int dtype, void *stream, int mult)
+{
+  const int code=mult >= 0 ? mult : multCode;
+  requireBinary(A,B,code);
+  if(fftx->realInput() || memoryLimit || timeline || rowHook || ffty->C != 1 ||
+     !rowsSupported(ffty,dtype))
+    return false;
+  const size_t q=fftx->q, rows=q*fftx->m, bytes=rows*ly*eltsize(dtype);
+  const void *in[3]={w,g[0],g[1]};
+  void *F[3]={work.get(0,bytes),work.get(1,bytes),work.get(11,bytes)};
+  check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,0,3,in,Sx,ly,1,0,F,ly,0,0,q,stream),
+        "x forward");
+  // every row is read whole before it is written: the product may replace the
+  // second factor
+  for(int k=1; k < 3; ++k)
+    fusedRows(ffty,work,2,dtype,code,F[0],F[k],rows,ly,F[k],ly,1.0,stream,"y rows");
+  check(fftwpp_amd_internal_backward_arrays(fftx->dev,dtype,2,F+1,ly,0,out,Sx,ly,1,0,0,q,0,
+                                            normalize ? scale : 1.0,stream),"x backward");
+  return true;
+}
+
 // Work bytes of an execution with Dx x residues per pass (0: all): the two
 // x-transformed arrays, the unfused row stage's two expanded arrays when it
 // runs, and with residue blocks a copy of the input an in-place call

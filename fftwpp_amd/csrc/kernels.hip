@@ -646,12 +646,13 @@ __global__ void symxy3_kernel(int64_t Hx, int64_t Hy, int64_t Hz, int64_t x0,
 // ------------------------------------------------------------------------
 template<typename T>
 __global__ void hplane_kernel(int op, int64_t Hx, int64_t Hy, int64_t x0,
-                              int64_t y0, cplx<T> *f, int64_t Sx, int64_t Sy)
+                              int64_t y0, ColArrays io, int64_t Sx, int64_t Sy)
 {
   int64_t t=(int64_t) blockIdx.x*blockDim.x+threadIdx.x;
   if(t >= (2*Hx-1)*Hy) return;
   const int64_t i=t/Hy-(Hx-1), j=t % Hy;
   if(j == 0 && i < 0) return;
+  cplx<T> *f=(cplx<T> *) (blockIdx.y == 0 ? io.out[0] : (blockIdx.y == 1 ? io.out[1] : io.out[2]));
   cplx<T> *u=f+(x0+i)*Sx+(y0+j)*Sy;
   if(i == 0 && j == 0) {
     const cplx<T> v=*u;
@@ -667,6 +668,37 @@ __global__ void hplane_kernel(int op, int64_t Hx, int64_t Hy, int64_t x0,
     *u=a+conjg(b);
     *l=b+conjg(a);
   } else *l=mk((T) 0,(T) 0);
+}
+
+// Copies of whole arrays of `words` words (element (x, y) of the plane at x Sx
+// + y Sy, Sx a multiple of Sy) with plane operation 0 (symmetrize) applied to
+// array z of the grid, or operation 1 where bit z of ops1 is set: one pass
+// where a copy and a launch on the plane took two.
+// I: the type of the index arithmetic (32 bits where the words allow it: the
+// divisions were most of the pass in 64).
+template<typename T, typename I>
+__global__ void __launch_bounds__(256)
+hplane_copy_kernel(ColArrays io, int ops1, I Hx, I Hy, I x0, I y0, I Sx, I Sy, I words)
+{
+  const ColBlock bk=col_block(io);
+  const cplx<T> *in=(const cplx<T> *) bk.in;
+  cplx<T> *out=(cplx<T> *) bk.out;
+  const bool add=(ops1 >> blockIdx.z) & 1;
+  for(I e=(I) blockIdx.x*256+threadIdx.x; e < words; e += (I) gridDim.x*256) {
+    cplx<T> v=in[e];
+    if(e % Sy == 0) {
+      const I x=e/Sx, i=x-x0, j=(e-x*Sx)/Sy-y0;
+      if(i > -Hx && i < Hx && j > -Hy && j < Hy) {
+        const bool upper=j > 0 || (j == 0 && i > 0);
+        if(add || !upper) {
+          const cplx<T> m=conjg(in[(x0-i)*Sx+(y0-j)*Sy]);
+          if(add) v=v+m;
+          else v=i == 0 && j == 0 ? mk(v.x,(T) 0) : m;
+        }
+      }
+    }
+    out[e]=v;
+  }
 }
 
 // Reference-layout residue blocks (fftBase::forward/backward of the C++
@@ -2197,25 +2229,73 @@ int fftwpp_amd_symmetrize_xy(size_t Hx, size_t Hy, size_t Hz, size_t x0,
   return rc;
 }
 
+// fftwpp_amd_hermitian_plane on n <= 3 arrays of one layout in one launch.
+int fftwpp_amd_internal_hplanes(int dtype, int op, int n, size_t Hx, size_t Hy, size_t x0,
+                                size_t y0, void *const *f, size_t Sx, size_t Sy, void *stream)
+{
+  if(!f || n < 1 || n > MAXARRAYS || Hx == 0 || Hy == 0) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
+  if(op < 0 || op > 2) return fail(FFTWPP_AMD_ERR_ARG,"unknown plane operation");
+  if(x0+1 < Hx || y0+1 < Hy) return fail(FFTWPP_AMD_ERR_ARG,"origin too small");
+  ColArrays io={};
+  io.n=n;
+  for(int a=0; a < n; ++a) {
+    if(!f[a]) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
+    io.out[a]=f[a];
+  }
+  hipStream_t st=(hipStream_t) stream;
+  const dim3 grid((unsigned) (((2*Hx-1)*Hy+255)/256),(unsigned) n);
+  if(dtype == FFTWPP_AMD_F32)
+    hipLaunchKernelGGL(hplane_kernel<float>,grid,dim3(256),0,st,op,(int64_t) Hx,
+                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,io,(int64_t) Sx,(int64_t) Sy);
+  else
+    hipLaunchKernelGGL(hplane_kernel<double>,grid,dim3(256),0,st,op,(int64_t) Hx,
+                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,io,(int64_t) Sx,(int64_t) Sy);
+  return launch_check("hplane_kernel");
+}
+
 int fftwpp_amd_hermitian_plane(int dtype, int op, size_t Hx, size_t Hy,
                                size_t x0, size_t y0, void *f, size_t Sx,
                                size_t Sy, void *stream)
 {
-  if(!f || Hx == 0 || Hy == 0) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
-  if(op < 0 || op > 2) return fail(FFTWPP_AMD_ERR_ARG,"unknown plane operation");
+  return fftwpp_amd_internal_hplanes(dtype,op,1,Hx,Hy,x0,y0,&f,Sx,Sy,stream);
+}
+
+// out[a] = in[a] (arrays of `words` words, none of them the same) with plane
+// operation 0 applied, or operation 1 where bit a of ops1 is set, for n <= 3
+// arrays in one launch.
+int fftwpp_amd_internal_hplane_copies(int dtype, int n, int ops1, size_t Hx, size_t Hy,
+                                      size_t x0, size_t y0, const void *const *in,
+                                      void *const *out, size_t Sx, size_t Sy, size_t words,
+                                      void *stream)
+{
+  if(!in || !out || n < 1 || n > MAXARRAYS || Hx == 0 || Hy == 0 || Sx == 0 || Sy == 0 || words == 0)
+    return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
   if(x0+1 < Hx || y0+1 < Hy) return fail(FFTWPP_AMD_ERR_ARG,"origin too small");
+  if(Sx % Sy || (x0+Hx-1)*Sx+(y0+Hy-1)*Sy >= words) return fail(FFTWPP_AMD_ERR_ARG,"bad plane strides");
+  ColArrays io={};
+  io.n=n;
+  for(int a=0; a < n; ++a) {
+    if(!in[a] || !out[a] || in[a] == out[a]) return fail(FFTWPP_AMD_ERR_ARG,"bad argument");
+    io.in[a]=in[a];
+    io.out[a]=out[a];
+  }
   hipStream_t st=(hipStream_t) stream;
-  const size_t n=(2*Hx-1)*Hy;
-  const dim3 grid((unsigned) ((n+255)/256));
-  if(dtype == FFTWPP_AMD_F32)
-    hipLaunchKernelGGL(hplane_kernel<float>,grid,dim3(256),0,st,op,(int64_t) Hx,
-                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,(cplx<float> *) f,
-                       (int64_t) Sx,(int64_t) Sy);
-  else
-    hipLaunchKernelGGL(hplane_kernel<double>,grid,dim3(256),0,st,op,(int64_t) Hx,
-                       (int64_t) Hy,(int64_t) x0,(int64_t) y0,(cplx<double> *) f,
-                       (int64_t) Sx,(int64_t) Sy);
-  return launch_check("hplane_kernel");
+  const dim3 grid((unsigned) std::min<size_t>((words+255)/256,8192),1,(unsigned) n);
+  auto launch=[&](auto kernel, auto zero) {
+    typedef decltype(zero) I;
+    hipLaunchKernelGGL(kernel,grid,dim3(256),0,st,io,ops1,(I) Hx,(I) Hy,(I) x0,(I) y0,(I) Sx,
+                       (I) Sy,(I) words);
+  };
+  // 32 bits: indices up to words plus one step of the grid
+  const bool small=words < ((size_t) 1 << 31)-8192*256;
+  if(dtype == FFTWPP_AMD_F32) {
+    if(small) launch(hplane_copy_kernel<float,int>,(int) 0);
+    else launch(hplane_copy_kernel<float,int64_t>,(int64_t) 0);
+  } else {
+    if(small) launch(hplane_copy_kernel<double,int>,(int) 0);
+    else launch(hplane_copy_kernel<double,int64_t>,(int64_t) 0);
+  }
+  return launch_check("hplane_copy_kernel");
 }
 
 // ---- memory and stream plumbing for host code that includes no HIP header

@@ -9,6 +9,7 @@ arithmetic runs in libfftwpp_amd.so.
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from ._lib import F32, F64, check, lib, sizes
 
@@ -31,6 +32,15 @@ def _dtype_code(dtype, kind="complex"):
 
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def _clone_is_bytes(t):
+    """Whether t.clone() does nothing but copy the bytes of the contiguous t,
+    so that a kernel that reads t may take its place: not where autograd
+    records it, a tangent goes with it or a lazy conjugation or sign is
+    resolved in it."""
+    return not (t.is_conj() or t.is_neg() or (t.requires_grad and torch.is_grad_enabled()) or
+                getattr(forward_ad, "_current_level", 0) >= 0)
 
 
 class DeviceConvolution:
@@ -121,6 +131,8 @@ class DeviceConvolution:
         return out
 
     def __call__(self, a, b):
+        if a.is_contiguous() and _clone_is_bytes(a):
+            return self.convolve_out(torch.empty_like(a), a, b)
         out = a.clone()
         return self.convolve_(out, b)
 
@@ -156,11 +168,26 @@ class DeviceConvolution:
         """Copy of t with the self-conjugate plane made Hermitian
         (HermitianSymmetrize{,X,XY}, convolve.h:1168-1256)."""
         self._check(t)
+        if _clone_is_bytes(t):
+            return self._symmetrized_copies(t)[0]
         out = t.clone()
         Hx, Hy, x0, y0, Sx, Sy = self._plane()
         check(lib().fftwpp_amd_hermitian_plane(_dtype_code(self.dtype), 0, Hx, Hy, x0, y0,
                                                out.data_ptr(), Sx, Sy, _stream()))
         return out
+
+    def _symmetrized_copies(self, *ts):
+        """symmetrized() of up to three tensors in one launch."""
+        plane = self._plane()
+        ts = [t.resolve_conj().resolve_neg() for t in ts]
+        outs = [torch.empty_like(t) for t in ts]
+        n = len(ts)
+        check(lib().fftwpp_amd_internal_hplane_copies(
+            _dtype_code(self.dtype), n, 0, *plane[:4],
+            (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts]),
+            (ctypes.c_void_p * n)(*[t.data_ptr() for t in outs]), *plane[4:], ts[0].numel(),
+            _stream()))
+        return outs
 
     def adjoint(self, w, a, b, need_a=True, need_b=True):
         """Cotangents of (a, b) for output cotangent w (PyTorch convention
@@ -187,7 +214,10 @@ class _ConvolveFn(torch.autograd.Function):
         ctx.plan = plan
         ctx.save_for_backward(a, b)
         if plan.kind == "hermitian":
-            return plan(plan.symmetrized(a), plan.symmetrized(b))
+            plan._check(a)
+            plan._check(b)
+            sa, sb = plan._symmetrized_copies(a, b)
+            return plan.convolve_(sa, sb)
         return plan(a, b)
 
     @staticmethod

@@ -453,6 +453,12 @@ public:
   // multiplier (the adjoint uses multcorrelation).
   void execDevice(void *out, const void *f0, const void *f1, bool normalize,
                   int dtype, void *stream, int mult=-1);
+  // out[k] <- w (*) g[k], k = 0, 1, with one x transform of w for both (the
+  // two products of the adjoint); the inputs are read before the outputs are
+  // written.  False, and nothing done, where the plan runs otherwise (real
+  // data, a memory limit, a timeline or row hook, rows without a fused kernel).
+  bool execShared(void *const out[2], const void *w, const void *const g[2], bool normalize,
+                  int dtype, void *stream, int mult=-1);
   size_t arraySize() const;
 
   Timeline *timeline=NULL;  // when set, every launch is timed

@@ -101,3 +101,21 @@ def test_call_keeps_what_it_accepted(gpu):
     assert torch.equal(plan(a, b), want)
     t = a.contiguous().requires_grad_(True)
     assert torch.equal(plan(t, b).detach(), want)
+
+
+@pytest.mark.parametrize("kind", ["complex", "hermitian"])
+def test_call_resolves_lazy_conjugates(gpu, kind):
+    """A first factor that is a lazy conjugate is read as its values (both
+    factors where the plan symmetrizes copies of them)."""
+    import torch
+    from fftwpp_amd.torch_conv import DeviceConvolution, convolve
+    plan = DeviceConvolution((7, 5), kind=kind)
+    a, b = (torch.randn(7, 5, dtype=torch.complex128, device=gpu) for _ in range(2))
+    want = plan(a.conj().resolve_conj(), b)
+    assert torch.equal(plan(a.conj(), b), want)
+    if kind == "hermitian":
+        assert torch.equal(plan.symmetrized(a.conj()), plan.symmetrized(a.conj().resolve_conj()))
+        ac, bc = a.conj().resolve_conj(), b.conj().resolve_conj()
+        assert torch.equal(convolve(a.conj(), b.conj(), plan), convolve(ac, bc, plan))
+    else:
+        assert torch.equal(convolve(a.conj(), b, plan), want)
