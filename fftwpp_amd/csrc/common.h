@@ -211,7 +211,12 @@ __device__ __forceinline__ cplx<T> table_word(const cplx<T> *p)
 // Buffer access: a complex word at byte offset off (per lane) + soff
 // (uniform) of a raw buffer; one offset register serves every load of a
 // thread whose words differ by uniform strides.
-// Store of one complex word at byte offset off + soff of the buffer r.
+// Store of one complex word at byte offset off + soff of the buffer r.  The
+// 16-byte store takes soff in its vector offset: with a scalar offset register
+// the compiler lets the next vector operation overwrite the stored registers,
+// and lanes 12..15 of each 16 were then seen to store the new values (rows of
+// 256 points differed from run to run).  Without one it keeps the two wait
+// states; 8-byte stores read their data at once.
 template<typename T>
 __device__ __forceinline__ void st_buf(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned soff,
                                        cplx<T> v);
@@ -222,7 +227,7 @@ __device__ __forceinline__ void st_buf<double>(__amdgpu_buffer_rsrc_t r, unsigne
   typedef double d2 __attribute__((ext_vector_type(2)));
   typedef unsigned u4 __attribute__((ext_vector_type(4)));
   d2 w; w.x=v.x; w.y=v.y;
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4,w),r,off,soff,0);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4,w),r,off+soff,0,0);
 }
 template<>
 __device__ __forceinline__ void st_buf<float>(__amdgpu_buffer_rsrc_t r, unsigned off,

@@ -111,7 +111,7 @@ __device__ __forceinline__ void fft256s(cplx<T> *v, T *row, int j, int h,
   lanes_sync<WAVE>();
 #pragma unroll
   for(int t=1; t < 16; ++t) {
-    cplx<T> w=(tw16+16*t)[j];
+    cplx<T> w=table_word(tw16+16*t+j);
     v[t]=S > 0 ? v[t]*w : mulc(v[t],w);
   }
   dft16<T,S>(v);
@@ -144,7 +144,7 @@ __device__ __forceinline__ void fft256s_pair(cplx<T> *v, cplx<T> *u, T *row, int
   }
 #pragma unroll
   for(int t=1; t < 16; ++t) {
-    const cplx<T> w=(tw16+16*t)[j];
+    const cplx<T> w=table_word(tw16+16*t+j);
     v[t]=S > 0 ? v[t]*w : mulc(v[t],w);
     u[t]=S > 0 ? u[t]*w : mulc(u[t],w);
   }

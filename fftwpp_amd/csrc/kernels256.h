@@ -79,7 +79,7 @@ __device__ __forceinline__ void colfwd_body(const cplx<T> *fb, cplx<T> *Fb,
     cplx<T> v[16];
 #pragma unroll
     for(int k=0; k < 16; ++k) {
-      v[k]=r == 0 ? x0[k] : x0[k]*(rt+16*k)[j];
+      v[k]=r == 0 ? x0[k] : x0[k]*table_word(rt+16*k+j);
     }
     fft256s<T,1,0>(v,row,j,h,tw16);
     cplx<T> *Fr=Fb+rr*256*SF;
@@ -116,7 +116,7 @@ __device__ __forceinline__ void colbwd_body(const cplx<T> *Fb, cplx<T> *fb,
     fft256s<T,-1,0>(v,row,j,h,tw16);
 #pragma unroll
     for(int k=0; k < 16; ++k)
-      acc[k]=acc[k]+(r == 0 ? v[k] : mulc(v[k],(rt+16*k)[j]));
+      acc[k]=acc[k]+(r == 0 ? v[k] : mulc(v[k],table_word(rt+16*k+j)));
   }
   if(ok) {
 #pragma unroll
@@ -242,7 +242,7 @@ rowconv256_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
         y=in ? (gr+16*k)[lin] : zero<T>();
       }
       if(r != 0) {
-        cplx<T> w=(rt+16*k)[j];
+        cplx<T> w=table_word(rt+16*k+j);
         x=x*w;
         y=y*w;
       }
@@ -259,7 +259,7 @@ rowconv256_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
     fft256s<T,-1,1>(a,row,j,0,tw16);
 #pragma unroll
     for(int k=0; k < 16; ++k)
-      acc[k]=acc[k]+(r == 0 ? a[k] : mulc(a[k],(rt+16*k)[j]));
+      acc[k]=acc[k]+(r == 0 ? a[k] : mulc(a[k],table_word(rt+16*k+j)));
   }
   if(ok) {
 #pragma unroll
@@ -268,21 +268,23 @@ rowconv256_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
   }
 }
 
-// Sum of a value over the two 16-lane groups of each 32-lane half of the
-// wave (lanes l and l ^ 16): v_permlane16_swap exchanges the odd 16-lane
-// rows of its first operand with the even rows of its second, so with both
-// operands v the two results hold v of the group and v of its partner.
-__device__ __forceinline__ float pair16_sum(float v)
+// Reduce-scatter over the two 16-lane groups of each 32-lane half of the wave
+// (groups 0 and 1): lanes of group 0 get the sum over the groups of x, lanes
+// of group 1 that of y.  v_permlane16_swap exchanges the odd 16-lane rows of
+// its first operand with the even rows of its second, so its results are
+// (x of group 0, y of group 0) and (x of group 1, y of group 1) on the lanes of
+// (group 0, group 1).
+__device__ __forceinline__ float pair16_scatter(float x, float y)
 {
-  auto s=__builtin_amdgcn_permlane16_swap(__float_as_uint(v),__float_as_uint(v),
-                                          false,false);
+  auto s=__builtin_amdgcn_permlane16_swap(__float_as_uint(x),__float_as_uint(y),false,false);
   return __uint_as_float(s[0])+__uint_as_float(s[1]);
 }
-__device__ __forceinline__ double pair16_sum(double v)
+__device__ __forceinline__ double pair16_scatter(double x, double y)
 {
-  const unsigned long long u=(unsigned long long) __double_as_longlong(v);
-  auto lo=__builtin_amdgcn_permlane16_swap((unsigned) u,(unsigned) u,false,false);
-  auto hi=__builtin_amdgcn_permlane16_swap((unsigned) (u >> 32),(unsigned) (u >> 32),
+  const unsigned long long u=(unsigned long long) __double_as_longlong(x);
+  const unsigned long long v=(unsigned long long) __double_as_longlong(y);
+  auto lo=__builtin_amdgcn_permlane16_swap((unsigned) u,(unsigned) v,false,false);
+  auto hi=__builtin_amdgcn_permlane16_swap((unsigned) (u >> 32),(unsigned) (v >> 32),
                                            false,false);
   const double a=__longlong_as_double((long long) (((unsigned long long) hi[0] << 32) | lo[0]));
   const double b=__longlong_as_double((long long) (((unsigned long long) hi[1] << 32) | lo[1]));
@@ -292,14 +294,22 @@ __device__ __forceinline__ double pair16_sum(double v)
 // Rows with q = 2 (N = 512): a wave holds 2 rows x 2 residues x 16 lanes,
 // lane = j + 16 (2 i + r) for row i of the wave and residue r.  The two
 // residue groups of a row load the same elements in the same instruction, so
-// f and g are read from memory once; each group transforms its residue and
-// the contributions are summed across the group pair in registers.  Group r
-// then stores the outputs j + 16 k with k in [8 r, 8 r + 8).  The grid is
-// persistent: each block fills its twiddle tables once and its waves, which
-// exchange only within themselves, loop over row pairs independently.
+// f and g are read from memory once; each group transforms its residue, and a
+// reduce-scatter across the group pair leaves lane j of group r with the
+// outputs j + 16 k, k in [8 r, 8 r + 8).  The grid is persistent: each block
+// fills its twiddle tables once and its waves, which exchange only within
+// themselves, loop over row pairs independently.  Rows are read and written
+// through buffers over the pair: one offset per lane, past the end (read as 0,
+// not stored) for padding and for a missing second row.
+//
+// Bound by the vector unit in FP64 (the loop issues 1765 -> 1591 vector
+// instructions per row pair, at four cycles each on one of 1024 SIMDs): the
+// branches around every load and store and the sum of all sixteen outputs in
+// both groups were an eighth of them.  262144 rows of 256: FP64 778 -> 705 us,
+// FP32 392 -> 376 us.
 // Dynamic LDS: row256_lds(4 WPB, 2).
 template<typename T, class Op, int WPB>
-__global__ void __launch_bounds__(64*WPB,2)
+__global__ void __launch_bounds__(64*WPB,sizeof(T) == 4 ? 4 : 2)
 rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
                    int64_t rs, cplx<T> *out, int64_t os, int L, T scale,
                    const cplx<T> *zN, Op op)
@@ -311,28 +321,42 @@ rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
   fill_rtab(rtab,zN,0,2,threadIdx.x,64*WPB);
   fill_tw16(tw16,zN,2,threadIdx.x,64*WPB);
   __syncthreads();
+  constexpr unsigned E=sizeof(cplx<T>), END=0x80000000u;
   const int j=threadIdx.x & 15;
   const int grp=threadIdx.x >> 4;          // 4 groups per wave
-  const int r=grp & 1;
-  const int wave=threadIdx.x >> 6;
+  const int r=grp & 1, i=(grp & 3) >> 1;   // residue and row of the wave
+  const int wave=__builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
   const cplx<T> *rt=rtab+256*r;
   constexpr int RS=17;                     // row stride of the exchange areas
   T *xrow=lds+grp*16*RS;
   const int64_t pairs=(rows+1)/2;
   for(int64_t pr=(int64_t) blockIdx.x*WPB+wave; pr < pairs; pr += (int64_t) gridDim.x*WPB) {
-    const int64_t row=2*pr+((grp & 3) >> 1);
+    const int64_t row=2*pr+i;
     const bool ok=row < rows;
-    const cplx<T> *fr=f+(ok ? row : 0)*rs;
-    const cplx<T> *gr=g+(ok ? row : 0)*rs;
+    const size_t two=2*pr+1 < rows;        // the pair's second row exists
+    const __amdgpu_buffer_rsrc_t rf=buf_rsrc(f+2*pr*rs,two*rs+L), rg=buf_rsrc(g+2*pr*rs,two*rs+L);
+    const unsigned in=ok ? (unsigned) (i*(int) rs+j)*E : END;
     cplx<T> a[16], b[16];
+    if(L == 256) {
+#pragma unroll
+      for(int k=0; k < 16; ++k) {
+        a[k]=ld_buf<T>(rf,in,16*k*E);
+        b[k]=ld_buf<T>(rg,in,16*k*E);
+      }
+    } else {
+      const int jf=fresh(j);
+#pragma unroll
+      for(int k=0; k < 16; ++k) {
+        const unsigned o=jf+16*k < L ? in : END;
+        a[k]=ld_buf<T>(rf,o,16*k*E);
+        b[k]=ld_buf<T>(rg,o,16*k*E);
+      }
+    }
 #pragma unroll
     for(int k=0; k < 16; ++k) {
-      bool in=ok && j+16*k < L;
-      cplx<T> x=in ? (fr+16*k)[j] : zero<T>();
-      cplx<T> y=in ? (gr+16*k)[j] : zero<T>();
-      cplx<T> w=(rt+16*k)[j];                 // w_512^{r (j + 16 k)}
-      a[k]=x*w;
-      b[k]=y*w;
+      const cplx<T> w=table_word(rt+16*k+j); // w_512^{r (j + 16 k)}
+      a[k]=a[k]*w;
+      b[k]=b[k]*w;
     }
     fft256s_pair<T,1,1,RS>(a,b,xrow,j,0,tw16);
     {
@@ -342,15 +366,14 @@ rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
     }
     fft256s<T,-1,1,RS>(a,xrow,j,0,tw16);
 #pragma unroll
-    for(int k=0; k < 16; ++k) {
-      cplx<T> y=mulc(a[k],(rt+16*k)[j]);
-      a[k]=mk(pair16_sum(y.x),pair16_sum(y.y));
-    }
-    if(ok) {
-      cplx<T> *orow=out+row*os;
+    for(int k=0; k < 16; ++k) a[k]=mulc(a[k],table_word(rt+16*k+j));
+    const __amdgpu_buffer_rsrc_t ro=buf_rsrc(out+2*pr*os,two*os+L);
+    const int j0=fresh(j)+128*r;           // this group's first output
+    const unsigned to=ok ? (unsigned) (i*(int) os+j0)*E : END;
 #pragma unroll
-      for(int k=0; k < 16; ++k)
-        if((k >> 3) == r && j+16*k < L) (orow+16*k)[j]=scale*a[k];
+    for(int k=0; k < 8; ++k) {
+      const cplx<T> v=mk(pair16_scatter(a[k].x,a[k+8].x),pair16_scatter(a[k].y,a[k+8].y));
+      st_buf<T>(ro,j0+16*k < L ? to : END,16*k*E,scale*v);
     }
   }
 }

@@ -282,13 +282,13 @@ plane256_kernel(const cplx<T> *Xf, const cplx<T> *Xg, cplx<T> *Xh,
         }
         fft256s<T,-1,1,17>(av,xrow,jr,0,tw16);
 #pragma unroll
-        for(int kk=0; kk < 16; ++kk) {
-          const cplx<T> y=mulc(av[kk],(rt+16*kk)[jr]);
-          av[kk]=mk(pair16_sum(y.x),pair16_sum(y.y));
-        }
+        for(int kk=0; kk < 16; ++kk) av[kk]=mulc(av[kk],(rt+16*kk)[jr]);
+        // group rz gets the sums of the words jr + 128 rz + 16 kk
+        const unsigned srow=frow+(unsigned) rz*128u*EW;
 #pragma unroll
-        for(int kk=0; kk < 16; ++kk)
-          if((kk >> 3) == rz) st_buf<T>(re,frow,16u*EW*kk,av[kk]);
+        for(int kk=0; kk < 8; ++kk)
+          st_buf<T>(re,srow,16u*EW*kk,mk(pair16_scatter(av[kk].x,av[kk+8].x),
+                                         pair16_scatter(av[kk].y,av[kk+8].y)));
       }
       plane_arrive(cB);
     }

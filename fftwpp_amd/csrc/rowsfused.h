@@ -62,6 +62,14 @@ inline size_t fused_resident(K kernel, int threads, size_t lds)
 
 inline int fused_status(hipError_t e) { return e == hipSuccess ? 0 : -(int) e; }
 
+// Rows of stride rs words of E bytes that one buffer resource covers (their
+// byte offsets and the last row's 4096 words stay below 2^31); at least 1.
+inline size_t rows_in_buffer(size_t rs, size_t E)
+{
+  const size_t span=((size_t) 1 << 31)-4096*E;
+  return rs == 0 ? ((size_t) 1 << 31) : std::max<size_t>(1,span/(rs*E));
+}
+
 template<typename T, class Op>
 inline int rows256_launch(const DimArgs &a, const void *f, const void *g, size_t rows,
                           size_t rs, void *out, size_t os, double scale, const Op &op,
@@ -69,8 +77,9 @@ inline int rows256_launch(const DimArgs &a, const void *f, const void *g, size_t
 {
   const cplx<T> *zt=(const cplx<T> *) a.zN;
   hipError_t e;
-  if(a.q == 2) {
-    // both residues of a row in one wave (each row read once); persistent grid
+  // both residues of a row in one wave (each row read once); persistent grid.
+  // A wave's two rows lie in one buffer.
+  if(a.q == 2 && rows_in_buffer(std::max(rs,os),sizeof(cplx<T>)) >= 2) {
     constexpr int WPB=4;
     const size_t need=(rows+2*WPB-1)/(2*WPB);
     const size_t lds=row256_lds<T>(4*WPB,2);
@@ -89,14 +98,6 @@ inline int rows256_launch(const DimArgs &a, const void *f, const void *g, size_t
                      (const cplx<T> *) f,(const cplx<T> *) g,(int64_t) rows,(int64_t) rs,
                      (cplx<T> *) out,(int64_t) os,(int) a.L,(T) scale,zt,(int64_t) a.q,op);
   return fused_status(hipGetLastError());
-}
-
-// Rows of stride rs words of E bytes that one buffer resource covers (their
-// byte offsets and the last row's 4096 words stay below 2^31); at least 1.
-inline size_t rows_in_buffer(size_t rs, size_t E)
-{
-  const size_t span=((size_t) 1 << 31)-4096*E;
-  return rs == 0 ? ((size_t) 1 << 31) : std::max<size_t>(1,span/(rs*E));
 }
 
 // RP residue lanes per row when rows are too few to fill the chip (under 512)

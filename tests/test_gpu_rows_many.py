@@ -58,11 +58,11 @@ def test_complex_rows(gpu, oracle, Ly, my, q, dtype):
     assert oracle.rel_l2(h, want) < TOL[dtype]
 
 
-@pytest.mark.parametrize("L,m", [(16, 16), (40, 64)])
-def test_rows_of_huge_stride(gpu, oracle, L, m):
+@pytest.mark.parametrize("L,m,rows,rs", [(16, 16, 10, 1 << 24), (40, 64, 10, 1 << 24),
+                                         (200, 256, 7, 1 << 24), (256, 256, 3, 1 << 27)])
+def test_rows_of_huge_stride(gpu, oracle, L, m, rows, rs):
     import torch
     from fftwpp_amd._lib import F64, MULT_BINARY, check, lib
-    rows, rs = 10, 1 << 24          # 256 MB from row to row
     rng = np.random.default_rng(L)
     f, g = _rnd(rng, (rows, L)), _rnd(rng, (rows, L))
     a, b = (torch.zeros((rows - 1) * rs + L, dtype=torch.complex128, device=gpu) for _ in range(2))
@@ -80,3 +80,35 @@ def test_rows_of_huge_stride(gpu, oracle, L, m):
         lib().fftwpp_amd_dim_destroy(d)
     for i in range(rows):
         assert oracle.rel_l2(h[i], oracle.direct_conv(f[i], g[i])) < 1e-12, i
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("L", [100, 128, 129, 255, 256])
+def test_rows_256_repeat(gpu, oracle, L, dtype):
+    """Rows of 256 points with two residues, an odd number of them in place:
+    every row right, and the same bits each time."""
+    import torch
+    from fftwpp_amd._lib import F32, F64, MULT_BINARY, check, lib
+    rows = 20001
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(L)
+    f, g = (torch.randn(rows, L, generator=gen, dtype=getattr(torch, dtype), device=gpu) for _ in range(2))
+    d = ctypes.c_void_p()
+    check(lib().fftwpp_amd_dim_create(ctypes.byref(d), L, 256, 2, 0))
+    try:
+        out = []
+        for _ in range(4):
+            h = f.clone()
+            torch.cuda.synchronize()
+            check(lib().fftwpp_amd_conv_rows(d, F64 if dtype == "complex128" else F32, MULT_BINARY,
+                                             h.data_ptr(), g.data_ptr(), rows, L, h.data_ptr(), L,
+                                             1.0 / 512, None))
+            torch.cuda.synchronize()
+            out.append(h)
+    finally:
+        lib().fftwpp_amd_dim_destroy(d)
+    assert all(torch.equal(out[0], o) for o in out[1:])
+    z = np.fft.ifft(np.fft.fft(f.cpu().numpy().astype(complex), 512) *
+                    np.fft.fft(g.cpu().numpy().astype(complex), 512))[:, :L]
+    err = np.linalg.norm(out[0].cpu().numpy() - z, axis=1) / np.linalg.norm(z, axis=1)
+    assert err.max() < TOL[dtype]
