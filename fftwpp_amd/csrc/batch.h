@@ -169,15 +169,16 @@ template<typename T> struct BatchV { static constexpr int V=sizeof(T) == 8 ? 8 :
 // of M words (the base advanced per block, so offsets stay below M words for
 // any L; fi must be wave-uniform); otherwise through pointers.  The forward
 // transforms of f and g run with their butterflies interleaved.
-template<typename T, int M>
+template<typename T, int M, class TW>
 __device__ __forceinline__ void batch_zm_unit(const cplx<T> *zN, const cplx<T> *fi,
                                               const cplx<T> *gi, int L, int r, int q,
-                                              const cplx<T> *tw, const cplx<T> *tq, T *xb,
+                                              const TW &tw, const cplx<T> *tq, T *xb,
                                               int t, int mult, cplx<T> *z)
 {
   constexpr int V=BatchV<T>::V;
   constexpr int TPS=RPlan<M,V>::TPS;
   constexpr bool BUF=sizeof(T) == 8 && TPS >= 64;
+  constexpr unsigned E=sizeof(cplx<T>);
   cplx<T> X[V], Y[V];
 #pragma unroll
   for(int k=0; k < V; ++k) X[k]=Y[k]=mk((T) 0,(T) 0);
@@ -189,10 +190,9 @@ __device__ __forceinline__ void batch_zm_unit(const cplx<T> *zN, const cplx<T> *
       const __amdgpu_buffer_rsrc_t rf=buf_rsrc<T>(fi+jb,(size_t) rem);
       const __amdgpu_buffer_rsrc_t rg=buf_rsrc<T>(gi+jb,(size_t) rem);
 #pragma unroll
-      for(int k=0; k < V; ++k) {
-        const unsigned o=(unsigned) min(t+TPS*k,rem-1)*(unsigned) sizeof(cplx<T>);
-        a[k]=ld_buf<T>(rf,o,0);
-        b[k]=ld_buf<T>(rg,o,0);
+      for(int k=0; k < V; ++k) {            // words past the end read zero
+        a[k]=ld_buf<T>(rf,(unsigned) t*E,TPS*k*E);
+        b[k]=ld_buf<T>(rg,(unsigned) t*E,TPS*k*E);
       }
     } else {
 #pragma unroll
@@ -204,7 +204,7 @@ __device__ __forceinline__ void batch_zm_unit(const cplx<T> *zN, const cplx<T> *
     }
 #pragma unroll
     for(int k=0; k < V; ++k) {
-      const cplx<T> w=t+TPS*k < rem ? wb : mk((T) 0,(T) 0);
+      const cplx<T> w=BUF || t+TPS*k < rem ? wb : mk((T) 0,(T) 0);
       X[k]=X[k]+w*a[k];
       Y[k]=Y[k]+w*b[k];
     }
@@ -262,20 +262,22 @@ batch_reg_kernel(DimArgs d, const BatchItem *items, int64_t count,
   typedef RPlan<M,V> P;
   constexpr int TPS=P::TPS;
   extern __shared__ char smem_raw[];
-  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
+  typedef SplitTw<T,M,V> ST;
+  cplx<T> *twl=reinterpret_cast<cplx<T> *>(smem_raw);
   const cplx<T> *zN=(const cplx<T> *) d.zN;
-  fill_twr<T,M,V>(tw,zN,(int) d.q,threadIdx.x,blockDim.x);
+  fill_twr<T,M,V,ST::USED>(twl,zN,(int) d.q,threadIdx.x,blockDim.x);
+  const auto tw=stage_table<T,M,V>(twl,d);
   const int slots=blockDim.x/TPS;
   // residue twiddles w_N^{(t + TPS k) r} = w_N^{t r} w_N^{TPS k r}: the
   // uniform factor from an LDS table tq[r V + k] after the exchange areas
-  cplx<T> *tq=reinterpret_cast<cplx<T> *>(reinterpret_cast<T *>(tw+M)+slots*2*P::PAD);
+  cplx<T> *tq=reinterpret_cast<cplx<T> *>(reinterpret_cast<T *>(twl+ST::LDS)+slots*2*P::PAD);
   for(int e=threadIdx.x; e < (int) d.q*V; e += blockDim.x) {
     const int r=e/V, k=e-r*V;
     tq[e]=zN[TPS*k*r];                   // TPS k r < M r < N
   }
   __syncthreads();
   const int slot=threadIdx.x/TPS, t=threadIdx.x-slot*TPS;
-  T *xb=reinterpret_cast<T *>(tw+M)+slot*2*P::PAD;
+  T *xb=reinterpret_cast<T *>(twl+ST::LDS)+slot*2*P::PAD;
   if constexpr(ZM && sizeof(T) == 8) {
     // the FP64 sequence mode (the host passes D = 0): units (item,
     // residue), dealt to XCDs as the residue groups below

@@ -241,25 +241,27 @@ bool tile_fits(const fftwpp_amd_batch &h, const Cls &c, size_t TR)
 
 // Sub-FFT size without tuning.  One residue (m = 2^ceil(log2 M)) needs no
 // second launch and folds nothing, up to the size where the transform's
-// exchange area and twiddles leave too few blocks on a CU: 4096 in FP32, 1024
-// in FP64; longer items take two or more residues of m = 1024 (M <= 2048) or
-// 2048 (FP64, L <= 8192), else of 4096.  4096 sequences of 64 ... 16384 words
-// in FP64, with the units of default_tile:
-// 1065 us with m = 2^ceil(log2 L) and two units per CU, 830 us so.
+// exchange area and twiddles leave too few blocks on a CU: 4096 in FP32, 2048
+// in FP64 (6000 items of 600 to 1024 words: 145 us, 168 with two residues of
+// 1024); longer FP64 items take residues of m = 2048 (L <= 8192; 1000 items of
+// 4097 to 7000 words: 248 us, 264 with 4096 and 292 with 1024), else of 4096
+// (300 items of 16000 words: 254 us, 272 with 2048).  4096 sequences of 64 to
+// 16384 words in FP64, with the units of default_tile: 1065 us with m =
+// 2^ceil(log2 L) and two units per CU, 570 us so.
 size_t default_m(size_t L, size_t M, int dtype)
 {
   const size_t e=std::max<size_t>(16,ceilpow2(M));
   if(dtype == FFTWPP_AMD_F32) return std::min<size_t>(e,BATCH_MAXM);
-  if(e <= 1024) return e;
-  if(e <= 2048) return 1024;
+  if(e <= 2048) return e;
   return L <= 8192 ? 2048 : BATCH_MAXM;
 }
 
 // Without tuning.  Register kernel: items of several residues run in the
 // sequence mode (D = 0: every residue a unit, the outputs folded by a second
-// launch), except q = 2 with m = 2048 in FP64, whose unit does both residues;
+// launch), except q = 2 with m = 2048 in FP64, whose unit does both residues
+// (4000 items of 1025 to 1700 words: 209 us, 226 in the sequence mode);
 // when several units share an item the grid is the blocks that stay resident
-// (two waves per SIMD, LDS permitting), so an item's units run close together
+// (two waves per SIMD, three in FP64, LDS permitting), so an item's units run close together
 // and find its words in L2.  LDS kernel: small tiles of short items, and
 // enough residue groups for about two work units per compute unit.
 Tile default_tile(const fftwpp_amd_batch &h, const Cls &c)
@@ -270,8 +272,9 @@ Tile default_tile(const fftwpp_amd_batch &h, const Cls &c)
     Tile t=make_tile(h,c,1,threads,D);
     if(tps > 64 && groups(c,t) > 1) {
       const size_t elt=h.dtype == FFTWPP_AMD_F32 ? 8 : 16;
-      const size_t lds=(2*c.m+c.m/16+c.q*(c.m/tps))*elt;     // twiddles, exchange area
-      const size_t per=std::max<size_t>(1,std::min<size_t>(160*1024/lds,512/tps));
+      const size_t tw=elt == 16 && c.m >= 1024 ? 512 : c.m;  // twiddles, exchange area
+      const size_t lds=(tw+c.m+c.m/16+c.q*(c.m/tps))*elt;
+      const size_t per=std::max<size_t>(1,std::min<size_t>(160*1024/lds,(elt == 16 ? 768 : 512)/tps));
       t.nblocks=std::min(t.nblocks,per*(size_t) h.cus);
     }
     return t;

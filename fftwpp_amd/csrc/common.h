@@ -121,6 +121,7 @@ struct DimArgs {
   int nstages;
   int radix[MAXSTAGES];
   const void *zN; // zN[j] = e^{2 pi i j/N}, j < N, in the kernel's precision
+  const void *last; // FP64, m = 1024, 2048, 4096: the last stage's twiddles (fftr.h)
 };
 
 // Column tile of block x of a grid row of gx blocks.  Blocks are dealt to

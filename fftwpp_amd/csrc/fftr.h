@@ -90,12 +90,12 @@ __device__ __forceinline__ int xidx(int e)
 }
 
 // Twiddle table (M - 1 complex words) from zN of a dimension with N = M q.
-template<typename T, int M, int V=16>
+template<typename T, int M, int V=16, bool SPLIT=false>
 __device__ __forceinline__ void fill_twr(cplx<T> *tw, const cplx<T> *zN, int q,
                                          int tid, int nthreads)
 {
   typedef RPlan<M,V> P;
-  for(int e=tid; e < M-1; e += nthreads) {
+  for(int e=tid; e < (SPLIT ? P::off(P::NST-1) : M-1); e += nthreads) {
     // locate the stage of entry e (constants per unrolled k); Ns and Ns R are
     // powers of two: shifts only
     int ln=P::logns(1), lr=P::logns(1)+__builtin_ctz(P::radix(1)), off=0;
@@ -115,6 +115,48 @@ __device__ __forceinline__ void bfly(cplx<T> *u)
 {
   if constexpr(R == 16) dft16<T,S>(u);
   else DFT<T,R>::run(u,S);
+}
+
+// Twiddles of a long FP64 transform: those of the last stage, which are most
+// of the table (M = 2048: 24 of 32 KB), stay in device memory in the table's
+// order (DimArgs::last) and are read from there by each transform, consecutive
+// lanes consecutive words; LDS holds the others.  These transforms wait on LDS
+// and barriers rather than compute (13% of the vector unit's cycles), and with
+// all of the table in LDS two waves per SIMD were resident; now three are.
+// 2048 rows of 1000 points padded to 2048: 46 -> 38 us; 4096 sequences of 64
+// to 16384 words: 830 -> 570 us.
+template<typename T, int M, int V> struct SplitTw {
+  static constexpr bool USED=sizeof(T) == 8 && V == 8 && M >= 1024;
+  static constexpr int LDS=USED ? 512 : M;
+  const cplx<T> *tw;
+  __amdgpu_buffer_rsrc_t last;
+};
+
+// The table as the kernels pass it on: split, or all of it in LDS.
+template<typename T, int M, int V>
+__device__ __forceinline__ auto stage_table(const cplx<T> *tw, const DimArgs &d)
+{
+  if constexpr(SplitTw<T,M,V>::USED) {
+    typedef RPlan<M,V> P;
+    return SplitTw<T,M,V>{tw,buf_rsrc((const cplx<T> *) d.last,(size_t) (M-1-P::off(P::NST-1)))};
+  } else return tw;
+}
+
+// Twiddle tp of stage s for butterfly j = t + J (J constant): word off(s) +
+// (tp - 1) ns(s) + (j mod ns(s)) of the table.
+template<typename T, int M, int V, int s>
+__device__ __forceinline__ cplx<T> stage_word(const cplx<T> *tw, int t, int J, int tp)
+{
+  typedef RPlan<M,V> P;
+  return table_word(tw+P::off(s)+((t+J) & (P::ns(s)-1))+(tp-1)*P::ns(s));
+}
+template<typename T, int M, int V, int s>
+__device__ __forceinline__ cplx<T> stage_word(const SplitTw<T,M,V> &w, int t, int J, int tp)
+{
+  typedef RPlan<M,V> P;
+  constexpr unsigned E=sizeof(cplx<T>);
+  if constexpr(s == P::NST-1) return ld_buf<T>(w.last,(unsigned) t*E,(J+(tp-1)*P::ns(s))*E);
+  else return stage_word<T,M,V,s>(w.tw,t,J,tp);
 }
 
 // Synchronisation of the threads of a sequence: the wave when a sequence
@@ -146,26 +188,23 @@ template<typename T, int M, int V> struct RowXI {
 // the second, and each exchange is one round (two synchronisations instead
 // of four); element e sits at word XI::at(e) ^ xm of each half.
 template<typename T, int M, int V, int S, int s, bool BLK, bool CX=false,
-         class XI=RowXI<T,M,V>>
-__device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const cplx<T> *tw,
+         class XI=RowXI<T,M,V>, class TW>
+__device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const TW &tw,
                                            int t, int xm=0)
 {
   typedef RPlan<M,V> P;
   constexpr int TPS=P::TPS;
-  constexpr int R=P::radix(s), NB=V/R, Ns=P::ns(s), OFF=P::off(s);
+  constexpr int R=P::radix(s), NB=V/R, Ns=P::ns(s);
   // butterflies in place: slot b + t' NB holds input t' / output u = t'
 #pragma unroll
   for(int b=0; b < NB; ++b) {
-    const int j=t+TPS*b;
-    const int kp=j & (Ns-1);
     cplx<T> u[R];
 #pragma unroll
     for(int tp=0; tp < R; ++tp) u[tp]=v[b+tp*NB];
     if constexpr(s > 0) {
-      const cplx<T> *w=tw+OFF+kp;
 #pragma unroll
       for(int tp=1; tp < R; ++tp) {
-        const cplx<T> z=table_word(w+(tp-1)*Ns);
+        const cplx<T> z=stage_word<T,M,V,s>(tw,t,TPS*b,tp);
         u[tp]=S > 0 ? u[tp]*z : mulc(u[tp],z);
       }
     }
@@ -223,18 +262,16 @@ __device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const cplx<T> *tw,
 // exchanges, the default index map): the butterflies of both sequences are
 // independent work for the same waves, then each is exchanged in turn through
 // the one area (the same barriers as two fftr calls).
-template<typename T, int M, int V, int S, int s>
+template<typename T, int M, int V, int S, int s, class TW>
 __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
-                                                const cplx<T> *tw, int t)
+                                                const TW &tw, int t)
 {
   typedef RPlan<M,V> P;
   typedef RowXI<T,M,V> XI;
   constexpr int TPS=P::TPS;
-  constexpr int R=P::radix(s), NB=V/R, Ns=P::ns(s), OFF=P::off(s);
+  constexpr int R=P::radix(s), NB=V/R, Ns=P::ns(s);
 #pragma unroll
   for(int b=0; b < NB; ++b) {
-    const int j=t+TPS*b;
-    const int kp=j & (Ns-1);
     cplx<T> u[R], v[R];
 #pragma unroll
     for(int tp=0; tp < R; ++tp) {
@@ -242,10 +279,9 @@ __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
       v[tp]=Y[b+tp*NB];
     }
     if constexpr(s > 0) {
-      const cplx<T> *w=tw+OFF+kp;
 #pragma unroll
       for(int tp=1; tp < R; ++tp) {
-        const cplx<T> z=table_word(w+(tp-1)*Ns);
+        const cplx<T> z=stage_word<T,M,V,s>(tw,t,TPS*b,tp);
         u[tp]=S > 0 ? u[tp]*z : mulc(u[tp],z);
         v[tp]=S > 0 ? v[tp]*z : mulc(v[tp],z);
       }
@@ -286,8 +322,8 @@ __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
 
 // fftr<T,M,V,S,true> of X and of Y, their butterflies interleaved stage by
 // stage; same results, same exchange area and barriers.
-template<typename T, int M, int V, int S>
-__device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const cplx<T> *tw,
+template<typename T, int M, int V, int S, class TW>
+__device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const TW &tw,
                                           int t)
 {
   fftr_pair_stage<T,M,V,S,0>(X,Y,xb,tw,fresh(t));
@@ -297,8 +333,8 @@ __device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const c
 // with kernel e^{S 2 pi i jk/M}; xb is the sequence's exchange area
 // (RPlan<M,V>::PAD scalar words), tw the twiddle table of RPlan<M,V>.  When
 // TPS > 64 every thread of the block must call this.
-template<typename T, int M, int V, int S, bool CX=false>
-__device__ __forceinline__ void fftr(cplx<T> *v, T *xb, const cplx<T> *tw, int t)
+template<typename T, int M, int V, int S, bool CX=false, class TW>
+__device__ __forceinline__ void fftr(cplx<T> *v, T *xb, const TW &tw, int t)
 {
   fftr_stage<T,M,V,S,0,false,CX>(v,xb,tw,fresh(t));
 }

@@ -42,15 +42,24 @@ namespace {
 // Twiddle generation: zN[j] = e^{2 pi i j/N} in FP64, rounded to FP32 for
 // the single-precision copy.
 // ------------------------------------------------------------------------
-__global__ void twiddle_kernel(int64_t N, cplx<double> *z64, cplx<float> *z32)
+// Words from N on of z64: the last stage's twiddles of the register transform
+// of m = 8 Ns or less points, word (tp - 1) Ns + kp = zN[q tp kp] (fill_twr's
+// order), nlast of them.
+__global__ void twiddle_kernel(int64_t N, cplx<double> *z64, cplx<float> *z32, int64_t q, int Ns,
+                               int64_t nlast)
 {
-  int64_t j=(int64_t) blockIdx.x*blockDim.x+threadIdx.x;
-  if(j >= N) return;
+  const int64_t e=(int64_t) blockIdx.x*blockDim.x+threadIdx.x;
+  if(e >= N+nlast) return;
+  int64_t j=e;
+  if(e >= N) {
+    const int w=(int) (e-N), tp=w/Ns+1;
+    j=q*tp*(w-(tp-1)*Ns);
+  }
   double s, c;
   // reduce to [0,1/2] octant-free: sincospi(2j/N) with exact integer ratio
   sincospi(2.0*(double) j/(double) N,&s,&c);
-  z64[j]=mk(c,s);
-  z32[j]=mk((float) c,(float) s);
+  z64[e]=mk(c,s);
+  if(e < N) z32[e]=mk((float) c,(float) s);
 }
 
 template<typename T>
@@ -1230,7 +1239,8 @@ static void batch_reg_shape(size_t m, size_t q, size_t elt, size_t threads,
   if(n > 512) n=512/tps*tps;
   const size_t pad=m >= 512 ? m : m+m/16;      // RPlan::PAD
   *nt=n;
-  *lds=m*elt+(n/tps)*2*pad*(elt/2)+q*(m/tps)*elt;
+  const size_t tw=elt == sizeof(cplx<double>) && m >= 1024 ? 512 : m;   // SplitTw::LDS
+  *lds=tw*elt+(n/tps)*2*pad*(elt/2)+q*(m/tps)*elt;
 }
 
 template<typename T, int M, bool ZM>
@@ -1678,17 +1688,23 @@ int fftwpp_amd_dim_create(fftwpp_amd_dim **out, size_t L, size_t m,
     while(r % p == 0 && ns < MAXSTAGES) { a.radix[ns++]=(int) p; r /= p; }
   if(r != 1) { delete d; return fail(FFTWPP_AMD_ERR_UNSUPPORTED,"too many FFT stages"); }
   a.nstages=ns;
-  int rc=hipcheck(hipMalloc(&d->z64,sizeof(cplx<double>)*N),"hipMalloc twiddles");
+  // last-stage twiddles after the N words (SplitTw in fftr.h)
+  int lastNs=0, off=0;
+  if(m == 1024) { lastNs=RPlan<1024,8>::ns(RPlan<1024,8>::NST-1); off=RPlan<1024,8>::off(RPlan<1024,8>::NST-1); }
+  if(m == 2048) { lastNs=RPlan<2048,8>::ns(RPlan<2048,8>::NST-1); off=RPlan<2048,8>::off(RPlan<2048,8>::NST-1); }
+  if(m == 4096) { lastNs=RPlan<4096,8>::ns(RPlan<4096,8>::NST-1); off=RPlan<4096,8>::off(RPlan<4096,8>::NST-1); }
+  const size_t nlast=lastNs ? m-1-off : 0;
+  int rc=hipcheck(hipMalloc(&d->z64,sizeof(cplx<double>)*(N+nlast)),"hipMalloc twiddles");
   if(rc) { delete d; return rc; }
   rc=hipcheck(hipMalloc(&d->z32,sizeof(cplx<float>)*N),"hipMalloc twiddles");
   if(rc) { (void) hipFree(d->z64); delete d; return rc; }
-  unsigned nb=(unsigned) ((N+255)/256);
+  unsigned nb=(unsigned) ((N+nlast+255)/256);
   twiddle_kernel<<<nb,256>>>((int64_t) N,(cplx<double> *) d->z64,
-                             (cplx<float> *) d->z32);
+                             (cplx<float> *) d->z32,(int64_t) q,lastNs,(int64_t) nlast);
   rc=launch_check("twiddle_kernel");
   if(!rc) rc=hipcheck(hipDeviceSynchronize(),"twiddle sync");
   if(rc) { (void) hipFree(d->z64); (void) hipFree(d->z32); delete d; return rc; }
-  d->a64=a; d->a64.zN=d->z64;
+  d->a64=a; d->a64.zN=d->z64; d->a64.last=(const cplx<double> *) d->z64+N;
   d->a32=a; d->a32.zN=d->z32;
   *out=d;
   return FFTWPP_AMD_OK;

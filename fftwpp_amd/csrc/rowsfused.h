@@ -112,7 +112,7 @@ inline int rowreg_launch_rp(const DimArgs &a, const void *f, const void *g, size
   constexpr int TPS=M/V;
   const size_t nt=RP > 1 ? RP*TPS : (TPS > 64 ? TPS : 256);
   const size_t slots=nt/TPS;
-  const size_t lds=M*sizeof(cplx<T>)+slots*2*RPlan<M,V>::PAD*sizeof(T);
+  const size_t lds=(HERM ? M : SplitTw<T,M,V>::LDS)*sizeof(cplx<T>)+slots*2*RPlan<M,V>::PAD*sizeof(T);
   const size_t rpb=RP > 1 ? 1 : slots;
   if constexpr(HERM) {
     const hipError_t e=fused_allow_lds(rowreg_kernel<T,M,RP,Op>,lds);

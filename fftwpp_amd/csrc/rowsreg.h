@@ -106,13 +106,15 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
   constexpr int TPS=P::TPS;
   constexpr unsigned E=sizeof(cplx<T>);
   extern __shared__ char smem_raw[];
-  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
+  typedef SplitTw<T,M,V> ST;
+  cplx<T> *twl=reinterpret_cast<cplx<T> *>(smem_raw);
+  const auto tw=stage_table<T,M,V>(twl,d);
   const cplx<T> *zN=(const cplx<T> *) d.zN;
   const int slots=RP > 1 ? 1 : blockDim.x/TPS;      // rows per block
   const int slot=threadIdx.x/TPS, t=threadIdx.x-slot*TPS;
   const int rp=RP > 1 ? slot : 0;                     // residue lane
   const int rslot=RP > 1 ? 0 : slot;
-  T *xbase=reinterpret_cast<T *>(tw+M);
+  T *xbase=reinterpret_cast<T *>(twl+ST::LDS);
   T *xb=xbase+slot*2*P::PAD;
   const int q=(int) d.q, L=(int) d.L, k0=(int) d.k0;
   cplx<T> a[V], b[V];
@@ -132,7 +134,7 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
   };
   const int64_t step=(int64_t) gridDim.x*slots;
   int64_t rb=(int64_t) blockIdx.x*slots;
-  fill_twr<T,M,V>(tw,zN,q,threadIdx.x,blockDim.x);
+  fill_twr<T,M,V,ST::USED>(twl,zN,q,threadIdx.x,blockDim.x);
   __syncthreads();
   for(; rb < rows; rb += step) {
     const int64_t row=rb+rslot;
