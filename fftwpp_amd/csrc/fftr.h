@@ -125,20 +125,20 @@ __device__ __forceinline__ void bfly(cplx<T> *u)
 // all of the table in LDS two waves per SIMD were resident; now three are.
 // 2048 rows of 1000 points padded to 2048: 46 -> 38 us; 4096 sequences of 64
 // to 16384 words: 830 -> 570 us.
-template<typename T, int M, int V> struct SplitTw {
-  static constexpr bool USED=sizeof(T) == 8 && V == 8 && M >= 1024;
+template<typename T, int M, int V, int MIN=1024> struct SplitTw {
+  static constexpr bool USED=sizeof(T) == 8 && V == 8 && M >= MIN;
   static constexpr int LDS=USED ? 512 : M;
   const cplx<T> *tw;
   __amdgpu_buffer_rsrc_t last;
 };
 
 // The table as the kernels pass it on: split, or all of it in LDS.
-template<typename T, int M, int V>
+template<typename T, int M, int V, int MIN=1024>
 __device__ __forceinline__ auto stage_table(const cplx<T> *tw, const DimArgs &d)
 {
-  if constexpr(SplitTw<T,M,V>::USED) {
+  if constexpr(SplitTw<T,M,V,MIN>::USED) {
     typedef RPlan<M,V> P;
-    return SplitTw<T,M,V>{tw,buf_rsrc((const cplx<T> *) d.last,(size_t) (M-1-P::off(P::NST-1)))};
+    return SplitTw<T,M,V,MIN>{tw,buf_rsrc((const cplx<T> *) d.last,(size_t) (M-1-P::off(P::NST-1)))};
   } else return tw;
 }
 
@@ -150,8 +150,8 @@ __device__ __forceinline__ cplx<T> stage_word(const cplx<T> *tw, int t, int J, i
   typedef RPlan<M,V> P;
   return table_word(tw+P::off(s)+((t+J) & (P::ns(s)-1))+(tp-1)*P::ns(s));
 }
-template<typename T, int M, int V, int s>
-__device__ __forceinline__ cplx<T> stage_word(const SplitTw<T,M,V> &w, int t, int J, int tp)
+template<typename T, int M, int V, int s, int MIN>
+__device__ __forceinline__ cplx<T> stage_word(const SplitTw<T,M,V,MIN> &w, int t, int J, int tp)
 {
   typedef RPlan<M,V> P;
   constexpr unsigned E=sizeof(cplx<T>);
@@ -350,8 +350,8 @@ __device__ __forceinline__ void fftr_blk(cplx<T> *v, T *xb, const cplx<T> *tw,
 
 // fftr_blk with one-round exchanges through the index map XI, XORed by xm.
 // FRESH: positions computed anew (see fresh()).
-template<typename T, int M, int V, int S, class XI, bool FRESH=true>
-__device__ __forceinline__ void fftr_blkx(cplx<T> *v, T *xb, const cplx<T> *tw,
+template<typename T, int M, int V, int S, class XI, bool FRESH=true, class TW>
+__device__ __forceinline__ void fftr_blkx(cplx<T> *v, T *xb, const TW &tw,
                                           int t, int xm)
 {
   fftr_stage<T,M,V,S,0,true,true,XI>(v,xb,tw,FRESH ? fresh(t) : t,xm);

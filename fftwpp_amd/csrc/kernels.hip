@@ -921,7 +921,7 @@ static int colreg_launch(const DimArgs &a, bool fwd, const ColArrays &io,
                          size_t ics, size_t ocs, hipStream_t st)
 {
   typedef ColReg<T,M> CR;
-  size_t lds=M*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
+  size_t lds=CR::ST::LDS*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
   dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
   grid.z=fwd ? col_depth(io,(size_t) grid.x*nbatch,nres) : (unsigned) io.n;
   const bool p2=a.L > M;
@@ -996,7 +996,7 @@ static int colreal_launch(const DimArgs &a, bool fwd, const ColArrays &io,
                           size_t ics, size_t ocs, hipStream_t st)
 {
   typedef ColReg<T,M> CR;
-  const size_t lds=M*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
+  const size_t lds=CR::ST::LDS*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
   dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
   if(fwd) grid.z=col_depth(io,(size_t) grid.x*nbatch,(size_t) RealKept::residues(a.q));
   const bool p2=a.L > M;

@@ -646,6 +646,7 @@ template<typename T, int M> struct ColReg {
     M == 1024 ? 10 : M == 2048 ? (F64 ? 28 : 20) : 1;
   static constexpr int CS=2*PAD+X;
   static constexpr int NT=TPS*TC;
+  typedef SplitTw<T,M,V,2048> ST;
   static __device__ __forceinline__ int at(int e)
   {
     if constexpr(BASE == 2 && F64) return e ^ ((e >> 4) & 7) ^ (((e >> 6) & 1) << 3);
@@ -660,11 +661,14 @@ template<typename T, int M> struct ColReg {
 
 // Waves per SIMD asked of the complex column kernels: four, so that two blocks
 // of 512 threads share a CU and one loads while the other transforms, where
-// the registers allow it without spills: all FP32 columns (at most 114), FP64
-// with p = 1 (110 forward; 122 to 128 backward with M = 64 and 512 above) and
-// M below 4096, whose LDS holds one block.
+// the registers allow it with at most a few spills: all FP32 columns (at most
+// 114), FP64 with p = 1 (110 forward; 122 to 128 backward with M = 64 and 512
+// above, 16 and 28 bytes spilled at 2048 and 4096).  FP64 columns of M >= 2048
+// leave room for the second block by reading the last stage's twiddles from
+// memory (SplitTw; 2D FP64 2000 x 500: 92 -> 81 us, 4000 x 500: 209 -> 170 us,
+// 4000 x 1000: 477 -> 428 us); at 1024 two blocks fit beside the whole table.
 template<typename T, int M, int P2, bool FWD> struct ColW {
-  static constexpr bool FIT=P2 == 1 && M < 4096 && (FWD || (M != 64 && M != 512));
+  static constexpr bool FIT=P2 == 1 && (FWD || (M != 64 && M != 512));
   static constexpr int W=sizeof(T) == 4 || FIT ? 4 : 2;
 };
 
@@ -684,8 +688,8 @@ __device__ __forceinline__ ColTwiddles<T,M> col_twiddles(const DimArgs &d, cplx<
 {
   typedef ColReg<T,M> CR;
   const cplx<T> *zN=(const cplx<T> *) d.zN;
-  fill_twr<T,M,CR::V>(tw,zN,(int) d.q,threadIdx.x,CR::NT);
-  cplx<T> *zl=reinterpret_cast<cplx<T> *>(reinterpret_cast<T *>(tw+M)+CR::TC*CR::CS);
+  fill_twr<T,M,CR::V,CR::ST::USED>(tw,zN,(int) d.q,threadIdx.x,CR::NT);
+  cplx<T> *zl=reinterpret_cast<cplx<T> *>(reinterpret_cast<T *>(tw+CR::ST::LDS)+CR::TC*CR::CS);
   if(zlds)
     for(int e=threadIdx.x; e < (int) d.N; e += CR::NT) zl[e]=zN[e];
   __syncthreads();
@@ -731,14 +735,15 @@ colfwd_reg_kernel(DimArgs d, ColArrays io, int64_t S, int64_t C,
   typedef ColReg<T,M> CR;
   constexpr int V=CR::V, TPS=CR::TPS, TC=CR::TC;
   extern __shared__ char smem_raw[];
-  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
-  const ColTwiddles<T,M> zt=col_twiddles<T,M>(d,tw,zlds);
+  cplx<T> *twl=reinterpret_cast<cplx<T> *>(smem_raw);
+  const ColTwiddles<T,M> zt=col_twiddles<T,M>(d,twl,zlds);
+  const auto tw=stage_table<T,M,V,2048>(twl,d);
   // interleaved columns: consecutive lanes on consecutive columns; rows
   // (column stride ics > 1): a row's threads on consecutive lanes
   const bool rowmap=ics != 1;
   const int c=rowmap ? threadIdx.x/TPS : threadIdx.x % TC;
   const int t=rowmap ? threadIdx.x % TPS : threadIdx.x/TC;
-  T *xb=reinterpret_cast<T *>(tw+M)+c*CR::CS;
+  T *xb=reinterpret_cast<T *>(twl+CR::ST::LDS)+c*CR::CS;
   const int xm=CR::xm(c);
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
@@ -791,14 +796,15 @@ colbwd_reg_kernel(DimArgs d, ColArrays io, int64_t SF, int64_t bsi,
   typedef ColReg<T,M> CR;
   constexpr int V=CR::V, TPS=CR::TPS, TC=CR::TC;
   extern __shared__ char smem_raw[];
-  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
-  const ColTwiddles<T,M> zt=col_twiddles<T,M>(d,tw,zlds);
+  cplx<T> *twl=reinterpret_cast<cplx<T> *>(smem_raw);
+  const ColTwiddles<T,M> zt=col_twiddles<T,M>(d,twl,zlds);
+  const auto tw=stage_table<T,M,V,2048>(twl,d);
   // interleaved columns: consecutive lanes on consecutive columns; rows
   // (column stride ics > 1): a row's threads on consecutive lanes
   const bool rowmap=ics != 1;
   const int c=rowmap ? threadIdx.x/TPS : threadIdx.x % TC;
   const int t=rowmap ? threadIdx.x % TPS : threadIdx.x/TC;
-  T *xb=reinterpret_cast<T *>(tw+M)+c*CR::CS;
+  T *xb=reinterpret_cast<T *>(twl+CR::ST::LDS)+c*CR::CS;
   const int xm=CR::xm(c);
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
@@ -889,14 +895,15 @@ colfwd_real_kernel(DimArgs d, ColArrays io, int64_t S, int64_t C, int64_t bsi,
   typedef ColReg<T,M> CR;
   constexpr int V=CR::V, TPS=CR::TPS, TC=CR::TC;
   extern __shared__ char smem_raw[];
-  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
+  cplx<T> *twl=reinterpret_cast<cplx<T> *>(smem_raw);
+  const auto tw=stage_table<T,M,V,2048>(twl,d);
   const cplx<T> *zN=(const cplx<T> *) d.zN;
-  fill_twr<T,M,V>(tw,zN,(int) d.q,threadIdx.x,CR::NT);
+  fill_twr<T,M,V,CR::ST::USED>(twl,zN,(int) d.q,threadIdx.x,CR::NT);
   __syncthreads();
   const bool rowmap=ics != 1;
   const int c=rowmap ? threadIdx.x/TPS : threadIdx.x % TC;
   const int t=rowmap ? threadIdx.x % TPS : threadIdx.x/TC;
-  T *xb=reinterpret_cast<T *>(tw+M)+c*CR::CS;
+  T *xb=reinterpret_cast<T *>(twl+CR::ST::LDS)+c*CR::CS;
   const int xm=CR::xm(c);
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
@@ -951,14 +958,15 @@ colbwd_real_kernel(DimArgs d, const cplx<T> *F, int64_t SF, int64_t bsi,
   typedef ColReg<T,M> CR;
   constexpr int V=CR::V, TPS=CR::TPS, TC=CR::TC;
   extern __shared__ char smem_raw[];
-  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
+  cplx<T> *twl=reinterpret_cast<cplx<T> *>(smem_raw);
+  const auto tw=stage_table<T,M,V,2048>(twl,d);
   const cplx<T> *zN=(const cplx<T> *) d.zN;
-  fill_twr<T,M,V>(tw,zN,(int) d.q,threadIdx.x,CR::NT);
+  fill_twr<T,M,V,CR::ST::USED>(twl,zN,(int) d.q,threadIdx.x,CR::NT);
   __syncthreads();
   const bool rowmap=ics != 1;
   const int c=rowmap ? threadIdx.x/TPS : threadIdx.x % TC;
   const int t=rowmap ? threadIdx.x % TPS : threadIdx.x/TC;
-  T *xb=reinterpret_cast<T *>(tw+M)+c*CR::CS;
+  T *xb=reinterpret_cast<T *>(twl+CR::ST::LDS)+c*CR::CS;
   const int xm=CR::xm(c);
   const int64_t c0=xcd_tile(blockIdx.x,gridDim.x)*TC;
   const bool ok=c0+c < C;
