@@ -325,7 +325,7 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
 // the wavenumbers k = sigma and sigma - M of the block (f(-k) = conj f(k),
 // w_N^{(sigma - M) r} = w_N^{sigma r} w_q^{-r}).  rf, rg: buffers over the
 // row's H words; tr[k] = w_N^{TPS k r}, tr[V] = w_N^{M r} (LDS); b = w_N^{t r}.
-// Out-of-range words are read at index 0 and then zeroed (no branches).
+// Out-of-range words read zero, past the end of the buffers (no branches).
 template<typename T, int M>
 __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buffer_rsrc_t rf,
                                           __amdgpu_buffer_rsrc_t rg, const cplx<T> *tr1,
@@ -333,18 +333,15 @@ __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buf
                                           int r1, int r2, int H, unsigned ro)
 {
   constexpr int V=RowV::V, TPS=M/V;
-  constexpr unsigned E=sizeof(cplx<T>);
+  constexpr unsigned E=sizeof(cplx<T>), END=0x80000000u;
   const cplx<T> c1=conjg(tr1[V]), c2=conjg(tr2[V]);
-  const cplx<T> zero=mk((T) 0,(T) 0);
 #pragma unroll
   for(int k=0; k < V; ++k) {
     const int sigma=t+TPS*k;
-    const bool iu=sigma < H, iv=M-sigma < H;
-    const unsigned ou=ro+(unsigned) (iu ? sigma : 0)*E, ov=ro+(unsigned) (iv ? M-sigma : 0)*E;
+    const unsigned ou=sigma < H ? ro+(unsigned) sigma*E : END, ov=M-sigma < H ? ro+(unsigned) (M-sigma)*E : END;
     const cplx<T> fu=ld_buf<T>(rf,ou,0), gu=ld_buf<T>(rg,ou,0);
     const cplx<T> fv=ld_buf<T>(rf,ov,0), gv=ld_buf<T>(rg,ov,0);
-    const cplx<T> u=iu ? mk(fu.x-gu.y,fu.y+gu.x) : zero;
-    const cplx<T> v=iv ? mk(fv.x+gv.y,gv.x-fv.y) : zero;
+    const cplx<T> u=mk(fu.x-gu.y,fu.y+gu.x), v=mk(fv.x+gv.y,gv.x-fv.y);
     cplx<T> a=u+c1*v, b=u+c2*v;
     if(r1) a=(b1*tr1[k])*a;
     if(r2) b=(b2*tr2[k])*b;
@@ -376,16 +373,16 @@ struct HRowPk {
   static constexpr int TPS=M/V;
   static constexpr int SLOTS=256/TPS > 0 ? 256/TPS : 1;
   static constexpr int NT=SLOTS*TPS;
-  // waves per SIMD where the short rows fit them without spills (150 and 90
-  // registers)
-  static constexpr int W=M > 256 ? 2 : sizeof(T) == 4 ? 4 : 3;
+  // waves per SIMD that fit without spills (150 to 158 and 90 registers)
+  static constexpr int W=sizeof(T) == 4 ? 4 : 3;
+  typedef SplitTw<T,M,V,2048> ST;           // at 2048 the table leaves two blocks
 };
 
 template<typename T, int M>
 inline size_t hrowpk_lds(int q)
 {
   typedef HRowPk<T,M> K;
-  return (size_t) (M+q*(K::V+1))*sizeof(cplx<T>)+(size_t) K::SLOTS*2*RPlan<M,K::V>::PAD*sizeof(T);
+  return (size_t) (K::ST::LDS+q*(K::V+1))*sizeof(cplx<T>)+(size_t) K::SLOTS*2*RPlan<M,K::V>::PAD*sizeof(T);
 }
 
 template<typename T, int M, class Op>
@@ -399,10 +396,11 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
   constexpr unsigned E=sizeof(cplx<T>);
   extern __shared__ char smem_raw[];
   const int q=(int) d.q, H=(int) d.H;
-  cplx<T> *tw=reinterpret_cast<cplx<T> *>(smem_raw);
-  cplx<T> *tq=tw+M;                           // tq[r (V + 1) + k] = w_N^{TPS k r}
+  cplx<T> *twl=reinterpret_cast<cplx<T> *>(smem_raw);
+  const auto tw=stage_table<T,M,V,2048>(twl,d);
+  cplx<T> *tq=twl+K::ST::LDS;                 // tq[r (V + 1) + k] = w_N^{TPS k r}
   const cplx<T> *zN=(const cplx<T> *) d.zN;
-  fill_twr<T,M,V>(tw,zN,q,threadIdx.x,blockDim.x);
+  fill_twr<T,M,V,K::ST::USED>(twl,zN,q,threadIdx.x,blockDim.x);
   for(int e=threadIdx.x; e < q*(V+1); e += blockDim.x) {
     const int r=e/(V+1), k=e-r*(V+1);
     tq[e]=zN[TPS*k*r];                        // TPS k r <= M r < N
@@ -429,9 +427,8 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
     const auto rop=bind_row(op,row);
     for(int r1=0; r1 < q; r1 += 2) {
       const int r2=r1+1 < q ? r1+1 : -1;
-      // (the loop's own positions too on short rows: 203 -> 183 us at M = 64,
-      // longer ones lose 2%)
-      const int ti=M <= 256 ? fresh(t) : t;
+      // the loop's own positions too (see fresh())
+      const int ti=fresh(t);
       const cplx<T> b1=zN[ti*r1];
       // both residues folded from one read of the row
       cplx<T> X[V], X2[V];
@@ -453,7 +450,7 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
       }
       fftr<T,M,V,-1,true>(X,xb,tw,t);
       // mirror elements Z(M - sigma) through LDS
-      const int tm=M <= 256 ? fresh(t) : t;
+      const int tm=fresh(t);
 #pragma unroll
       for(int k=0; k < V; ++k) {
         const int e=xidx<T,M,V>(tm+TPS*k);
@@ -474,7 +471,7 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
       rsync<TPS>();
     }
     if(live) {
-      const int to=M <= 256 ? fresh(t) : t;
+      const int to=fresh(t);
       if constexpr(TPS >= 64) {
         const __amdgpu_buffer_rsrc_t rw=buf_rsrc(out+row*os,H);
 #pragma unroll
