@@ -97,7 +97,8 @@ template<typename T, int M, int RP, class Op> struct RowCx {
   static constexpr int W=MORE && std::is_same<Op,RunMult>::value ? 3 : 2;
 };
 template<typename T, int M, int RP, class Op>
-__global__ void __launch_bounds__(RP*M/RowV::V > 256 ? 512 : 256,(RowCx<T,M,RP,Op>::W))
+__global__ void __launch_bounds__(RP*M/RowV::V > 512 ? 1024 : RP*M/RowV::V > 256 ? 512 : 256,
+                                  (RP*M/RowV::V > 512 ? 4 : RowCx<T,M,RP,Op>::W))
 rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_t rows,
              int64_t rs, cplx<T> *out, int64_t os, T scale, Op op)
 {
@@ -141,7 +142,11 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
-    for(int r=rp; r < q; r += RP) {
+    // residue lanes take the same number of passes, as the block's barriers
+    // need; one past the last residue repeats residue 0 and adds nothing
+    for(int r0=0; r0 < q; r0 += RP) {
+      const bool on=RP == 1 || r0+rp < q;
+      const int r=on ? r0+rp : 0;
       // w_N^{(j+k0) r}: j + k0 is sigma or sigma - M
       const cplx<T> bt=zN[t*r], zm=conjg(zN[M*r]);
       cplx<T> X[V], Y[V];
@@ -184,7 +189,7 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
           cplx<T> w=bt*zN[TPS*k*r];
           if(j+k0 < 0) w=w*zm;
           acc[k]=acc[k]+mulc(X[k],w);
-        } else
+        } else if(on)
           acc[k]=acc[k]+X[k];
       }
     }
@@ -234,7 +239,10 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
-    for(int r1=2*rp; r1 < q; r1 += 2*RP) {
+    // the same number of passes in every lane, as in rowcx_kernel
+    for(int p0=0; p0 < q; p0 += 2*RP) {
+      const bool on=RP == 1 || p0+2*rp < q;
+      const int r1=on ? p0+2*rp : 0;
       const int r2=r1+1 < q ? r1+1 : -1;
       // w_N^{sigma r} = w_N^{t r} w_N^{TPS k r}; w_N^{(sigma - M) r} adds
       // the factor conj w_N^{M r}
@@ -291,7 +299,7 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
 #pragma unroll
       for(int k=0; k < V; ++k) {
         const int sigma=t+TPS*k;
-        if(sigma < H) {
+        if(on && sigma < H) {
           const cplx<T> z=X[k], zc=conjg(Zm[k]);
           const cplx<T> y1=(T) 0.5*(z+zc);
           cplx<T> v=mulc(y1,b1*zN[TPS*k*r1]);

@@ -58,6 +58,24 @@ def test_complex_rows(gpu, oracle, Ly, my, q, dtype):
     assert oracle.rel_l2(h, want) < TOL[dtype]
 
 
+# two residue lanes per row (under 512 rows) and an odd number of passes: every
+# lane of the block has to reach the same barriers
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("kind,Ly,my,q", [("complex", 900, 1024, 3), ("complex", 2000, 2048, 3),
+                                          ("complex", 4000, 4096, 3), ("complex", 4000, 4096, 2),
+                                          ("hermitian", 600, 1024, 5), ("hermitian", 1100, 2048, 5)])
+def test_few_rows_odd_passes(gpu, oracle, kind, Ly, my, q, dtype):
+    rng = np.random.default_rng(Ly)
+    f, g = (_rnd(rng, (201, Ly)) for _ in range(2))
+    if kind == "hermitian":
+        f, g = oracle.symmetrize_x(f), oracle.symmetrize_x(g)
+    h, plan = _plan_run(gpu, f, g, kind, dtype, [402, my * q], [201, my])
+    N, m, _ = plan.geometry()
+    assert m == (201, my)
+    want = (oracle.explicit_hconv if kind == "hermitian" else oracle.explicit_conv)(f, g, N)
+    assert oracle.rel_l2(h, want) < TOL[dtype]
+
+
 @pytest.mark.parametrize("L,m,rows,rs", [(16, 16, 10, 1 << 24), (40, 64, 10, 1 << 24),
                                          (200, 256, 7, 1 << 24), (256, 256, 3, 1 << 27)])
 def test_rows_of_huge_stride(gpu, oracle, L, m, rows, rs):
