@@ -179,8 +179,12 @@ inline int rowreg_launch(const DimArgs &a, const void *f, const void *g, size_t 
     if(rows >= 512 && (size_t) HRowPk<T,M>::SLOTS <= rows_in_buffer(rs,sizeof(cplx<T>)) &&
        (size_t) a.q*(RowV::V+1)*sizeof(cplx<T>) <= 16*1024)
       return hrowpk_launch<T,M>(a,f,g,rows,rs,out,os,scale,op,st);
-  if(TPS <= 256 && rows < 512 && passes >= 2)
-    return rowreg_launch_rp<T,M,HERM,2>(a,f,g,rows,rs,out,os,scale,op,st);
+  // (both lanes of a row within one block: 1024 threads take 128 registers
+  // each, which complex FP32 rows of M = 4096 fit; one of 3000 points: 16.4 us,
+  // 18.4 us with its residues in turn)
+  if constexpr(TPS <= 256 || (sizeof(T) == 4 && !HERM))
+    if(rows < 512 && passes >= 2)
+      return rowreg_launch_rp<T,M,HERM,2>(a,f,g,rows,rs,out,os,scale,op,st);
   return rowreg_launch_rp<T,M,HERM,1>(a,f,g,rows,rs,out,os,scale,op,st);
 }
 

@@ -36,7 +36,7 @@ def test_default_units(gpu, oracle, L, dtype, tol):
 
 
 @pytest.mark.parametrize("dtype,tol", [("complex128", 1e-12), ("complex64", 1e-5)])
-@pytest.mark.parametrize("shape", [(4097,), (10000,), (30000,), (3, 5000)])
+@pytest.mark.parametrize("shape", [(2049,), (3000,), (4096,), (5, 4000), (4097,), (10000,), (30000,), (3, 5000)])
 def test_long_rows(gpu, oracle, shape, dtype, tol):
     import torch
     from fftwpp_amd.torch_conv import DeviceConvolution
