@@ -123,7 +123,7 @@ __device__ __forceinline__ void bfly(cplx<T> *u)
 // lanes consecutive words; LDS holds the others.  These transforms wait on LDS
 // and barriers rather than compute (13% of the vector unit's cycles), and with
 // all of the table in LDS two waves per SIMD were resident; now three are.
-// 2048 rows of 1000 points padded to 2048: 46 -> 38 us; 4096 sequences of 64
+// 2048 rows of 1000 points padded to 2048: 49 -> 41.5 us; 4096 sequences of 64
 // to 16384 words: 830 -> 570 us.
 template<typename T, int M, int V, int MIN=1024> struct SplitTw {
   static constexpr bool USED=sizeof(T) == 8 && V == 8 && M >= MIN;
