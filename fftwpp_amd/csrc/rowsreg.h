@@ -18,6 +18,7 @@
 // after the inverse with the mirror element Z(M - sigma), fetched through the
 // slot's LDS exchange area.
 #pragma once
+#include <limits>
 #include <type_traits>
 #include "batch.h"
 
@@ -324,6 +325,179 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
 }
 
 
+// The 32-bit words of a value.
+template<int N> struct Words { unsigned w[N]; };
+
+// c over the values of the TPS consecutive lanes of a slot (at most a wave), the
+// same bits in each of them; c is a sum or a maximum.  Within 16 lanes by lane
+// permutations (lane ^ 1, lane ^ 2, then mirrors, whose groups are uniform by
+// then), beyond by swaps of 16 or 32 lanes between two copies of the value.
+template<int TPS, typename T, class Combine>
+__device__ __forceinline__ T lanes_combine(T v, Combine c)
+{
+  constexpr int N=sizeof(T)/4;
+  auto words=[](T x) { return __builtin_bit_cast(Words<N>,x); };
+  auto value=[](Words<N> w) { return __builtin_bit_cast(T,w); };
+  auto permuted=[&](auto ctrl) {
+    Words<N> w=words(v);
+#pragma unroll
+    for(int i=0; i < N; ++i)
+      w.w[i]=(unsigned) __builtin_amdgcn_update_dpp(0,(int) w.w[i],decltype(ctrl)::value,0xF,0xF,true);
+    v=c(v,value(w));
+  };
+  auto swapped=[&](auto swap) {
+    const Words<N> w=words(v);
+    Words<N> a, b;
+#pragma unroll
+    for(int i=0; i < N; ++i) {
+      const auto s=swap(w.w[i]);
+      a.w[i]=s[0];
+      b.w[i]=s[1];
+    }
+    v=c(value(a),value(b));
+  };
+  if constexpr(TPS >= 2) permuted(std::integral_constant<int,0xB1>());
+  if constexpr(TPS >= 4) permuted(std::integral_constant<int,0x4E>());
+  if constexpr(TPS >= 8) permuted(std::integral_constant<int,0x141>());
+  if constexpr(TPS >= 16) permuted(std::integral_constant<int,0x140>());
+  if constexpr(TPS >= 32)
+    swapped([](unsigned u) { return __builtin_amdgcn_permlane16_swap(u,u,false,false); });
+  if constexpr(TPS >= 64)
+    swapped([](unsigned u) { return __builtin_amdgcn_permlane32_swap(u,u,false,false); });
+  return v;
+}
+
+// The same over the TPS threads of a slot of whole waves, through red (two
+// words for each of the block's waves) when it has several; one block barrier
+// then, and the next use takes other words.
+template<int TPS, typename T, class Combine>
+__device__ __forceinline__ void slot_combine(T &x, T &y, T *red, Combine c)
+{
+  x=lanes_combine<(TPS < 64 ? TPS : 64)>(x,c);
+  y=lanes_combine<(TPS < 64 ? TPS : 64)>(y,c);
+  if constexpr(TPS > 64) {
+    constexpr int W=TPS/64;
+    const int wave=__builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+    if((threadIdx.x & 63) == 0) {
+      red[2*wave]=x;
+      red[2*wave+1]=y;
+    }
+    __syncthreads();
+    const T *r=red+2*(wave & ~(W-1));
+    x=r[0];
+    y=r[1];
+#pragma unroll
+    for(int w=1; w < W; ++w) {
+      x=c(x,r[2*w]);
+      y=c(y,r[2*w+1]);
+    }
+  }
+}
+
+// The two factors of a Hermitian row share a transform, whose rounding errors
+// are relative to the larger one: exact powers of two bring them to one
+// magnitude first, 2^-ef F and 2^-eg G, whose norms then differ by at most a
+// factor sqrt(2).  near: ef = 0, only G is scaled.  Otherwise (far) both are, to
+// norms near 1.  (FP32, H = 128, q = 3, relative error of a row's product: F of
+// 1e-4 times G's magnitude 6e-4 unscaled, 2e-7 scaled or transformed apart.)
+struct RowScales {
+  int ef, eg;
+  bool near;     // the same over the wave, or over the block where slots span waves
+  bool zf, zg;   // far: a factor of zeros (its transform is 0, not the other's rounding errors)
+};
+
+// Squares of norms from 2^LO to 2^HI are near: their sums lose nothing that
+// matters to underflow, ratios of norms stay normal numbers and the transforms in
+// range.  2^-LIM and 2^LIM are normal numbers too.
+template<typename T> struct ScaleRange;
+template<> struct ScaleRange<double> { static constexpr int LO=-900, HI=900, LIM=1022; };
+template<> struct ScaleRange<float> { static constexpr int LO=-120, HI=120, LIM=126; };
+
+__device__ __forceinline__ int exponent(double v) { return __builtin_amdgcn_frexp_exp(v); }
+__device__ __forceinline__ int exponent(float v) { return __builtin_amdgcn_frexp_expf(v); }
+__device__ __forceinline__ double mantissa(double v) { return __builtin_amdgcn_frexp_mant(v); }
+__device__ __forceinline__ float mantissa(float v) { return __builtin_amdgcn_frexp_mantf(v); }
+__device__ __forceinline__ double scaled(double v, int e) { return __builtin_amdgcn_ldexp(v,e); }
+__device__ __forceinline__ float scaled(float v, int e) { return __builtin_amdgcn_ldexpf(v,e); }
+
+// The scales of a row, given its words a of f and b of g in this thread (each
+// word of the row in one thread of the slot).  red: 3 x 2 words per wave of the
+// block (slots of several waves).  Far rows take their whole wave along (or the
+// block, whose barriers all its threads must reach); their norms are summed
+// after a scaling by the largest magnitude.
+template<typename T, int M, int SLOTS>
+__device__ __forceinline__ RowScales row_scales(const cplx<T> *a, const cplx<T> *b, T *red)
+{
+  constexpr int V=RowV::V, TPS=M/V, WAVES=(SLOTS*TPS+63)/64;
+  typedef ScaleRange<T> SR;
+  static_assert(TPS <= 64 || SLOTS <= 2,"every slot of the block is looked at");
+  auto add=[](T x, T y) { return x+y; };
+  T x=0, y=0;
+#pragma unroll
+  for(int k=0; k < V; ++k) {
+    x=fma(a[k].x,a[k].x,fma(a[k].y,a[k].y,x));
+    y=fma(b[k].x,b[k].x,fma(b[k].y,b[k].y,y));
+  }
+  slot_combine<TPS>(x,y,red,add);
+  const T lo=scaled((T) 1,SR::LO), hi=scaled((T) 1,SR::HI);
+  auto outside=[&](T u, T v) { return !(u >= lo && u <= hi && v >= lo && v <= hi); };
+  bool far=outside(x,y);                 // zeros too: they may be squares that vanished
+  if constexpr(TPS > 64 && SLOTS == 2) {
+    const int wave=(int) threadIdx.x >> 6;
+    const T *r=red+2*((wave & (WAVES/2)) ^ (WAVES/2));    // the other slot
+    T u=r[0], v=r[1];
+#pragma unroll
+    for(int w=1; w < TPS/64; ++w) {
+      u=u+r[2*w];
+      v=v+r[2*w+1];
+    }
+    far=far || outside(u,v);
+  }
+  RowScales s={0,0,true,false,false};
+  if(__any(far)) {
+    const T top=std::numeric_limits<T>::max();
+    T mx=0, my=0;
+#pragma unroll
+    for(int k=0; k < V; ++k) {
+      mx=fmax(mx,fmax(fabs(a[k].x),fabs(a[k].y)));
+      my=fmax(my,fmax(fabs(b[k].x),fabs(b[k].y)));
+    }
+    slot_combine<TPS>(mx,my,red+2*WAVES,[](T u, T v) { return fmax(u,v); });
+    const int px=mx > 0 && mx <= top ? exponent(mx) : 0, py=my > 0 && my <= top ? exponent(my) : 0;
+    x=y=0;
+#pragma unroll
+    for(int k=0; k < V; ++k) {
+      const T fx=scaled(a[k].x,-px), fy=scaled(a[k].y,-px), gx=scaled(b[k].x,-py), gy=scaled(b[k].y,-py);
+      x=fma(fx,fx,fma(fy,fy,x));
+      y=fma(gx,gx,fma(gy,gy,y));
+    }
+    slot_combine<TPS>(x,y,red+4*WAVES,add);
+    // a factor of zeros, or with Inf or NaN, takes the other's scale
+    s.near=false;
+    s.zf=x == 0;
+    s.zg=y == 0;
+    const bool vf=x > 0 && x <= top, vg=y > 0 && y <= top;
+    s.ef=vf ? px+(exponent(x) >> 1) : (vg ? py+(exponent(y) >> 1) : 0);
+    s.eg=s.ef;
+    if(vf && vg) {
+      const int d=exponent(y)-exponent(x)+2*(py-px);
+      s.eg=s.ef+((d+(mantissa(y) >= mantissa(x) ? 1 : 0)) >> 1);
+    }
+    s.ef=min(max(s.ef,-SR::LIM),SR::LIM);
+    s.eg=min(max(s.eg,-SR::LIM),SR::LIM);
+  } else
+    // log2 of |g|/|f| rounded: half of the difference of the squares'
+    // exponents, up where that is odd and the mantissas make up the rest
+    s.eg=(exponent(y)-exponent(x)+(mantissa(y) >= mantissa(x) ? 1 : 0)) >> 1;
+  if constexpr(TPS >= 64) {              // the same over the wave: scalar registers
+    s.ef=__builtin_amdgcn_readfirstlane(s.ef);
+    s.eg=__builtin_amdgcn_readfirstlane(s.eg);
+    s.zf=__builtin_amdgcn_readfirstlane(s.zf);
+    s.zg=__builtin_amdgcn_readfirstlane(s.zg);
+  }
+  return s;
+}
+
 // Residues r1 and r2 of the f + i g pair of a Hermitian row (H <= M), folded
 // for the forward transform from one read of the row: X1[k] = U_r1(sigma),
 // X2[k] = U_r2(sigma) at sigma = t + TPS k, with
@@ -331,14 +505,18 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
 //   u(sigma) = f(sigma) + i g(sigma)                    (sigma < H),
 //   v(sigma) = conj f(M - sigma) + i conj g(M - sigma)  (M - sigma < H),
 // the wavenumbers k = sigma and sigma - M of the block (f(-k) = conj f(k),
-// w_N^{(sigma - M) r} = w_N^{sigma r} w_q^{-r}).  rf, rg: buffers over the
-// row's H words; tr[k] = w_N^{TPS k r}, tr[V] = w_N^{M r} (LDS); b = w_N^{t r}.
-// Out-of-range words read zero, past the end of the buffers (no branches).
+// w_N^{(sigma - M) r} = w_N^{sigma r} w_q^{-r}); f and g stand for the row's
+// factors scaled by 2^-ef and 2^-eg (RowScales).  fu, gu: the words sigma, of
+// which g's still take the factor su; sf, sg: the factors of the words M - sigma,
+// read from rf, rg, the buffers, at byte offset ro; tr[k] = w_N^{TPS k r}, tr[V] =
+// w_N^{M r} (LDS); b = w_N^{t r}.  Out-of-range words read zero, past the end of
+// the buffers (no branches).
 template<typename T, int M>
-__device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buffer_rsrc_t rf,
+__device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, const cplx<T> *fu,
+                                          const cplx<T> *gu, __amdgpu_buffer_rsrc_t rf,
                                           __amdgpu_buffer_rsrc_t rg, const cplx<T> *tr1,
                                           const cplx<T> *tr2, cplx<T> b1, cplx<T> b2, int t,
-                                          int r1, int r2, int H, unsigned ro)
+                                          int r1, int r2, int H, unsigned ro, T sf, T sg, T su)
 {
   constexpr int V=RowV::V, TPS=M/V;
   constexpr unsigned E=sizeof(cplx<T>), END=0x80000000u;
@@ -346,10 +524,10 @@ __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buf
 #pragma unroll
   for(int k=0; k < V; ++k) {
     const int sigma=t+TPS*k;
-    const unsigned ou=sigma < H ? ro+(unsigned) sigma*E : END, ov=M-sigma < H ? ro+(unsigned) (M-sigma)*E : END;
-    const cplx<T> fu=ld_buf<T>(rf,ou,0), gu=ld_buf<T>(rg,ou,0);
+    const unsigned ov=M-sigma < H ? ro+(unsigned) (M-sigma)*E : END;
     const cplx<T> fv=ld_buf<T>(rf,ov,0), gv=ld_buf<T>(rg,ov,0);
-    const cplx<T> u=mk(fu.x-gu.y,fu.y+gu.x), v=mk(fv.x+gv.y,gv.x-fv.y);
+    const cplx<T> u=mk(fma(-su,gu[k].y,fu[k].x),fma(su,gu[k].x,fu[k].y));
+    const cplx<T> v=mk(fma(sg,gv.y,sf*fv.x),fma(sg,gv.x,-sf*fv.y));
     cplx<T> a=u+c1*v, b=u+c2*v;
     if(r1) a=(b1*tr1[k])*a;
     if(r2) b=(b2*tr2[k])*b;
@@ -370,28 +548,41 @@ __device__ __forceinline__ void hpk_fold2(cplx<T> *X1, cplx<T> *X2, __amdgpu_buf
 // rowreg_kernel (backward2, convolve.cc:4749-4843): q forward and ceil(q/2)
 // inverse transforms per row instead of 3 ceil(q/2).  Rows are read through
 // buffer resources (a 32-bit offset per element; over one row when a slot is
-// whole waves, else over the block's rows with the row's offset per lane) and the uniform residue
-// twiddles w_N^{TPS k r} come from an LDS table, which keeps addresses and
-// twiddles out of the registers that the residue loop carries.  Slots past
-// the last row run on row rows - 1 without storing (the block barriers of the
-// transforms need every thread).  Dynamic LDS: hrowpk_lds().
+// whole waves, else over the block's rows with the row's offset per lane) and
+// the uniform residue twiddles w_N^{TPS k r} come from an LDS table, which keeps
+// addresses and twiddles out of the registers that the residue loop carries.
+// A row's words sigma are loaded ahead of its pairs: the first loads also give the
+// norms by which the factors are scaled (RowScales), which takes 4 to 8% (3072
+// rows of H = 1024, q = 3, FP64 80.5 -> 84.2 us, 73728 of 128 182 -> 187 us; with the
+// words read again for the first pair 87 and 188 us; both factors scaled at every
+// element instead of one 89.5 us).  Slots past the last row run on row rows - 1
+// without storing (the block barriers of the transforms need every thread).
+// Dynamic LDS: hrowpk_lds().
 template<typename T, int M>
 struct HRowPk {
   static constexpr int V=RowV::V;
   static constexpr int TPS=M/V;
   static constexpr int SLOTS=256/TPS > 0 ? 256/TPS : 1;
   static constexpr int NT=SLOTS*TPS;
-  // waves per SIMD that fit without spills (150 to 158 and 90 registers)
+  // waves per SIMD that fit without spills (157 to 168 and 90 to 100 registers)
   static constexpr int W=sizeof(T) == 4 ? 4 : 3;
   typedef SplitTw<T,M,V,2048> ST;           // at 2048 the table leaves two blocks
+  static constexpr int RED=TPS > 64 ? 3*2*NT/64 : 0;  // words of row_scales
 };
 
 template<typename T, int M>
 inline size_t hrowpk_lds(int q)
 {
   typedef HRowPk<T,M> K;
-  return (size_t) (K::ST::LDS+q*(K::V+1))*sizeof(cplx<T>)+(size_t) K::SLOTS*2*RPlan<M,K::V>::PAD*sizeof(T);
+  return (size_t) (K::ST::LDS+q*(K::V+1))*sizeof(cplx<T>)+
+    ((size_t) K::SLOTS*2*RPlan<M,K::V>::PAD+K::RED)*sizeof(T);
 }
+
+// Products that are a factor of F times one of G: the scales of a row's
+// factors may be undone on the results.
+template<class Op> struct IsProduct { static constexpr bool value=false; };
+template<> struct IsProduct<RunMult> { static constexpr bool value=true; };
+template<int MULT> struct IsProduct<LibMult<MULT>> { static constexpr bool value=true; };
 
 template<typename T, int M, class Op>
 __global__ void __launch_bounds__((HRowPk<T,M>::NT),(HRowPk<T,M>::W))
@@ -418,7 +609,8 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
   int slot=(int) threadIdx.x/TPS;
   if constexpr(TPS >= 64) slot=__builtin_amdgcn_readfirstlane(slot);
   const int t=threadIdx.x-slot*TPS;
-  T *xb=reinterpret_cast<T *>(tq+q*(V+1))+slot*2*P::PAD;
+  T *xbase=reinterpret_cast<T *>(tq+q*(V+1));
+  T *xb=xbase+slot*2*P::PAD;
   for(int64_t rb=(int64_t) blockIdx.x*SLOTS; rb < rows; rb += (int64_t) gridDim.x*SLOTS) {
     const int64_t row=rb+slot;
     const bool live=row < rows;
@@ -429,11 +621,38 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
     const size_t nw=TPS >= 64 ? (size_t) H : (size_t) ((rows-1 < rb+SLOTS-1 ? rows-1-rb : SLOTS-1)*rs+H);
     const unsigned ro=TPS >= 64 ? 0 : (unsigned) ((rr-rb)*rs)*E;
     const __amdgpu_buffer_rsrc_t rf=buf_rsrc(f+b0*rs,nw), rg=buf_rsrc(g+b0*rs,nw);
+    // the row's words sigma = t + TPS k
+    cplx<T> fu[V], gu[V];
+    auto load=[&](int ts) {
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        const unsigned o=ts+TPS*k < H ? ro+(unsigned) (ts+TPS*k)*E : 0x80000000u;  // past the end: 0
+        fu[k]=ld_buf<T>(rf,o,0);
+        gu[k]=ld_buf<T>(rg,o,0);
+      }
+    };
+    auto prescale=[&](const RowScales &s) {
+      if(s.near) return;                 // hpk_fold2 scales g
+#pragma unroll
+      for(int k=0; k < V; ++k) {
+        fu[k]=mk(scaled(fu[k].x,-s.ef),scaled(fu[k].y,-s.ef));
+        gu[k]=mk(scaled(gu[k].x,-s.eg),scaled(gu[k].y,-s.eg));
+      }
+    };
+    load(fresh(t));
+    const RowScales sc=row_scales<T,M,SLOTS>(fu,gu,xbase+SLOTS*2*P::PAD);
+    prescale(sc);
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
-    const auto rop=bind_row(op,row);
-    for(int r1=0; r1 < q; r1 += 2) {
+    const auto bound=bind_row(op,row);
+    // the product of the unscaled transforms; of far rows, where it is a factor
+    // of each, the scales are undone on the results
+    auto rop=[&](T F, T G, int l) {
+      if constexpr(IsProduct<Op>::value) return bound(F,sc.near ? scaled(G,sc.eg) : G,l);
+      else return bound(sc.zf ? (T) 0*F : scaled(F,sc.ef),sc.zg ? (T) 0*G : scaled(G,sc.eg),l);
+    };
+    for(int r1=0;;) {
       const int r2=r1+1 < q ? r1+1 : -1;
       // the loop's own positions too (see fresh())
       const int ti=fresh(t);
@@ -441,8 +660,10 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
       // both residues folded from one read of the row
       cplx<T> X[V], X2[V];
       T p1[V];
-      hpk_fold2<T,M>(X,X2,rf,rg,tq+r1*(V+1),tq+(r2 >= 0 ? r2 : r1)*(V+1),b1,
-                       r2 >= 0 ? zN[ti*r2] : b1,ti,r1,r2 >= 0 ? r2 : r1,H,ro);
+      const T sg=scaled((T) 1,-fresh(sc.eg));
+      hpk_fold2<T,M>(X,X2,fu,gu,rf,rg,tq+r1*(V+1),tq+(r2 >= 0 ? r2 : r1)*(V+1),b1,
+                     r2 >= 0 ? zN[ti*r2] : b1,ti,r1,r2 >= 0 ? r2 : r1,H,ro,
+                     scaled((T) 1,-fresh(sc.ef)),sg,sc.near ? sg : (T) 1);
       if(r2 >= 0) {
         // the two residues' transforms with their butterflies interleaved
         fftr_pair<T,M,V,1>(X,X2,xb,tw,t);
@@ -477,19 +698,31 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
         acc[k]=acc[k]+v;
       }
       rsync<TPS>();
+      r1 += 2;
+      if(r1 >= q) break;
+      load(fresh(t));
+      prescale(sc);
     }
     if(live) {
       const int to=fresh(t);
+#pragma unroll
+      for(int k=0; k < V; ++k) acc[k]=scale*acc[k];
+      if(IsProduct<Op>::value && !sc.near) {
+        const int e=sc.ef+sc.eg;
+        const T z=sc.zf || sc.zg ? (T) 0 : (T) 1;
+#pragma unroll
+        for(int k=0; k < V; ++k) acc[k]=mk(scaled(z*acc[k].x,e),scaled(z*acc[k].y,e));
+      }
       if constexpr(TPS >= 64) {
         const __amdgpu_buffer_rsrc_t rw=buf_rsrc(out+row*os,H);
 #pragma unroll
         for(int k=0; k < V; ++k)
-          if(to+TPS*k < H) st_buf<T>(rw,(unsigned) (to+TPS*k)*E,0,scale*acc[k]);
+          if(to+TPS*k < H) st_buf<T>(rw,(unsigned) (to+TPS*k)*E,0,acc[k]);
       } else {
         cplx<T> *orow=out+row*os;
 #pragma unroll
         for(int k=0; k < V; ++k)
-          if(to+TPS*k < H) orow[to+TPS*k]=scale*acc[k];
+          if(to+TPS*k < H) orow[to+TPS*k]=acc[k];
       }
     }
   }
