@@ -53,7 +53,7 @@ __device__ __forceinline__ cplx<T> muli(cplx<T> a, int sign)
 // the product of the two transformed inputs at padded index l = q s + r of
 // row `row` of the row stage; op(u, v, row, l) on two reals is the product of
 // one residue of Hermitian rows, whose transforms are real (realMultBinary).
-// The kernels call it through bind_row (below) once per row.
+// The kernels call it for rows that exist, bound by bind_row (below) once per row.
 // LibMult<MULT>: multNone (0), multBinary (1), multcorrelation (3) fixed at
 // compile time; RunMult: the same chosen at run time.  A caller's functor with
 // these two members runs in the same kernels (fused user multipliers).
@@ -107,6 +107,12 @@ struct RunMult {
   template<typename T>
   __device__ __forceinline__ T operator()(T a, T b, int64_t, int) const { return a*b; }
 };
+
+// The library's products: a factor of F times one of G, which the kernels may
+// also evaluate on the empty slots of a block, and scale before or after.
+template<class Op> struct IsProduct { static constexpr bool value=false; };
+template<> struct IsProduct<RunMult> { static constexpr bool value=true; };
+template<int MULT> struct IsProduct<LibMult<MULT>> { static constexpr bool value=true; };
 
 // Geometry of one padded dimension as seen by a kernel.
 constexpr int MAXSTAGES=24;

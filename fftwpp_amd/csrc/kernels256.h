@@ -227,6 +227,7 @@ rowconv256_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
       b0[k]=in ? (gr+16*k)[lin] : zero<T>();
     }
   }
+  const auto rop=bind_row(op,ok ? row0+i : rows-1);
   for(int r=0; r < qi; ++r) {
     const cplx<T> *rt=rtab+256*r;
     cplx<T> a[16], b[16];
@@ -251,8 +252,7 @@ rowconv256_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
     }
     fft256s<T,1,1>(a,row,j,0,tw16);
     fft256s<T,1,1>(b,row,j,0,tw16);
-    {
-      const auto rop=bind_row(op,row0+i);
+    if(IsProduct<Op>::value || ok) {
 #pragma unroll
       for(int k=0; k < 16; ++k) a[k]=rop(a[k],b[k],qi*(j+16*k)+r);
     }
@@ -359,8 +359,8 @@ rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
       b[k]=b[k]*w;
     }
     fft256s_pair<T,1,1,RS>(a,b,xrow,j,0,tw16);
-    {
-      const auto rop=bind_row(op,row);
+    if(IsProduct<Op>::value || ok) {
+      const auto rop=bind_row(op,ok ? row : rows-1);
 #pragma unroll
       for(int k=0; k < 16; ++k) a[k]=rop(a[k],b[k],2*(j+16*k)+r);
     }

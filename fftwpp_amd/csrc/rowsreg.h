@@ -140,6 +140,7 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
   __syncthreads();
   for(; rb < rows; rb += step) {
     const int64_t row=rb+rslot;
+    const auto rop=bind_row(op,row0+(row < rows ? row : rows-1));
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
@@ -177,9 +178,10 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
           for(int k=0; k < V; ++k) X[k]=mulc(X[k],Y[k]);
         }
       } else {
-        const auto rop=bind_row(op,row0+row);
+        if(IsProduct<Op>::value || (on && row < rows)) {
 #pragma unroll
-        for(int k=0; k < V; ++k) X[k]=rop(X[k],Y[k],q*(t+TPS*k)+r);
+          for(int k=0; k < V; ++k) X[k]=rop(X[k],Y[k],q*(t+TPS*k)+r);
+        }
       }
       fftr<T,M,V,-1,true>(X,xb,tw,t);
 #pragma unroll
@@ -240,6 +242,7 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
+    const auto rop=bind_row(op,row);
     // the same number of passes in every lane, as in rowcx_kernel
     for(int p0=0; p0 < q; p0 += 2*RP) {
       const bool on=RP == 1 || p0+2*rp < q;
@@ -273,8 +276,7 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
       }
       fftr<T,M,V,1,true>(X,xb,tw,t);
       fftr<T,M,V,1,true>(Y,xb,tw,t);
-      {
-        const auto rop=bind_row(op,row);
+      if(IsProduct<Op>::value || on) {
 #pragma unroll
         for(int k=0; k < V; ++k) {
           const int l=q*(t+TPS*k);
@@ -578,12 +580,6 @@ inline size_t hrowpk_lds(int q)
     ((size_t) K::SLOTS*2*RPlan<M,K::V>::PAD+K::RED)*sizeof(T);
 }
 
-// Products that are a factor of F times one of G: the scales of a row's
-// factors may be undone on the results.
-template<class Op> struct IsProduct { static constexpr bool value=false; };
-template<> struct IsProduct<RunMult> { static constexpr bool value=true; };
-template<int MULT> struct IsProduct<LibMult<MULT>> { static constexpr bool value=true; };
-
 template<typename T, int M, class Op>
 __global__ void __launch_bounds__((HRowPk<T,M>::NT),(HRowPk<T,M>::W))
 hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
@@ -645,11 +641,12 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
-    const auto bound=bind_row(op,row);
+    const auto bound=bind_row(op,rr);
     // the product of the unscaled transforms; of far rows, where it is a factor
     // of each, the scales are undone on the results
     auto rop=[&](T F, T G, int l) {
       if constexpr(IsProduct<Op>::value) return bound(F,sc.near ? scaled(G,sc.eg) : G,l);
+      else if(!live) return F;
       else return bound(sc.zf ? (T) 0*F : scaled(F,sc.ef),sc.zg ? (T) 0*G : scaled(G,sc.eg),l);
     };
     for(int r1=0;;) {

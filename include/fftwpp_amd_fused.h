@@ -29,7 +29,10 @@
  * fftwpp_amd_rows_args).  Work that depends on the row alone belongs in an
  * optional member `__device__ R at(int64_t row) const`: the kernels then call
  * at(row) once per row and R's operator()(F, G, l) (complex and real forms)
- * for every element.  Multipliers on Hermitian or real plans must keep
+ * for every element.  Only rows that exist are asked for, 0 <= row < rows (of
+ * fftwpp_amd_rows_args): both members may read tables of one entry per row, and
+ * the products are called once for every (row, l); an empty slot of a last
+ * block may bind at(rows - 1) once more.  Multipliers on Hermitian or real plans must keep
  * the conjugate symmetry of the data (a product weighted by a function of
  * |k| in every dimension does).  Row geometries outside the register row
  * kernels (power-of-two m in [16, 4096] covering the row) are refused with

@@ -66,7 +66,54 @@ struct Binary {
   __device__ T operator()(T F, T G, int64_t, int) const { return F*G; }
 };
 
+// w[row] F G: a table of one weight per row.  bound[row] is set when a row is
+// bound, calls[row] counts the products of the row.
+struct RowTable {
+  const double *w;
+  int *bound, *calls;
+
+  struct Row {
+    double w;
+    int *calls;
+    template<typename T>
+    __device__ fftwpp_amd::cplx<T> operator()(fftwpp_amd::cplx<T> F, fftwpp_amd::cplx<T> G,
+                                             int) const
+    {
+      atomicAdd(calls,1);
+      return (T) w*(F*G);
+    }
+    template<typename T>
+    __device__ T operator()(T F, T G, int) const
+    {
+      atomicAdd(calls,1);
+      return (T) w*(F*G);
+    }
+  };
+  __device__ Row at(int64_t row) const
+  {
+    bound[row]=1;
+    return Row{w[row],calls+row};
+  }
+  template<typename T>
+  __device__ fftwpp_amd::cplx<T> operator()(fftwpp_amd::cplx<T> F, fftwpp_amd::cplx<T> G,
+                                           int64_t row, int l) const
+  {
+    return at(row)(F,G,l);
+  }
+  template<typename T>
+  __device__ T operator()(T F, T G, int64_t row, int l) const { return at(row)(F,G,l); }
+};
+
 } // namespace
+
+// out <- a (*) b with the product of each row weighted by the row's table entry;
+// row sizes m = 16, 128, 256 and 1024.
+extern "C" int fusedmult_table(fftwpp_amd_conv *h, void *out, const void *a, const void *b,
+                               const double *w, int *bound, int *calls, void *stream)
+{
+  return fftwpp_amd::conv_execute_fused(h,out,a,b,RowTable{w,bound,calls},stream,
+                                        fftwpp_amd::FusedSet<0x59u>());
+}
 
 extern "C" int fusedmult_binary(fftwpp_amd_conv *h, void *out, const void *a,
                                 const void *b, void *stream)
