@@ -53,7 +53,8 @@ __device__ __forceinline__ cplx<T> muli(cplx<T> a, int sign)
 // the product of the two transformed inputs at padded index l = q s + r of
 // row `row` of the row stage; op(u, v, row, l) on two reals is the product of
 // one residue of Hermitian rows, whose transforms are real (realMultBinary).
-// The kernels call it for rows that exist, bound by bind_row (below) once per row.
+// The kernels bind it (bind_row, below) to rows that exist, once per row and
+// residue pass at most; empty slots of a last block take the last row.
 // LibMult<MULT>: multNone (0), multBinary (1), multcorrelation (3) fixed at
 // compile time; RunMult: the same chosen at run time.  A caller's functor with
 // these two members runs in the same kernels (fused user multipliers).
@@ -70,7 +71,7 @@ template<int MULT> struct LibMult {
 };
 
 // A product functor bound to one row: op.at(row) when Op provides it (the
-// functor's work that depends on the row alone, done once per row), else a
+// functor's work that depends on the row alone), else a
 // wrapper that passes the row to every call.  Either way rop(F, G, l).
 template<class Op> struct RowBound {
   Op op;
@@ -108,8 +109,8 @@ struct RunMult {
   __device__ __forceinline__ T operator()(T a, T b, int64_t, int) const { return a*b; }
 };
 
-// The library's products: a factor of F times one of G, which the kernels may
-// also evaluate on the empty slots of a block, and scale before or after.
+// The library's products: a factor of F times one of G, so that scales of the
+// factors may be undone on the product.
 template<class Op> struct IsProduct { static constexpr bool value=false; };
 template<> struct IsProduct<RunMult> { static constexpr bool value=true; };
 template<int MULT> struct IsProduct<LibMult<MULT>> { static constexpr bool value=true; };

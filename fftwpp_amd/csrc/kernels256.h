@@ -227,7 +227,6 @@ rowconv256_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
       b0[k]=in ? (gr+16*k)[lin] : zero<T>();
     }
   }
-  const auto rop=bind_row(op,ok ? row0+i : rows-1);
   for(int r=0; r < qi; ++r) {
     const cplx<T> *rt=rtab+256*r;
     cplx<T> a[16], b[16];
@@ -252,7 +251,8 @@ rowconv256_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
     }
     fft256s<T,1,1>(a,row,j,0,tw16);
     fft256s<T,1,1>(b,row,j,0,tw16);
-    if(IsProduct<Op>::value || ok) {
+    {
+      const auto rop=bind_row(op,ok ? row0+i : rows-1);
 #pragma unroll
       for(int k=0; k < 16; ++k) a[k]=rop(a[k],b[k],qi*(j+16*k)+r);
     }
@@ -306,10 +306,12 @@ __device__ __forceinline__ double pair16_scatter(double x, double y)
 // instructions per row pair, at four cycles each on one of 1024 SIMDs): the
 // branches around every load and store and the sum of all sixteen outputs in
 // both groups were an eighth of them.  262144 rows of 256: FP64 778 -> 705 us,
-// FP32 392 -> 376 us.
+// FP32 392 -> 376 us (four waves per SIMD with the library's products; a caller's
+// functor keeps the registers of two: the tests' weight 1/(1 + c k^2) spilled 284
+// bytes at four and took 666 to 712 us, 525 us at two).
 // Dynamic LDS: row256_lds(4 WPB, 2).
 template<typename T, class Op, int WPB>
-__global__ void __launch_bounds__(64*WPB,sizeof(T) == 4 ? 4 : 2)
+__global__ void __launch_bounds__(64*WPB,(sizeof(T) == 4 && IsProduct<Op>::value ? 4 : 2))
 rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
                    int64_t rs, cplx<T> *out, int64_t os, int L, T scale,
                    const cplx<T> *zN, Op op)
@@ -359,7 +361,7 @@ rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
       b[k]=b[k]*w;
     }
     fft256s_pair<T,1,1,RS>(a,b,xrow,j,0,tw16);
-    if(IsProduct<Op>::value || ok) {
+    {
       const auto rop=bind_row(op,ok ? row : rows-1);
 #pragma unroll
       for(int k=0; k < 16; ++k) a[k]=rop(a[k],b[k],2*(j+16*k)+r);

@@ -140,7 +140,6 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
   __syncthreads();
   for(; rb < rows; rb += step) {
     const int64_t row=rb+rslot;
-    const auto rop=bind_row(op,row0+(row < rows ? row : rows-1));
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
@@ -178,10 +177,9 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
           for(int k=0; k < V; ++k) X[k]=mulc(X[k],Y[k]);
         }
       } else {
-        if(IsProduct<Op>::value || (on && row < rows)) {
+        const auto rop=bind_row(op,row0+(row < rows ? row : rows-1));
 #pragma unroll
-          for(int k=0; k < V; ++k) X[k]=rop(X[k],Y[k],q*(t+TPS*k)+r);
-        }
+        for(int k=0; k < V; ++k) X[k]=rop(X[k],Y[k],q*(t+TPS*k)+r);
       }
       fftr<T,M,V,-1,true>(X,xb,tw,t);
 #pragma unroll
@@ -242,7 +240,6 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
     cplx<T> acc[V];
 #pragma unroll
     for(int k=0; k < V; ++k) acc[k]=mk((T) 0,(T) 0);
-    const auto rop=bind_row(op,row);
     // the same number of passes in every lane, as in rowcx_kernel
     for(int p0=0; p0 < q; p0 += 2*RP) {
       const bool on=RP == 1 || p0+2*rp < q;
@@ -276,7 +273,8 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
       }
       fftr<T,M,V,1,true>(X,xb,tw,t);
       fftr<T,M,V,1,true>(Y,xb,tw,t);
-      if(IsProduct<Op>::value || on) {
+      {
+        const auto rop=bind_row(op,row);
 #pragma unroll
         for(int k=0; k < V; ++k) {
           const int l=q*(t+TPS*k);
@@ -405,8 +403,9 @@ __device__ __forceinline__ void slot_combine(T &x, T &y, T *red, Combine c)
 struct RowScales {
   int ef, eg;
   bool near;     // the same over the wave, or over the block where slots span waves
-  bool zf, zg;   // far: a factor of zeros (its transform is 0, not the other's rounding errors)
 };
+// ef or eg of a factor of zeros: undone, it makes 0 of the other's rounding errors
+constexpr int ZEROS=-10000;
 
 // Squares of norms from 2^LO to 2^HI are near: their sums lose nothing that
 // matters to underflow, ratios of norms stay normal numbers and the transforms in
@@ -455,7 +454,7 @@ __device__ __forceinline__ RowScales row_scales(const cplx<T> *a, const cplx<T> 
     }
     far=far || outside(u,v);
   }
-  RowScales s={0,0,true,false,false};
+  RowScales s={0,0,true};
   if(__any(far)) {
     const T top=std::numeric_limits<T>::max();
     T mx=0, my=0;
@@ -476,8 +475,6 @@ __device__ __forceinline__ RowScales row_scales(const cplx<T> *a, const cplx<T> 
     slot_combine<TPS>(x,y,red+4*WAVES,add);
     // a factor of zeros, or with Inf or NaN, takes the other's scale
     s.near=false;
-    s.zf=x == 0;
-    s.zg=y == 0;
     const bool vf=x > 0 && x <= top, vg=y > 0 && y <= top;
     s.ef=vf ? px+(exponent(x) >> 1) : (vg ? py+(exponent(y) >> 1) : 0);
     s.eg=s.ef;
@@ -485,8 +482,8 @@ __device__ __forceinline__ RowScales row_scales(const cplx<T> *a, const cplx<T> 
       const int d=exponent(y)-exponent(x)+2*(py-px);
       s.eg=s.ef+((d+(mantissa(y) >= mantissa(x) ? 1 : 0)) >> 1);
     }
-    s.ef=min(max(s.ef,-SR::LIM),SR::LIM);
-    s.eg=min(max(s.eg,-SR::LIM),SR::LIM);
+    s.ef=x == 0 ? ZEROS : min(max(s.ef,-SR::LIM),SR::LIM);
+    s.eg=y == 0 ? ZEROS : min(max(s.eg,-SR::LIM),SR::LIM);
   } else
     // log2 of |g|/|f| rounded: half of the difference of the squares'
     // exponents, up where that is odd and the mantissas make up the rest
@@ -494,8 +491,6 @@ __device__ __forceinline__ RowScales row_scales(const cplx<T> *a, const cplx<T> 
   if constexpr(TPS >= 64) {              // the same over the wave: scalar registers
     s.ef=__builtin_amdgcn_readfirstlane(s.ef);
     s.eg=__builtin_amdgcn_readfirstlane(s.eg);
-    s.zf=__builtin_amdgcn_readfirstlane(s.zf);
-    s.zg=__builtin_amdgcn_readfirstlane(s.zg);
   }
   return s;
 }
@@ -566,8 +561,10 @@ struct HRowPk {
   static constexpr int TPS=M/V;
   static constexpr int SLOTS=256/TPS > 0 ? 256/TPS : 1;
   static constexpr int NT=SLOTS*TPS;
-  // waves per SIMD that fit without spills (157 to 168 and 90 to 100 registers)
-  static constexpr int W=sizeof(T) == 4 ? 4 : 3;
+  // waves per SIMD that fit without spills with the library's products (157 to
+  // 168 and 90 to 100 registers); a caller's functor keeps the registers of two
+  // (the tests' weight 1/(1 + c k^2), 73728 rows of H = 128, FP64: 254 us with three, 246)
+  static constexpr int W=sizeof(T) == 4 ? 4 : 3, WF=2;
   typedef SplitTw<T,M,V,2048> ST;           // at 2048 the table leaves two blocks
   static constexpr int RED=TPS > 64 ? 3*2*NT/64 : 0;  // words of row_scales
 };
@@ -581,7 +578,7 @@ inline size_t hrowpk_lds(int q)
 }
 
 template<typename T, int M, class Op>
-__global__ void __launch_bounds__((HRowPk<T,M>::NT),(HRowPk<T,M>::W))
+__global__ void __launch_bounds__((HRowPk<T,M>::NT),(IsProduct<Op>::value ? HRowPk<T,M>::W : HRowPk<T,M>::WF))
 hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64_t rs,
               cplx<T> *out, int64_t os, T scale, Op op)
 {
@@ -646,8 +643,7 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
     // of each, the scales are undone on the results
     auto rop=[&](T F, T G, int l) {
       if constexpr(IsProduct<Op>::value) return bound(F,sc.near ? scaled(G,sc.eg) : G,l);
-      else if(!live) return F;
-      else return bound(sc.zf ? (T) 0*F : scaled(F,sc.ef),sc.zg ? (T) 0*G : scaled(G,sc.eg),l);
+      else return bound(scaled(F,sc.ef),scaled(G,sc.eg),l);
     };
     for(int r1=0;;) {
       const int r2=r1+1 < q ? r1+1 : -1;
@@ -657,10 +653,12 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
       // both residues folded from one read of the row
       cplx<T> X[V], X2[V];
       T p1[V];
-      const T sg=scaled((T) 1,-fresh(sc.eg));
+      // (2^-ZEROS is Inf, which a zero must not meet)
+      const T sf=scaled((T) 1,-max(fresh(sc.ef),-ScaleRange<T>::LIM));
+      const T sg=scaled((T) 1,-max(fresh(sc.eg),-ScaleRange<T>::LIM));
       hpk_fold2<T,M>(X,X2,fu,gu,rf,rg,tq+r1*(V+1),tq+(r2 >= 0 ? r2 : r1)*(V+1),b1,
                      r2 >= 0 ? zN[ti*r2] : b1,ti,r1,r2 >= 0 ? r2 : r1,H,ro,
-                     scaled((T) 1,-fresh(sc.ef)),sg,sc.near ? sg : (T) 1);
+                     sf,sg,sc.near ? sg : (T) 1);
       if(r2 >= 0) {
         // the two residues' transforms with their butterflies interleaved
         fftr_pair<T,M,V,1>(X,X2,xb,tw,t);
@@ -705,10 +703,8 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
 #pragma unroll
       for(int k=0; k < V; ++k) acc[k]=scale*acc[k];
       if(IsProduct<Op>::value && !sc.near) {
-        const int e=sc.ef+sc.eg;
-        const T z=sc.zf || sc.zg ? (T) 0 : (T) 1;
 #pragma unroll
-        for(int k=0; k < V; ++k) acc[k]=mk(scaled(z*acc[k].x,e),scaled(z*acc[k].y,e));
+        for(int k=0; k < V; ++k) acc[k]=mk(scaled(acc[k].x,sc.ef+sc.eg),scaled(acc[k].y,sc.ef+sc.eg));
       }
       if constexpr(TPS >= 64) {
         const __amdgpu_buffer_rsrc_t rw=buf_rsrc(out+row*os,H);
