@@ -22,6 +22,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -900,15 +901,48 @@ static ColArrays col_arrays(const void *in, void *out)
   return io;
 }
 
+// Words from the first to past the last one of nbatch sets of C columns of n
+// elements (strides bs, cs, S).
+static size_t col_span(size_t n, size_t S, size_t C, size_t cs, size_t nbatch, size_t bs)
+{
+  return n == 0 ? 0 : (n-1)*S+(C-1)*cs+(nbatch-1)*bs+1;
+}
+
+// Whether an input of `in` bytes and an output of `out` bytes share memory.
+static bool col_overlap(const ColArrays &io, size_t in, size_t out)
+{
+  for(int a=0; a < io.n; ++a)
+    for(int b=0; b < io.n; ++b) {
+      const uintptr_t f=(uintptr_t) io.in[a], F=(uintptr_t) io.out[b];
+      if(f < F+out && F < f+in) return true;
+    }
+  return false;
+}
+
+// Compute units of the current device (256 when it cannot be asked).
+static size_t device_cus()
+{
+  static std::atomic<int> known[64];
+  int dev=0, cus=0;
+  if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if((cus=known[dev].load(std::memory_order_relaxed))) return (size_t) cus;
+  if(hipDeviceGetAttribute(&cus,hipDeviceAttributeMultiprocessorCount,dev) != hipSuccess || cus < 1)
+    return 256;
+  known[dev].store(cus,std::memory_order_relaxed);
+  return (size_t) cus;
+}
+
 // Grid depth of a forward column launch of `blocks` blocks per array over nr
 // residues: one per array, times the parts the residues are dealt to when the
-// arrays' blocks leave compute units idle (256 CUs, two blocks of 512 threads
-// each).  A part reads its columns again, from the caches at these sizes.
+// arrays' blocks leave compute units idle (two blocks of 512 threads fit a CU).
+// A part reads its columns again, from the caches at these sizes, and while
+// others store: one part where the arrays overlap (a column transformed in place
+// is read before its block stores).
 // 1023 x 512 modes, FP32 (64 blocks per array, 3 residues): two arrays in 128
 // blocks of three residues each took as long as one array alone.
-static unsigned col_depth(const ColArrays &io, size_t blocks, size_t nr)
+static unsigned col_depth(const ColArrays &io, size_t blocks, size_t nr, bool overlap)
 {
-  size_t parts=512/std::max<size_t>(1,blocks*(size_t) io.n);
+  size_t parts=overlap ? 1 : 2*device_cus()/std::max<size_t>(1,blocks*(size_t) io.n);
   parts=std::max<size_t>(1,std::min(parts,nr));
   return (unsigned) (parts*(size_t) io.n);
 }
@@ -923,7 +957,12 @@ static int colreg_launch(const DimArgs &a, bool fwd, const ColArrays &io,
   typedef ColReg<T,M> CR;
   size_t lds=CR::ST::LDS*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
   dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
-  grid.z=fwd ? col_depth(io,(size_t) grid.x*nbatch,nres) : (unsigned) io.n;
+  if(fwd) {
+    const size_t E=sizeof(cplx<T>);
+    const bool overlap=col_overlap(io,E*col_span((size_t) a.L,s_in,C,ics,nbatch,bsi),
+                                   E*col_span(nres*M,s_out,C,ocs,nbatch,bso));
+    grid.z=col_depth(io,(size_t) grid.x*nbatch,nres,overlap);
+  } else grid.z=(unsigned) io.n;
   const bool p2=a.L > M;
   // the N residue twiddles in LDS when they fit without lowering occupancy
   auto zfit=[&](auto kernel) {
@@ -998,7 +1037,12 @@ static int colreal_launch(const DimArgs &a, bool fwd, const ColArrays &io,
   typedef ColReg<T,M> CR;
   const size_t lds=CR::ST::LDS*sizeof(cplx<T>)+CR::TC*CR::CS*sizeof(T);
   dim3 grid((unsigned) ((C+CR::TC-1)/CR::TC),(unsigned) nbatch);
-  if(fwd) grid.z=col_depth(io,(size_t) grid.x*nbatch,(size_t) RealKept::residues(a.q));
+  if(fwd) {
+    const bool overlap=col_overlap(io,sizeof(T)*col_span((size_t) a.L,s_in,C,ics,nbatch,bsi),
+                                   sizeof(cplx<T>)*col_span((size_t) RealKept::planes(M,a.q),s_out,C,ocs,
+                                                            nbatch,bso));
+    grid.z=col_depth(io,(size_t) grid.x*nbatch,(size_t) RealKept::residues(a.q),overlap);
+  }
   const bool p2=a.L > M;
   int rc;
   if(fwd) {
@@ -1075,7 +1119,10 @@ static int fwd_many_t(const fftwpp_amd_dim *d, const ColArrays &io, size_t S,
   if(ics == 1 && ocs == 1 && C >= (size_t) Col256<T>::TC && fast256(d,S,SF)) {
     constexpr int TC=Col256<T>::TC;
     dim3 grid((unsigned) ((C+TC-1)/TC),(unsigned) nbatch);
-    grid.z=col_depth(io,(size_t) grid.x*nbatch,nres);
+    const size_t E=sizeof(cplx<T>);
+    const bool overlap=col_overlap(io,E*col_span(d->L,S,C,1,nbatch,bsi),
+                                   E*col_span(nres*d->m,SF,C,1,nbatch,bso));
+    grid.z=col_depth(io,(size_t) grid.x*nbatch,nres,overlap);
     size_t lds=col256_lds<T>(nres);
     int rc=allow_lds(colfwd256_kernel<T>,lds);
     if(rc) return rc;

@@ -77,6 +77,10 @@ size_t fftwpp_amd_max_m(int dtype);
 /* Forward residues [r0, r0+nres) of nbatch x C columns.
  * Input element (b, j, c) at f[b*bstride_in + j*S + c], j < L.
  * Output F[b*bstride_out + ((r-r0)*m + s)*SF + c] = sum_k f_k zeta_N^{k(q s+r)}.
+ * f and F must not overlap, but for columns that are transformed in place by
+ * the register kernels (F = f with SF = S, bstride_out = bstride_in, power-of-two
+ * m in [16, 4096], L <= 2m, and C >= 8 or m >= 2048): they read a column before
+ * they write it.
  * Replaces fftPad::forward*Many / fftPadCentered::forward*Many
  * (convolve.cc:771-1466, 2199-4307). */
 int fftwpp_amd_forward_many(const fftwpp_amd_dim *d, int dtype,
