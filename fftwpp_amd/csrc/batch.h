@@ -191,8 +191,8 @@ __device__ __forceinline__ void batch_zm_unit(const cplx<T> *zN, const cplx<T> *
       const __amdgpu_buffer_rsrc_t rg=buf_rsrc<T>(gi+jb,(size_t) rem);
 #pragma unroll
       for(int k=0; k < V; ++k) {            // words past the end read zero
-        a[k]=ld_buf<T>(rf,(unsigned) t*E,TPS*k*E);
-        b[k]=ld_buf<T>(rg,(unsigned) t*E,TPS*k*E);
+        a[k]=ld_buf<T>(rf,(unsigned) (t+TPS*k)*E,0);
+        b[k]=ld_buf<T>(rg,(unsigned) (t+TPS*k)*E,0);
       }
     } else {
 #pragma unroll

@@ -267,7 +267,9 @@ __device__ __forceinline__ cplx<float> ld_buf<float>(__amdgpu_buffer_rsrc_t r, u
 }
 
 // Raw buffer resource over `words` complex words from base (offsets at or
-// beyond the end read 0 and drop stores).
+// beyond the end read 0 and drop stores).  The hardware holds the lane's offset
+// against the number of bytes less the scalar offset: where soff may exceed that
+// number, all of an access's offset is in off.
 template<typename T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const cplx<T> *base, size_t words)
 {

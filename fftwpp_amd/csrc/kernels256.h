@@ -339,7 +339,7 @@ rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
     const __amdgpu_buffer_rsrc_t rf=buf_rsrc(f+2*pr*rs,two*rs+L), rg=buf_rsrc(g+2*pr*rs,two*rs+L);
     const unsigned in=ok ? (unsigned) (i*(int) rs+j)*E : END;
     cplx<T> a[16], b[16];
-    if(L == 256) {
+    if(L == 256) {                         // the buffers hold every scalar offset
 #pragma unroll
       for(int k=0; k < 16; ++k) {
         a[k]=ld_buf<T>(rf,in,16*k*E);
@@ -350,8 +350,8 @@ rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
 #pragma unroll
       for(int k=0; k < 16; ++k) {
         const unsigned o=jf+16*k < L ? in : END;
-        a[k]=ld_buf<T>(rf,o,16*k*E);
-        b[k]=ld_buf<T>(rg,o,16*k*E);
+        a[k]=ld_buf<T>(rf,o+16*k*E,0);
+        b[k]=ld_buf<T>(rg,o+16*k*E,0);
       }
     }
 #pragma unroll
@@ -375,7 +375,7 @@ rowconv256p_kernel(const cplx<T> *f, const cplx<T> *g, int64_t rows,
 #pragma unroll
     for(int k=0; k < 8; ++k) {
       const cplx<T> v=mk(pair16_scatter(a[k].x,a[k+8].x),pair16_scatter(a[k].y,a[k+8].y));
-      st_buf<T>(ro,j0+16*k < L ? to : END,16*k*E,scale*v);
+      st_buf<T>(ro,(j0+16*k < L ? to : END)+16*k*E,0,scale*v);
     }
   }
 }
