@@ -89,7 +89,10 @@ __device__ __forceinline__ void rowreg_combine(cplx<T> *acc, T *xbase, T *xb,
 // points (q = 2) from 152 to 113 us in FP64 and from 72 to 55 us in FP32, 8192
 // rows of 500 points from 79 to 60 and from 52 to 38 us, 2048 rows of 1000
 // points padded to 2048 from 56 to 46 and from 31.5 to 25 us, one such FP64
-// row from 10.1 to 9.0 us.
+// row from 10.1 to 9.0 us.  One row of 1500 points with its residues on two
+// lanes: FP32 10.7 us with a branch per load, 11.25 with all words loaded and the
+// residue twiddles read at each use, 10.1 with them read once; FP64 17.1, 14.5,
+// 13.3 us.  (One lane per row has no registers to keep them in.)
 // W: waves per SIMD asked of the compiler; three in FP64 where the library's
 // own products fit without spills and LDS leaves room for the blocks (113
 // against 124 us at M = 128); a caller's functor keeps the registers of two.
@@ -113,7 +116,10 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
   const auto tw=stage_table<T,M,V>(twl,d);
   const cplx<T> *zN=(const cplx<T> *) d.zN;
   const int slots=RP > 1 ? 1 : blockDim.x/TPS;      // rows per block
-  const int slot=threadIdx.x/TPS, t=threadIdx.x-slot*TPS;
+  // a slot of whole waves: its index, and its residue, are uniform over the wave
+  int slot=(int) threadIdx.x/TPS;
+  if constexpr(TPS >= 64) slot=__builtin_amdgcn_readfirstlane(slot);
+  const int t=threadIdx.x-slot*TPS;
   const int rp=RP > 1 ? slot : 0;                     // residue lane
   const int rslot=RP > 1 ? 0 : slot;
   T *xbase=reinterpret_cast<T *>(twl+ST::LDS);
@@ -150,6 +156,14 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
       const int r=on ? r0+rp : 0;
       // w_N^{(j+k0) r}: j + k0 is sigma or sigma - M
       const cplx<T> bt=zN[t*r], zm=conjg(zN[M*r]);
+      // w_N^{TPS k r}: of a residue lane read with the row and kept, so that the
+      // few blocks of a single row don't wait for them twice
+      cplx<T> wk[RP > 1 ? V : 1];
+      if constexpr(RP > 1) {
+#pragma unroll
+        for(int k=0; k < V; ++k) wk[k]=zN[TPS*k*r];
+      }
+      auto wkr=[&](int k) { return RP > 1 ? wk[RP > 1 ? k : 0] : zN[TPS*k*r]; };
       cplx<T> X[V], Y[V];
       load(rb);
 #pragma unroll
@@ -158,7 +172,7 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
         const int j=(sigma-k0) & (M-1);
         cplx<T> u=a[k], v=b[k];
         if(r) {
-          cplx<T> w=bt*zN[TPS*k*r];
+          cplx<T> w=bt*wkr(k);
           if(j+k0 < 0) w=w*zm;
           u=w*u;
           v=w*v;
@@ -187,7 +201,7 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
         if(r) {
           const int sigma=t+TPS*k;
           const int j=(sigma-k0) & (M-1);
-          cplx<T> w=bt*zN[TPS*k*r];
+          cplx<T> w=bt*wkr(k);
           if(j+k0 < 0) w=w*zm;
           acc[k]=acc[k]+mulc(X[k],w);
         } else if(on)
