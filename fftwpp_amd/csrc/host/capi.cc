@@ -606,7 +606,7 @@ int fftwpp_amd_conv_work_bytes(const fftwpp_amd_conv *c, size_t *bytes, int *pla
     if(plane) *plane=p ? 1 : 0;
   } else if(c->c2 || c->h2) {
     const Convolution2 *k=c->c2 ? c->c2->convolve2 : c->h2->convolve2;
-    *bytes=k->workBytes(c->dtype,k->residueBlock(c->dtype,real));
+    *bytes=k->workBytes(c->dtype,k->residueBlock(c->dtype,real))+k->gradientBytes();
     if(plane) *plane=0;
   } else {
     fftwpp_amd_internal_set_error("fftwpp_amd_conv_work_bytes: 2D and 3D plans only");

@@ -2370,6 +2370,16 @@ int fftwpp_amd_malloc(void **p, size_t bytes)
   return hipcheck(hipMalloc(p,bytes),"hipMalloc");
 }
 
+// Device memory when there is room: false, with no error left behind, when not.
+int fftwpp_amd_internal_try_malloc(void **p, size_t bytes)
+{
+  *p=NULL;
+  if(hipMalloc(p,bytes) == hipSuccess) return 1;
+  *p=NULL;
+  (void) hipGetLastError();               // launches ask for the last error too
+  return 0;
+}
+
 int fftwpp_amd_free(void *p)
 {
   if(!p) return FFTWPP_AMD_OK;

@@ -137,6 +137,8 @@ public:
   std::vector<size_t> sizes;
   std::vector<std::vector<size_t>> keys;  // what a slot holds (empty: nothing known), e.g. an item table
   void *get(size_t slot, size_t bytes);
+  void *find(size_t slot, size_t bytes);  // NULL when there is no room
+  size_t held(size_t slot) const { return slot < sizes.size() ? sizes[slot] : 0; }
   ~DeviceWork();
 
 };
@@ -456,7 +458,8 @@ public:
   // out[k] <- w (*) g[k], k = 0, 1, with one x transform of w for both (the
   // two products of the adjoint); the inputs are read before the outputs are
   // written.  False, and nothing done, where the plan runs otherwise (real
-  // data, a memory limit, a timeline or row hook, rows without a fused kernel).
+  // data, a memory limit, a timeline or row hook, rows without a fused kernel,
+  // no room for a third x-transformed array).
   bool execShared(void *const out[2], const void *w, const void *const g[2], bool normalize,
                   int dtype, void *stream, int mult=-1);
   size_t arraySize() const;
@@ -471,10 +474,13 @@ public:
   size_t memoryLimit=0;
   // Work bytes with Dx x residues per pass (0: all of them).
   size_t workBytes(int dtype, size_t Dx=0) const;
+  // Bytes of the third x-transformed array that execShared keeps.
+  size_t gradientBytes() const;
   // x residues per pass (0: none fits the limit).
   size_t residueBlock(int dtype, bool real) const;
 
 protected:
+  static const size_t GRADIENTS=11;  // its work slot
   int multCode;
   size_t ly;  // stored length of a y row (Ly or ceil(Ly/2))
   DeviceWork work;

@@ -339,7 +339,9 @@ int fftwpp_amd_conv_create_tuned(fftwpp_amd_conv **h, int dim, int hermitian,
  * execution that fits none of these fails with FFTWPP_AMD_ERR_UNSUPPORTED.
  * Results are the same in every case.  fftwpp_amd_conv_work_bytes reports the
  * bytes the next execution in the plan's precision holds and whether it takes
- * the plane kernel. */
+ * the plane kernel.  A 2D plan without a limit that has computed both
+ * gradients of an adjoint at once keeps a third x-transformed array for it, which
+ * the report then counts. */
 int fftwpp_amd_conv_set_memory_limit(fftwpp_amd_conv *h, size_t bytes);
 int fftwpp_amd_conv_work_bytes(const fftwpp_amd_conv *h, size_t *bytes, int *plane);
 

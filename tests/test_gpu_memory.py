@@ -75,3 +75,23 @@ def test_memory_limit_too_small_is_refused(gpu, oracle):
     a = torch.ones((40, 33), dtype=torch.complex128, device=gpu)
     with pytest.raises(FFTWPPError):
         plan.convolve_out(torch.empty_like(a), a, a)
+
+
+@pytest.mark.parametrize("kind", ["complex", "hermitian"])
+def test_gradient_array_is_reported(gpu, kind):
+    """Both gradients at once keep a third x-transformed array, which the report
+    counts; one gradient, and a plan under a limit, keep none."""
+    import torch
+    from fftwpp_amd.torch_conv import DeviceConvolution
+    w, a, b = (torch.randn((41, 33), dtype=torch.complex128, device=gpu) for _ in range(3))
+    plan, capped = (DeviceConvolution((41, 33), kind=kind) for _ in range(2))
+    full, _ = plan.work_bytes()
+    plan.adjoint(w, a, b, need_b=False)
+    assert plan.work_bytes()[0] == full
+    ga, gb = plan.adjoint(w, a, b)
+    assert plan.work_bytes()[0] == full + full // 2
+    capped.set_memory_limit(full)
+    ga1, gb1 = capped.adjoint(w, a, b)
+    assert capped.work_bytes()[0] == full
+    for x, y in ((ga, ga1), (gb, gb1)):
+        assert (x - y).norm() <= 1e-13 * y.norm()
