@@ -225,7 +225,7 @@ __device__ __forceinline__ void batch_zm_unit(const cplx<T> *zN, const cplx<T> *
 #pragma unroll
   for(int k=0; k < V; ++k)
     X[k]=mult == 1 ? X[k]*Y[k] : (mult == 3 ? mulc(X[k],Y[k]) : X[k]);
-  fftr<T,M,V,-1,true>(X,xb,tw,t);
+  fftr<T,M,V,-1>(X,xb,tw,t);
   if(r) {
 #pragma unroll
     for(int k=0; k < V; ++k) X[k]=mulc(X[k],bt*tr[k]);
@@ -373,12 +373,12 @@ batch_reg_kernel(DimArgs d, const BatchItem *items, int64_t count,
           Y[k]=w*Y[k];
         }
       }
-      fftr<T,M,V,1,true>(X,xb,tw,t);
-      fftr<T,M,V,1,true>(Y,xb,tw,t);
+      fftr<T,M,V,1>(X,xb,tw,t);
+      fftr<T,M,V,1>(Y,xb,tw,t);
 #pragma unroll
       for(int k=0; k < V; ++k)
         X[k]=mult == 1 ? X[k]*Y[k] : (mult == 3 ? mulc(X[k],Y[k]) : X[k]);
-      fftr<T,M,V,-1,true>(X,xb,tw,t);
+      fftr<T,M,V,-1>(X,xb,tw,t);
       if(r) {
 #pragma unroll
         for(int k=0; k < V; ++k) X[k]=mulc(X[k],bt*tr[k]);

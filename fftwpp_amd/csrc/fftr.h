@@ -11,9 +11,9 @@
 // j = t + TPS b (b < V/R) with k' = j mod Ns,
 //     u_t' = v[b + t' V/R] w^{t' k'},   w = e^{S 2 pi i/(Ns R)},
 //     out[(j/Ns) Ns R + k' + u Ns] = sum_t' u_t' e^{S 2 pi i u t'/R},
-// in place in registers; between stages the outputs go through LDS (real
-// and imaginary parts in two rounds, scalar words at e + e/16, which keeps
-// every access of the gfx950 LDS bank-conflict free) and come back as
+// in place in registers; between stages the outputs go through LDS in one round
+// (an area of 2 PAD scalar words: real parts, then imaginary parts PAD words on;
+// element e at the word that an index map names, see xidx()) and come back as
 // v[k] = out[t + TPS k].  After the last stage v[k] holds X[t + TPS k].
 //
 // Twiddles: one LDS table of M-1 complex words, stage s at offset off_s
@@ -66,7 +66,7 @@ template<int M, int V=16> struct RPlan {
 
 __device__ __forceinline__ int padr(int e) { return e+(e >> 4); }
 
-// Word of sequence element e in a one-round (CX) exchange area: an XOR
+// Word of sequence element e in each half of an exchange area: an XOR
 // swizzle of the low bits by higher bits that makes every exchange of the
 // transform conflict-free on gfx950's LDS (64-bit words: writes served 16
 // lanes per pass over 32 banks, reads 32 lanes over 64 banks; 32-bit words:
@@ -172,7 +172,7 @@ __device__ __forceinline__ void rsync()
     __syncthreads();
 }
 
-// Word of element e in a one-round exchange area (the default index map).
+// Word of element e in each half of an exchange area (the default index map).
 // The maps act on disjoint bit fields one by one, so the word of an element
 // whose thread part and compile-time part have no bit in common is
 // join(at(thread part), at(constant)): one instruction per access and one
@@ -184,11 +184,8 @@ template<typename T, int M, int V> struct RowXI {
 };
 
 // Stage s of the transform (see the top of this file); recurses into s+1.
-// CX: xb holds 2 PAD words, real parts in the first PAD and imaginary parts in
-// the second, and each exchange is one round (two synchronisations instead
-// of four); element e sits at word XI::at(e) ^ xm of each half.
-template<typename T, int M, int V, int S, int s, bool BLK, bool CX=false,
-         class XI=RowXI<T,M,V>, class TW>
+// Element e sits at word XI::at(e) ^ xm of each half of the exchange area xb.
+template<typename T, int M, int V, int S, int s, bool BLK, class XI=RowXI<T,M,V>, class TW>
 __device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const TW &tw,
                                            int t, int xm=0)
 {
@@ -212,7 +209,7 @@ __device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const TW &tw,
 #pragma unroll
     for(int tp=0; tp < R; ++tp) v[b+tp*NB]=u[tp];
   }
-  if constexpr(s+1 < P::NST && CX) {
+  if constexpr(s+1 < P::NST) {
     // exchange: output u of butterfly b goes to (j/Ns) Ns R + k' + u Ns
     const int wo=XI::at(P::template dest<s>(t)) ^ xm, ro=XI::at(t) ^ xm;
 #pragma unroll
@@ -231,30 +228,7 @@ __device__ __forceinline__ void fftr_stage(cplx<T> *v, T *xb, const TW &tw,
       v[k]=mk(xb[e],xb[P::PAD+e]);
     }
     rsync<TPS,BLK>();
-    fftr_stage<T,M,V,S,s+1,BLK,CX,XI>(v,xb,tw,t,xm);
-  } else if constexpr(s+1 < P::NST) {
-    // exchange: output u of butterfly b goes to (j/Ns) Ns R + k' + u Ns
-#pragma unroll
-    for(int part=0; part < 2; ++part) {
-#pragma unroll
-      for(int b=0; b < NB; ++b) {
-        const int j=t+TPS*b;
-        const int kp=j & (Ns-1);
-        const int base=(j-kp)*R+kp;
-#pragma unroll
-        for(int u=0; u < R; ++u)
-          xb[padr(base+u*Ns)]=part == 0 ? v[b+u*NB].x : v[b+u*NB].y;
-      }
-      rsync<TPS,BLK>();
-#pragma unroll
-      for(int k=0; k < V; ++k) {
-        const T val=xb[padr(t+TPS*k)];
-        if(part == 0) v[k].x=val;
-        else v[k].y=val;
-      }
-      rsync<TPS,BLK>();
-    }
-    fftr_stage<T,M,V,S,s+1,BLK>(v,xb,tw,t);
+    fftr_stage<T,M,V,S,s+1,BLK,XI>(v,xb,tw,t,xm);
   }
 }
 
@@ -320,7 +294,7 @@ __device__ __forceinline__ void fftr_pair_stage(cplx<T> *X, cplx<T> *Y, T *xb,
   }
 }
 
-// fftr<T,M,V,S,true> of X and of Y, their butterflies interleaved stage by
+// fftr<T,M,V,S> of X and of Y, their butterflies interleaved stage by
 // stage; same results, same exchange area and barriers.
 template<typename T, int M, int V, int S, class TW>
 __device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const TW &tw,
@@ -330,31 +304,23 @@ __device__ __forceinline__ void fftr_pair(cplx<T> *X, cplx<T> *Y, T *xb, const T
 }
 
 // In-place transform of the sequence held by threads t < TPS (v[V] each)
-// with kernel e^{S 2 pi i jk/M}; xb is the sequence's exchange area
-// (RPlan<M,V>::PAD scalar words), tw the twiddle table of RPlan<M,V>.  When
+// with kernel e^{S 2 pi i jk/M}; xb is the sequence's exchange area (2
+// RPlan<M,V>::PAD scalar words), tw the twiddle table of RPlan<M,V>.  When
 // TPS > 64 every thread of the block must call this.
-template<typename T, int M, int V, int S, bool CX=false, class TW>
+template<typename T, int M, int V, int S, class TW>
 __device__ __forceinline__ void fftr(cplx<T> *v, T *xb, const TW &tw, int t)
 {
-  fftr_stage<T,M,V,S,0,false,CX>(v,xb,tw,fresh(t));
+  fftr_stage<T,M,V,S,0,false>(v,xb,tw,fresh(t));
 }
 
 // The same transform when the threads of a sequence are not consecutive
-// lanes (block barriers; every thread of the block must call it).
-template<typename T, int M, int V, int S, bool CX=false>
-__device__ __forceinline__ void fftr_blk(cplx<T> *v, T *xb, const cplx<T> *tw,
-                                         int t)
-{
-  fftr_stage<T,M,V,S,0,true,CX>(v,xb,tw,fresh(t));
-}
-
-// fftr_blk with one-round exchanges through the index map XI, XORed by xm.
-// FRESH: positions computed anew (see fresh()).
+// lanes (block barriers; every thread of the block must call it), through the
+// index map XI, XORed by xm.  FRESH: positions computed anew (see fresh()).
 template<typename T, int M, int V, int S, class XI, bool FRESH=true, class TW>
 __device__ __forceinline__ void fftr_blkx(cplx<T> *v, T *xb, const TW &tw,
                                           int t, int xm)
 {
-  fftr_stage<T,M,V,S,0,true,true,XI>(v,xb,tw,FRESH ? fresh(t) : t,xm);
+  fftr_stage<T,M,V,S,0,true,XI>(v,xb,tw,FRESH ? fresh(t) : t,xm);
 }
 
 } // namespace fftwpp_amd

@@ -1589,12 +1589,18 @@ void Convolution3::execComplex(void *out, const void *f0, const void *f1, bool n
     const size_t nplanes=real ? maxplanes : nres*mx;
     const bool first=r0 == 0, last=r0+nres == qx;
     // x forward: columns (y,z); non-contiguous y strides become batches.  Both
-    // inputs in one launch (one long tail per stage instead of two: 255 x 255 x
-    // 128 Hermitian modes FP64 1023 -> 999 us), unless their stages are timed
-    // one by one or an x-transformed array exceeds the 256 MB Infinity Cache:
-    // then f's y stage runs at once on what its x stage left there (real 256^3
-    // FP64, 270 MB: 1204 us against 1257 us paired).
-    const int na=timeline || nplanes*plane*E > ((size_t) 256 << 20) ? 1 : 2;
+    // inputs in one launch per stage (one tail instead of two), unless their
+    // stages are timed one by one or no stage takes several arrays in a launch
+    // (generic LDS columns in x and y): then f's y stage runs at once on what its
+    // x stage left in the Infinity Cache.  One by one against paired, us: complex
+    // 64^3 to 160^3 FP32 47 -> 41.5 to 688 -> 665, FP64 58 -> 51 to 1323 -> 1325, 192^3 to
+    // 256^3 FP64 1556 -> 1556 to 2148 -> 2148, 255 x 255 x 128 Hermitian FP64 941 -> 911,
+    // real 256^3 FP64 1201 -> 1204; slower paired only where one array's x and y
+    // stages fit the cache and two do not (64 + 128 MB: 128^3 FP64 289.5 -> 292,
+    // 32 x 256 x 256 269 -> 275; but not 35 + 120 MB 267 -> 254, 96 + 144 MB 477 -> 458);
+    // LDS columns of 96 points, 191 x 191 x 96 Hermitian FP64 939 -> 962.
+    const int na=timeline || (fftwpp_amd_internal_engine(fftx->dev,0) == 0 &&
+                              fftwpp_amd_internal_engine(ffty->dev,0) == 0) ? 1 : 2;
     for(int a=0; a < 2; a += na) {
       if(contiguous())
         check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,real,na,in+a,Sx,plane,1,0,X+a,plane,0,

@@ -195,7 +195,7 @@ rowcx_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t row0, int64_
 #pragma unroll
         for(int k=0; k < V; ++k) X[k]=rop(X[k],Y[k],q*(t+TPS*k)+r);
       }
-      fftr<T,M,V,-1,true>(X,xb,tw,t);
+      fftr<T,M,V,-1>(X,xb,tw,t);
 #pragma unroll
       for(int k=0; k < V; ++k) {
         if(r) {
@@ -285,8 +285,8 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
         X[k]=a;
         Y[k]=b;
       }
-      fftr<T,M,V,1,true>(X,xb,tw,t);
-      fftr<T,M,V,1,true>(Y,xb,tw,t);
+      fftr<T,M,V,1>(X,xb,tw,t);
+      fftr<T,M,V,1>(Y,xb,tw,t);
       {
         const auto rop=bind_row(op,row);
 #pragma unroll
@@ -295,7 +295,7 @@ rowreg_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
           X[k]=mk(rop(X[k].x,Y[k].x,l+r1),r2 >= 0 ? rop(X[k].y,Y[k].y,l+r2) : (T) 0);
         }
       }
-      fftr<T,M,V,-1,true>(X,xb,tw,t);
+      fftr<T,M,V,-1>(X,xb,tw,t);
       // mirror elements Z(M - sigma) through LDS
       cplx<T> Zm[V];
 #pragma unroll
@@ -682,11 +682,11 @@ hrowpk_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows, int64
           X[k]=mk(p1[k],rop(X2[k].x,X2[k].y,q*(t+TPS*k)+r2));
         }
       } else {
-        fftr<T,M,V,1,true>(X,xb,tw,t);
+        fftr<T,M,V,1>(X,xb,tw,t);
 #pragma unroll
         for(int k=0; k < V; ++k) X[k]=mk(rop(X[k].x,X[k].y,q*(t+TPS*k)+r1),(T) 0);
       }
-      fftr<T,M,V,-1,true>(X,xb,tw,t);
+      fftr<T,M,V,-1>(X,xb,tw,t);
       // mirror elements Z(M - sigma) through LDS
       const int tm=fresh(t);
 #pragma unroll
@@ -804,11 +804,11 @@ hrows_long_kernel(DimArgs d, const cplx<T> *f, const cplx<T> *g, int64_t rows,
         if(e2 >= q) e2 -= q;
       }
     }
-    fftr<T,M,V,1,true>(X,xb,tw,t);
-    fftr<T,M,V,1,true>(Y,xb,tw,t);
+    fftr<T,M,V,1>(X,xb,tw,t);
+    fftr<T,M,V,1>(Y,xb,tw,t);
 #pragma unroll
     for(int k=0; k < V; ++k) X[k]=mk(X[k].x*Y[k].x,X[k].y*Y[k].y);
-    fftr<T,M,V,-1,true>(X,xb,tw,t);
+    fftr<T,M,V,-1>(X,xb,tw,t);
     // mirror elements Z(M - sigma) through LDS
 #pragma unroll
     for(int k=0; k < V; ++k) {
