@@ -13,7 +13,7 @@
 // kernel-layer queries (kernels.hip): does a fused row kernel take a row;
 // which engine takes the rows (stage 1) of a dimension (2: register FFT).
 extern "C" int fftwpp_amd_internal_rows_fit(const fftwpp_amd_dim *d, int dtype);
-extern "C" int fftwpp_amd_internal_try_malloc(void **p, size_t bytes);
+extern "C" int fftwpp_amd_internal_try_malloc(void **p, size_t bytes, void *stream);
 extern "C" int fftwpp_amd_internal_engine(const fftwpp_amd_dim *d, int stage);
 // the forward residue transforms of up to three arrays of one layout in one launch
 extern "C" int fftwpp_amd_internal_forward_arrays(const fftwpp_amd_dim *d, int dtype, int real,
@@ -712,11 +712,11 @@ void *DeviceWork::get(size_t slot, size_t bytes)
   return bufs[slot];
 }
 
-void *DeviceWork::find(size_t slot, size_t bytes)
+void *DeviceWork::find(size_t slot, size_t bytes, void *stream)
 {
   if(held(slot) < bytes) {
     void *p;
-    if(!fftwpp_amd_internal_try_malloc(&p,bytes)) return NULL;
+    if(!fftwpp_amd_internal_try_malloc(&p,bytes,stream)) return NULL;
     get(slot,0);                           // the slot exists
     fftwpp_amd_free(bufs[slot]);
     bufs[slot]=p;
@@ -1370,7 +1370,7 @@ bool Convolution2::execShared(void *const out[2], const void *w, const void *con
     return false;
   const size_t q=fftx->q, rows=q*fftx->m, bytes=rows*ly*eltsize(dtype);
   const void *in[3]={w,g[0],g[1]};
-  void *F[3]={work.get(0,bytes),work.get(1,bytes),work.find(GRADIENTS,bytes)};
+  void *F[3]={work.get(0,bytes),work.get(1,bytes),work.find(GRADIENTS,bytes,stream)};
   if(!F[2]) return false;                  // no room: the products in turn take two arrays
   check(fftwpp_amd_internal_forward_arrays(fftx->dev,dtype,0,3,in,Sx,ly,1,0,F,ly,0,0,q,stream),
         "x forward");

@@ -2370,10 +2370,17 @@ int fftwpp_amd_malloc(void **p, size_t bytes)
   return hipcheck(hipMalloc(p,bytes),"hipMalloc");
 }
 
-// Device memory when there is room: false, with no error left behind, when not.
-int fftwpp_amd_internal_try_malloc(void **p, size_t bytes)
+// Device memory when there is room: false, with no error left behind, when not,
+// and while `stream` is being captured (an allocation would end the capture).
+int fftwpp_amd_internal_try_malloc(void **p, size_t bytes, void *stream)
 {
   *p=NULL;
+  hipStreamCaptureStatus status=hipStreamCaptureStatusNone;
+  if(hipStreamIsCapturing((hipStream_t) stream,&status) != hipSuccess ||
+     status != hipStreamCaptureStatusNone) {
+    (void) hipGetLastError();
+    return 0;
+  }
   if(hipMalloc(p,bytes) == hipSuccess) return 1;
   *p=NULL;
   (void) hipGetLastError();               // launches ask for the last error too

@@ -137,7 +137,7 @@ public:
   std::vector<size_t> sizes;
   std::vector<std::vector<size_t>> keys;  // what a slot holds (empty: nothing known), e.g. an item table
   void *get(size_t slot, size_t bytes);
-  void *find(size_t slot, size_t bytes);  // NULL when there is no room
+  void *find(size_t slot, size_t bytes, void *stream);  // NULL when there is no room, or under capture
   size_t held(size_t slot) const { return slot < sizes.size() ? sizes[slot] : 0; }
   ~DeviceWork();
 
@@ -459,7 +459,7 @@ public:
   // two products of the adjoint); the inputs are read before the outputs are
   // written.  False, and nothing done, where the plan runs otherwise (real
   // data, a memory limit, a timeline or row hook, rows without a fused kernel,
-  // no room for a third x-transformed array).
+  // no room for a third x-transformed array, none held while the stream is captured).
   bool execShared(void *const out[2], const void *w, const void *const g[2], bool normalize,
                   int dtype, void *stream, int mult=-1);
   size_t arraySize() const;
