@@ -167,8 +167,13 @@ inline size_t plane_lds()
 // Planes of 256 x 256 words (Ly = lz = 256).  Sub-team s of XCD x takes
 // the planes x + 8 (2 i + s); its block k owns z columns [8k, 8k+8) in
 // phases A and C and rows [16k, 16k+16) of its E in phase B.
+// Exactly n waves per SIMD, so that every CU holds one block of each sub-team,
+// with its waves one to a SIMD: with registers for one wave more (FP32: 126) the
+// 256^3 convolution took 1610 to 1630 us, also where LDS admitted only n blocks;
+// with 132 1400 us.
 template<typename T, int MULT>
-__global__ void __launch_bounds__(PLANE_THREADS,PlaneSub<T>::n)
+__global__ void __attribute__((amdgpu_waves_per_eu(PlaneSub<T>::n,PlaneSub<T>::n)))
+__launch_bounds__(PLANE_THREADS,PlaneSub<T>::n)
 plane256_kernel(const cplx<T> *Xf, const cplx<T> *Xg, cplx<T> *Xh,
                 int64_t planes, const cplx<T> *zN, cplx<T> *E, PlaneCtl *ctl)
 {

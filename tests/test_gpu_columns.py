@@ -1,8 +1,7 @@
-"""Column transforms where their launches differ: 256-point columns in more
-tiles than blocks stay resident (each block then takes several), partly filled
-tiles, real columns over every residue pattern, several arrays in one launch
-with the residues dealt to different blocks, and the adjoint's shared
-transform of the cotangent.
+"""Column transforms where their launches differ: 256-point columns in few
+tiles (residues dealt to different blocks) and in more tiles than blocks stay
+resident, partly filled tiles, real columns over every residue pattern, several
+arrays in one launch, and the adjoint's shared transform of the cotangent.
 
 Bar: relative L2 error <= 1e-12 in FP64, <= 1e-5 in FP32 against the oracle."""
 import numpy as np
@@ -29,8 +28,8 @@ def _conv(gpu, f, g, kind, dtype, M=None, m=None):
     return out.cpu().numpy(), plan
 
 
-# x columns of m = 256 (Lx <= 256), q = 1 ... 4; Ly columns: one tile, a partly
-# filled tile, and more tiles than resident blocks
+# x columns of m = 256 (Lx <= 256), q = 1 ... 4; Ly columns: one tile, partly
+# filled last tiles, and 125 tiles (63 in FP32)
 @pytest.mark.parametrize("kind,dtype", [("complex", "complex128"), ("complex", "complex64"),
                                         ("real", "float64"), ("real", "float32")])
 @pytest.mark.parametrize("Lx,Mx,Ly", [(256, 512, 8), (256, 512, 21), (100, 256, 40), (255, 768, 33),
