@@ -252,8 +252,10 @@ __device__ __forceinline__ void batch_zm_unit(const cplx<T> *zN, const cplx<T> *
 // the backward fold over the blocks b of the reference's backward transforms
 // (convolve.cc:1468-1613, 1765-1965), so no output word is read and written
 // once per residue.
+// The FP64 sequence mode of M = 1024 and 2048 asks for three waves per SIMD (170
+// registers without it, one too many for the third).
 template<typename T, int M, bool ZM=false>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512,(ZM && sizeof(T) == 8 && (M == 1024 || M == 2048) ? 3 : 1))
 batch_reg_kernel(DimArgs d, const BatchItem *items, int64_t count,
                  const cplx<T> *f, const cplx<T> *g, cplx<T> *out, T scale,
                  int mult, int D, cplx<T> *part, int64_t ptotal)
@@ -373,12 +375,14 @@ batch_reg_kernel(DimArgs d, const BatchItem *items, int64_t count,
           Y[k]=w*Y[k];
         }
       }
-      fftr<T,M,V,1>(X,xb,tw,t);
-      fftr<T,M,V,1>(Y,xb,tw,t);
+      // (two waves per SIMD either way: positions stay in registers; 26666 items
+      // of 300 words, m = 512, q = 2, FP64 257 us with them computed anew, 249)
+      fftr<T,M,V,1,false>(X,xb,tw,t);
+      fftr<T,M,V,1,false>(Y,xb,tw,t);
 #pragma unroll
       for(int k=0; k < V; ++k)
         X[k]=mult == 1 ? X[k]*Y[k] : (mult == 3 ? mulc(X[k],Y[k]) : X[k]);
-      fftr<T,M,V,-1>(X,xb,tw,t);
+      fftr<T,M,V,-1,false>(X,xb,tw,t);
       if(r) {
 #pragma unroll
         for(int k=0; k < V; ++k) X[k]=mulc(X[k],bt*tr[k]);
