@@ -239,44 +239,60 @@ bool tile_fits(const fftwpp_amd_batch &h, const Cls &c, size_t TR)
   return fftwpp_amd_batch_rows_lds(c.dim,h.dtype,TR,0) != 0;
 }
 
-// Sub-FFT size without tuning.  One residue (m = 2^ceil(log2 M)) needs no
-// second launch and folds nothing, up to the size where the transform's
-// exchange area and twiddles leave too few blocks on a CU: 4096 in FP32, 2048
-// in FP64 (6000 items of 600 to 1024 words: 145 us, 168 with two residues of
-// 1024); longer FP64 items take residues of m = 2048 (L <= 8192; 1000 items of
-// 4097 to 7000 words: 248 us, 264 with 4096 and 292 with 1024), else of 4096
-// (300 items of 16000 words: 254 us, 272 with 2048).  4096 sequences of 64 to
-// 16384 words in FP64, with the units of default_tile: 1065 us with m =
-// 2^ceil(log2 L) and two units per CU, 570 us so.
-size_t default_m(size_t L, size_t M, int dtype)
+// Sub-FFT size without tuning, in a batch of n items.  One residue (m =
+// 2^ceil(log2 M)) needs no second launch and folds nothing, up to the size where
+// the transform's exchange area and twiddles leave too few blocks on a CU: 4096
+// in FP32, 2048 in FP64 (6000 items of 600 to 1024 words: 145 us, 168 with two
+// residues of 1024), and in FP64 but for items of 257 to 512 words that fill the
+// chip several times, whose sequence of 1024 leaves two waves per SIMD little to
+// overlap (26666 items of 300 words: 249 us in two residues of 512, 296 in one of
+// 1024; 16000 of 500 words 182 and 194; 1000 items of 300 words 16 and 13.6).
+// Longer FP64 items take residues of m = 2048 (L <= 8192; 1000 items of 4097 to
+// 7000 words: 248 us, 264 with 4096 and 292 with 1024), else of 4096 (300 items
+// of 16000 words: 254 us, 272 with 2048).  4096 sequences of 64 to 16384 words in
+// FP64, in a process of their own: 857 us with m = 2^ceil(log2 L) and two units
+// per CU; 632 us so, with the units of default_tile.
+size_t default_m(size_t L, size_t M, size_t n, int dtype)
 {
   const size_t e=std::max<size_t>(16,ceilpow2(M));
   if(dtype == FFTWPP_AMD_F32) return std::min<size_t>(e,BATCH_MAXM);
+  if(e == 1024 && n >= 4096) return 512;
   if(e <= 2048) return e;
   return L <= 8192 ? 2048 : BATCH_MAXM;
 }
 
 // Without tuning.  Register kernel: items of several residues run in the
 // sequence mode (D = 0: every residue a unit, the outputs folded by a second
-// launch), except q = 2 with m = 2048 in FP64, whose unit does both residues
-// (4000 items of 1025 to 1700 words: 209 us, 226 in the sequence mode);
-// when several units share an item the grid is the blocks that stay resident
-// (two waves per SIMD, three in FP64, LDS permitting), so an item's units run close together
-// and find its words in L2.  LDS kernel: small tiles of short items, and
-// enough residue groups for about two work units per compute unit.
+// launch), except two residues where one unit does both and saves that launch:
+// FP64 with m = 512, and with m = 2048 when the items fill the chip (4000 items of
+// 1025 to 1700 words: 209 us, 226 in the sequence mode; 16 of 1200 words 19.6 and
+// 11.9); FP32 where the units of two residues take about as many rounds of the
+// resident blocks (3200 items of 2500 words: 169 us, 195 in the sequence mode;
+// 666 of 3000 words, 2 x 2 rounds against 3: 68 and 57).  When several units share
+// an item the grid is the blocks that stay resident (two waves per SIMD, three in
+// FP64, LDS permitting), so an item's units run close together and find its words
+// in L2; FP32 grids always, since more blocks run in rounds of unequal size (8000
+// items of 1000 words, m = 2048: 110 us in 8 blocks per CU, 89 in the 4 that fit).
+// LDS kernel: small tiles of short items, and enough residue groups for about
+// two work units per compute unit.
 Tile default_tile(const fftwpp_amd_batch &h, const Cls &c)
 {
   if(size_t tps=fftwpp_amd_batch_rows_tps(c.dim,h.dtype)) {
-    const size_t threads=std::max<size_t>(256,tps);
-    const size_t D=c.q == 1 ? 1 : c.q == 2 && c.m == 2048 && h.dtype == FFTWPP_AMD_F64 ? 2 : 0;
-    Tile t=make_tile(h,c,1,threads,D);
-    if(tps > 64 && groups(c,t) > 1) {
-      const size_t elt=h.dtype == FFTWPP_AMD_F32 ? 8 : 16;
-      const size_t tw=elt == 16 && c.m >= 1024 ? 512 : c.m;  // twiddles, exchange area
-      const size_t lds=(tw+c.m+c.m/16+c.q*(c.m/tps))*elt;
-      const size_t per=std::max<size_t>(1,std::min<size_t>(160*1024/lds,(elt == 16 ? 768 : 512)/tps));
-      t.nblocks=std::min(t.nblocks,per*(size_t) h.cus);
+    const bool f32=h.dtype == FFTWPP_AMD_F32;
+    const size_t threads=std::max<size_t>(256,tps), n=c.ids.size();
+    const size_t elt=f32 ? 8 : 16, tw=!f32 && c.m >= 1024 ? 512 : c.m;
+    const size_t lds=(tw+c.m+c.m/16+c.q*(c.m/tps))*elt;        // twiddles, exchange area
+    const size_t per=std::max<size_t>(1,std::min<size_t>(160*1024/lds,(f32 ? 512 : 768)/tps));
+    const size_t resident=per*(size_t) h.cus;
+    size_t D=c.q == 1 ? 1 : 0;
+    if(c.q == 2 && tps > 64) {
+      const bool both=f32 ? 20*ceilquot(n,resident) <= 11*ceilquot(2*n,resident) :
+        c.m == 2048 && n >= (size_t) h.cus;
+      if(both) D=2;
     }
+    if(c.q == 2 && c.m == 512 && !f32) D=2;
+    Tile t=make_tile(h,c,1,threads,D);
+    if(tps > 64 && (groups(c,t) > 1 || f32)) t.nblocks=std::min(t.nblocks,resident);
     return t;
   }
   size_t TR=std::max<size_t>(1,std::min<size_t>(32,2048/c.m));
@@ -896,7 +912,7 @@ int fftwpp_amd_batch_create(fftwpp_amd_batch **out, size_t n, const size_t *L,
   if(rc) { destroy(h); return rc; }
   const size_t maxm=BATCH_MAXM;
   h->mof.resize(n);
-  for(size_t i=0; i < n; ++i) h->mof[i]=default_m(h->L[i],h->M[i],dtype);
+  for(size_t i=0; i < n; ++i) h->mof[i]=default_m(h->L[i],h->M[i],n,dtype);
   const bool tuned=flags & FFTWPP_AMD_BATCH_TUNE;
   TuneArrays ta;
   bool timing=false;                      // ta holds the timing arrays
@@ -913,7 +929,7 @@ int fftwpp_amd_batch_create(fftwpp_amd_batch **out, size_t n, const size_t *L,
       else h->mof[i]=it->second;
     }
     if(!cached) {
-      for(size_t i=0; i < n; ++i) h->mof[i]=default_m(h->L[i],h->M[i],dtype);
+      for(size_t i=0; i < n; ++i) h->mof[i]=default_m(h->L[i],h->M[i],n,dtype);
       rc=ta.init(*h);
       timing=true;
       if(!rc) rc=tune_geometry(*h,ta);
