@@ -117,14 +117,14 @@ __device__ __forceinline__ void bfly(cplx<T> *u)
   else DFT<T,R>::run(u,S);
 }
 
-// Twiddles of a long FP64 transform: those of the last stage, which are most
-// of the table (M = 2048: 24 of 32 KB), stay in device memory in the table's
+// Twiddles of a long FP64 transform: those of the last stage, half of the table
+// at 1024 points, three quarters at 2048 and seven eighths at 4096, stay in device memory in the table's
 // order (DimArgs::last) and are read from there by each transform, consecutive
 // lanes consecutive words; LDS holds the others.  These transforms wait on LDS
 // and barriers rather than compute (13% of the vector unit's cycles), and with
 // all of the table in LDS two waves per SIMD were resident; now three are.
 // 2048 rows of 1000 points padded to 2048: 49 -> 41.5 us; 4096 sequences of 64
-// to 16384 words: 830 -> 570 us.
+// to 16384 words, in a process of their own: 632 -> 541 us.
 template<typename T, int M, int V, int MIN=1024> struct SplitTw {
   static constexpr bool USED=sizeof(T) == 8 && V == 8 && M >= MIN;
   static constexpr int LDS=USED ? 512 : M;

@@ -171,9 +171,9 @@ inline int rowreg_launch(const DimArgs &a, const void *f, const void *g, size_t 
   constexpr int TPS=M/RowV::V;
   const int64_t passes=HERM ? (a.q+1)/2 : a.q;
   // Hermitian rows of up to 2048 points with enough rows to fill the chip:
-  // the packed kernel (rowreg_kernel takes 1.3 to 1.5 times as long there:
-  // 73728 rows of H = M = 128, q = 3, FP64 207 against 297 us, 36864 of 256
-  // 205 against 302 us, FP32 99 against 140 us), whose block reads its rows
+  // the packed kernel (rowreg_kernel takes 1.4 to 1.6 times as long there:
+  // 73728 rows of H = M = 128, q = 3, FP64 185 against 297 us, 36864 of 256
+  // 186 against 302 us, FP32 99 against 140 us), whose block reads its rows
   // through one buffer and whose residue twiddles stay within 16 KB of LDS
   if constexpr(HERM && M <= 2048)
     if(rows >= 512 && (size_t) HRowPk<T,M>::SLOTS <= rows_in_buffer(rs,sizeof(cplx<T>)) &&

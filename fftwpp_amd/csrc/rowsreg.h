@@ -412,8 +412,11 @@ __device__ __forceinline__ void slot_combine(T &x, T &y, T *red, Combine c)
 // are relative to the larger one: exact powers of two bring them to one
 // magnitude first, 2^-ef F and 2^-eg G, whose norms then differ by at most a
 // factor sqrt(2).  near: ef = 0, only G is scaled.  Otherwise (far) both are, to
-// norms near 1.  (FP32, H = 128, q = 3, relative error of a row's product: F of
-// 1e-4 times G's magnitude 6e-4 unscaled, 2e-7 scaled or transformed apart.)
+// norms near 1.  Relative error of a row's product, FP32, H = 128: F of 1e-3 of G's
+// magnitude 1e-3 unscaled, 1.6e-7 scaled.  (rowreg_kernel, which transforms the
+// factors apart, two residues of one at a time: 1.5e-7 for odd q, whose last
+// residue has a transform of its own and drops half of its rounding errors; the
+// same as here for even q.)
 struct RowScales {
   int ef, eg;
   bool near;     // the same over the wave, or over the block where slots span waves
@@ -906,15 +909,13 @@ template<typename T, int M> struct ColReg {
 
 // Waves per SIMD asked of the complex column kernels: four, so that two blocks
 // of 512 threads share a CU and one loads while the other transforms, where
-// the registers allow it with at most a few spills: all FP32 columns (at most
-// 114), FP64 with p = 1 (110 forward; 122 to 128 backward with M = 64 and 512
-// above, 16 and 28 bytes spilled at 2048 and 4096).  FP64 columns of M >= 2048
+// the registers allow it: all FP32 columns (at most 101), FP64 with p = 1 (at
+// most 128 forward, 114 backward).  FP64 columns of M >= 2048
 // leave room for the second block by reading the last stage's twiddles from
 // memory (SplitTw; 2D FP64 2000 x 500: 92 -> 81 us, 4000 x 500: 209 -> 170 us,
 // 4000 x 1000: 477 -> 428 us); at 1024 two blocks fit beside the whole table.
-template<typename T, int M, int P2, bool FWD> struct ColW {
-  static constexpr bool FIT=P2 == 1 && (FWD || (M != 64 && M != 512));
-  static constexpr int W=sizeof(T) == 4 || FIT ? 4 : 2;
+template<typename T, int P2> struct ColW {
+  static constexpr int W=sizeof(T) == 4 || P2 == 1 ? 4 : 2;
 };
 
 // The stage twiddle table of the column kernels (tw) and the residue twiddle
@@ -974,7 +975,7 @@ __device__ __forceinline__ void col_residue(cplx<T> (*w)[KH], const ColTwiddles<
 // column c starts at c*ics of f and c*ocs of F (unit strides for
 // interleaved columns, row strides for contiguous rows taken as columns).
 template<typename T, int M, int P2>
-__global__ void __launch_bounds__(512,(ColW<T,M,P2,true>::W))
+__global__ void __launch_bounds__(512,(ColW<T,P2>::W))
 colfwd_reg_kernel(DimArgs d, ColArrays io, int64_t S, int64_t C,
                   int64_t bsi, int64_t SF, int64_t bso, int64_t r0,
                   int64_t nres, int64_t ics, int64_t ocs, int zlds)
@@ -1039,7 +1040,7 @@ colfwd_reg_kernel(DimArgs d, ColArrays io, int64_t S, int64_t C,
 // f[b][j][c] = scale * ((accumulate ? f : 0) + sum_r w_N^{-(j+k0) r}
 // DFT^{-1}[F_r]((j+k0) mod M)), j < L, for each array (F, f) of io.
 template<typename T, int M, int P2>
-__global__ void __launch_bounds__(512,(ColW<T,M,P2,false>::W))
+__global__ void __launch_bounds__(512,(ColW<T,P2>::W))
 colbwd_reg_kernel(DimArgs d, ColArrays io, int64_t SF, int64_t bsi,
                   int64_t S, int64_t C, int64_t bso, int64_t r0,
                   int64_t nres, int accumulate, T scale, int64_t ics, int64_t ocs,

@@ -29,13 +29,18 @@
  * fftwpp_amd_rows_args).  Work that depends on the row alone belongs in an
  * optional member `__device__ R at(int64_t row) const`: the kernels then call
  * at(row) once per row and residue pass at most, not per element, and R's
- * operator()(F, G, l) (complex and real forms) for every element.  Only rows that exist are asked for, 0 <= row < rows (of
+ * operator()(F, G, l) (complex and real forms) for every element.
+ *
+ * Only rows that exist are asked for, 0 <= row < rows (of
  * fftwpp_amd_rows_args), so both members may read tables of one entry per row.
- * Empty slots of a last block repeat the last row, idle residue lanes a residue,
- * and drop the results: the functor returns values and has no other effects.  Multipliers on Hermitian or real plans must keep
- * the conjugate symmetry of the data (a product weighted by a function of
- * |k| in every dimension does).  Row geometries outside the register row
- * kernels (power-of-two m in [16, 4096] covering the row) are refused with
+ * Empty slots of a last block repeat the last row, idle residue lanes a
+ * residue, and drop the results: the functor returns values and has no other
+ * effects.  Multipliers on Hermitian or real plans must keep the conjugate
+ * symmetry of the data (a product weighted by a function of |k| in every
+ * dimension does).
+ *
+ * Row geometries outside the register row kernels (power-of-two m in
+ * [16, 4096] covering the row) are refused with
  * FFTWPP_AMD_ERR_UNSUPPORTED. */
 #ifndef FFTWPP_AMD_FUSED_H
 #define FFTWPP_AMD_FUSED_H
